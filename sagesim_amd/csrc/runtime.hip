@@ -420,6 +420,9 @@ int ss_create(int device, ss_ctx **out) {
         (e = hipMalloc((void **)&ctx->d_stats, 8 * sizeof(unsigned long long))) != hipSuccess ||
         (e = hipMemset(ctx->d_work, 0, SS_WORK_N * sizeof(unsigned long long))) != hipSuccess ||
         (e = hipMalloc((void **)&ctx->d_counters, 64 * sizeof(int32_t))) != hipSuccess ||
+        (e = hipHostMalloc((void **)&ctx->h_stats,
+                           sizeof(unsigned long long) * SS_STATS_ROW * 4 * prop.multiProcessorCount,
+                           hipHostMallocDefault)) != hipSuccess ||
         (e = create_halo_events(ctx)) != hipSuccess) {
         delete ctx;
         SS_FAIL(nullptr, SS_ERR_HIP, "context setup: %s", hipGetErrorString(e));
@@ -447,6 +450,7 @@ int ss_destroy(ss_ctx *ctx) {
     if (ctx->t_start) (void)hipEventDestroy(ctx->t_start);
     if (ctx->t_stop) (void)hipEventDestroy(ctx->t_stop);
     if (ctx->h_reps) (void)hipHostFree(ctx->h_reps);
+    if (ctx->h_stats) (void)hipHostFree(ctx->h_stats);
     for (int i = 0; i < SS_HALO_RING; ++i) {
         if (ctx->h_halo_pin[i]) (void)hipHostFree(ctx->h_halo_pin[i]);
         if (ctx->halo_ev[i]) (void)hipEventDestroy(ctx->halo_ev[i]);
@@ -1482,14 +1486,14 @@ int ss_replica_push_ok(ss_ctx *ctx, int32_t rep, int32_t *out) {
 int ss_census(ss_ctx *ctx, int32_t rep, int64_t *out) {
     if (!valid_rep(ctx, rep) || !out) SS_FAIL(ctx, SS_ERR_INVALID, "bad replica or NULL");
     ss_replica &r = ctx->reps[rep];
+    // everything on the context's stream: in order after the ticks before it
+    int blocks = 0;
+    SS_HIP(ctx, ss_launch_stats(r.state[r.tick & 1], r.deg8, r.row_ptr, r.n_local, r.dev.s_code, ctx->h_stats,
+                                ctx->num_cus * 4, &blocks, ctx->stream));
     SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    SS_HIP(ctx, hipMemset(ctx->d_stats, 0, 8 * sizeof(unsigned long long)));
-    SS_HIP(ctx, ss_launch_stats(r.state[r.tick & 1], r.row_ptr, r.n_local, r.dev.s_code, ctx->d_stats,
-                                ctx->num_cus * 8, ctx->stream));
-    unsigned long long h[8];
-    SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    SS_HIP(ctx, hipMemcpy(h, ctx->d_stats, sizeof h, hipMemcpyDeviceToHost));
-    for (int i = 0; i < 5; ++i) out[i] = (int64_t)h[i];
+    for (int i = 0; i < 5; ++i) out[i] = 0;
+    for (int b = 0; b < blocks; ++b)
+        for (int i = 0; i < 5; ++i) out[i] += (int64_t)ctx->h_stats[SS_STATS_ROW * b + i];
     return SS_OK;
 }
 

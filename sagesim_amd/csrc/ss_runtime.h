@@ -58,8 +58,11 @@ hipError_t ss_launch_gather_probe(const uint32_t *src, int64_t n_words, int64_t 
 hipError_t ss_launch_fill_u32(uint32_t *p, int64_t n, uint32_t v, int grid, hipStream_t s);
 hipError_t ss_launch_check_cols(const int32_t *col, int64_t nnz, int64_t n_total, unsigned long long *first_bad,
                                 int grid, hipStream_t s);
-hipError_t ss_launch_stats(const int8_t *st, const int64_t *row_ptr, int64_t n_local, int8_t s_code,
-                           unsigned long long *out, int grid, hipStream_t s);
+// census: row b of part (SS_STATS_ROW words) gets block b's counts of states
+// 0..3 and sum of degrees in s_code; *blocks rows are written
+#define SS_STATS_ROW 8
+hipError_t ss_launch_stats(const int8_t *st, const uint8_t *deg8, const int64_t *row_ptr, int64_t n_local,
+                           int8_t s_code, unsigned long long *part, int max_blocks, int *blocks, hipStream_t s);
 // push decision of the current tick from its statistics acc_t, then (when
 // pushing) its infectious-neighbour counts (cleared before) from the bitmap
 hipError_t ss_launch_count_init(const int64_t *row_ptr, const int32_t *col_idx, const uint64_t *bits,
@@ -147,7 +150,8 @@ struct ss_ctx {
     std::map<int64_t, hipGraphExec_t> graphs;   // by tick count
     int32_t *d_counters = nullptr;              // misc device counters (misses, overflow)
     unsigned long long *d_work = nullptr;       // [SS_WORK_N] tick-kernel work counters
-    unsigned long long *d_stats = nullptr;      // [8] census output
+    unsigned long long *d_stats = nullptr;      // [8] results of the checks at replica creation
+    unsigned long long *h_stats = nullptr;      // census rows, page-locked, 4 blocks per CU
     bool counting = false;
     uint32_t push_num = 4;                      // direction rule, 16 * ratio (0: pull only); ratio 0.25
     hipEvent_t t_start = nullptr, t_stop = nullptr;
