@@ -178,9 +178,9 @@ void drop_graphs(ss_ctx *ctx) {
 // past the rows of degree >= heavy_deg, LIGHT tiles for the rest (light tiles
 // start 64-aligned: no bitmap word is shared by two light tiles, the hub and
 // heavy tiles set single bits).  A light tile holds 256 * apl agents; with 16
-// agents per lane it holds 4 * 1024, fewer where its rows are longer than the
-// replica's average light row: a tile of rows of degree d > dbar holds dbar / d
-// of that (about as many CSR entries as an average tile), in steps of 256
+// agents per lane it holds up to 4 * 1024 (see `base`), fewer where its rows are
+// longer than the replica's average light row: a tile of rows of degree d > dbar
+// holds dbar / d of that (about as many CSR entries as an average tile), in steps of 256
 // agents down to 256 and of 64 below, so that the tiles at the long-row end
 // cost about as much as the others.  Blocks stride over the list (see below).
 int build_tiles(ss_ctx *ctx) {
@@ -193,6 +193,23 @@ int build_tiles(ss_ctx *ctx) {
     struct Pos { int64_t hub, heavy, light, lblocks; };
     std::vector<Pos> pos(ctx->reps.size(), Pos{0, 0, 0, 0});
     int64_t n_lblocks = 0;                       // tag slots of light agents, all replicas
+    // Agents of a wide tile of average rows: a block per CU when the light
+    // agents are few (in whole 256s, 64s below), at most the capacity.  More
+    // blocks than that cost more in set-up than their shorter tiles save:
+    // reset, 100 ticks and readback of WS(100k, 10) SEIR took 2.45 ms at 256
+    // blocks or fewer, 3.0-3.1 ms at 400-1600 blocks and 3.5 ms at 25 blocks
+    // of 4096 agents; G(10k, 0.001) SIR 0.96 ms at 64 agents a tile, 1.0 ms
+    // at 256 and 1.38 ms at 4096; BA(1M, 5) 2.75-2.85 ms at 3072-4096 agents,
+    // 3.3-3.5 ms at 1024.
+    int64_t base = cap;
+    if (ctx->apl == 16) {
+        int64_t light_n = 0;
+        for (const ss_replica &r : ctx->reps)
+            if (r.live) light_n += std::max<int64_t>(0, r.n_total - std::max<int64_t>(0, heavy_prefix(r, ctx->heavy_deg)));
+        const int64_t share = (light_n + ctx->num_cus - 1) / ctx->num_cus;
+        const int64_t step = share >= 256 ? 256 : 64;
+        base = std::min(cap, std::max<int64_t>(64, (share + step - 1) / step * step));
+    }
     for (int32_t ri = 0; ri < (int32_t)ctx->reps.size(); ++ri) {
         ss_replica &r = ctx->reps[ri];
         if (!r.live || r.n_total == 0) continue;
@@ -213,8 +230,8 @@ int build_tiles(ss_ctx *ctx) {
         for (int64_t b = H64; b < nt;) {
             const int64_t g1 = std::min<int64_t>(b + 64, nt);
             const double d = (double)(E(g1) - E(b)) / (double)(g1 - b);
-            int64_t a = cap;
-            if (ctx->apl == 16 && dbar > 0.0 && d > dbar) a = (int64_t)((double)cap * dbar / d);
+            int64_t a = base;
+            if (ctx->apl == 16 && dbar > 0.0 && d > dbar) a = (int64_t)((double)base * dbar / d);
             // whole groups of 4 x 64 agents: the 4 wavefronts of a wide tile get
             // equal chunks of whole bitmap words; a wide tile of long rows may
             // hold 64, 128 or 192 agents (chunks of 16, 32 or 48)
