@@ -501,7 +501,7 @@ int ss_device_info(ss_ctx *ctx, int32_t *num_cus, int64_t *total_mem, int64_t *c
 int64_t ss_replica_footprint(int64_t n_local, int64_t n_ghost, int64_t nnz, int32_t with_history, int64_t max_deg) {
     int64_t n_total = n_local + n_ghost;
     int64_t words = (n_total + 63) / 64;
-    int64_t b = 8 * (n_total + 1) + 4 * nnz + 6 * pad_agents(n_local) + 2 * pad_agents(n_total) + n_total +
+    int64_t b = 8 * (n_total + 1) + 4 * (nnz + SS_COL_PAD) + 6 * pad_agents(n_local) + 2 * pad_agents(n_total) + n_total +
                 2 * 8 * words + 4 * (std::min<int64_t>(max_deg, 1 << 24) + 1) + 8 * SS_ACC_WORDS +
                 (n_ghost == 0 ? 4 * pad_agents(n_local) + 8 : 0);
     if (with_history) b += 2 * 4 * n_local * SS_HISTORY_WIDTH;
@@ -564,9 +564,9 @@ int ss_replica_create(ss_ctx *ctx, const ss_replica_spec *sp, int32_t *rep_out) 
         }                                                                            \
     } while (0)
     R_HIP(dalloc(ctx, &r, &r.row_ptr, (size_t)nt + 1));
-    // whole 16-byte groups: a lane's scan reads its row through aligned 16-byte loads
-    R_HIP(dalloc(ctx, &r, &r.col_idx, (size_t)(nnz + 3) / 4 * 4));
-    if (nnz & 3) R_HIP(hipMemset(r.col_idx + nnz, 0, sizeof(int32_t) * (size_t)(4 - (nnz & 3))));
+    // a lane's scan reads its row eight entries at a time
+    R_HIP(dalloc(ctx, &r, &r.col_idx, (size_t)nnz + SS_COL_PAD));
+    R_HIP(hipMemset(r.col_idx + nnz, 0, sizeof(int32_t) * SS_COL_PAD));
     // per-agent arrays the light tiles read as 16-agent vectors are padded
     R_HIP(dalloc(ctx, &r, &r.rng_lo, (size_t)pad_agents(nl)));
     R_HIP(dalloc(ctx, &r, &r.deg8, (size_t)pad_agents(nl)));

@@ -15,7 +15,7 @@
 // ghost slots whose state is carried over and refreshed from the halo.
 struct ss_rep_dev {
     const int64_t *row_ptr;     // [n_total + 1]; ghost rows are empty
-    const int32_t *col_idx;     // [nnz] slot indices
+    const int32_t *col_idx;     // [nnz + SS_COL_PAD] slot indices, then zeros
     const uint32_t *rng_lo;     // [n_local] low word of the agent's RNG key id
     const uint32_t *rng_hi;     // [n_local] high word, or null when all ids < 2^32
     int8_t *state[2];           // ping-pong; tick t reads state[t & 1]
@@ -73,6 +73,7 @@ struct ss_rep_dev {
 };
 
 #define SS_LTAG_SHIFT 10
+#define SS_COL_PAD 8            // entries a row's scan may read past its end
 
 #define SS_ACC_SLOTS 16
 #define SS_ACC_WORDS (3 * SS_ACC_SLOTS * 2)

@@ -261,49 +261,43 @@ __device__ __forceinline__ void st4(SS_G void *p, const uint4 v) {
     *(SS_G v4u32 *)p = x;
 }
 
-// Scan of one row by one lane, eight entries per round.  The entries come
-// from at most three aligned 16-byte loads (col_idx is padded to whole
-// 16-byte groups) and only entries inside the row look up the bitmap, so a
-// round costs the memory pipeline a few lines per lane instead of one per
-// entry.  Returns whether the count of infectious neighbours reaches the
-// agent's draw.
+// Scan of one row by one lane, eight entries per round: two 16-byte loads at the
+// row's own 4-byte alignment (col_idx is padded by a round), one 32-bit bitmap
+// word per entry inside the row, and one threshold lookup for the round's count
+// (T is non-decreasing, so the count after the round infects when some count
+// within it does).  A scan is bound by its chain of round trips and, at the
+// middle of an epidemic, by the instructions around them (the vector units are
+// busy 45 % of the time there); against aligned loads with a select per entry,
+// 64-bit bitmap words, a threshold lookup per hit and a row pointer per row:
+// 200 ticks of BA(10M, 5) 9.47 -> 8.71 ms, of BA(1M, 5) 2.80 -> 2.60, 100 ticks
+// of WS(100k, 10) SEIR 1.31 -> 1.25.  Returns whether the count of infectious
+// neighbours reaches the agent's draw; with `hist`, first is the first of them.
 __device__ __forceinline__ bool scan_lane(const TickView V, const LCold *C, int64_t b, int64_t e, uint32_t m,
-                                          int32_t &first, Work &w) {
-    const SS_G int32_t *__restrict__ col = V.col_idx;
-    const SS_G uint64_t *__restrict__ cb = V.cb;
+                                          bool hist, int32_t &first, Work &w) {
+    typedef uint32_t v4 __attribute__((ext_vector_type(4), aligned(4)));
+    const SS_G int32_t *__restrict__ col = V.col_idx + b;
+    const SS_G uint8_t *__restrict__ cb = (const SS_G uint8_t *)V.cb;
     int32_t k = 0;
-    for (int64_t j = b; j < e; j += 8) {
-        const int64_t a = j & ~(int64_t)3;
-        const int64_t lim = e < j + 8 ? e : j + 8;
-        const uint4 x0 = ld4(col + a);
-        const uint4 x1 = a + 4 < lim ? ld4(col + a + 4) : make_uint4(0u, 0u, 0u, 0u);
-        const uint4 x2 = a + 8 < lim ? ld4(col + a + 8) : make_uint4(0u, 0u, 0u, 0u);
-        // entries j .. j + 7 are words (j & 3) .. (j & 3) + 7 of x0 x1 x2,
-        // selected with named values (an indexed array would go to scratch)
-        const bool s2 = (j & 2) != 0, s1 = (j & 1) != 0;
-        const uint32_t h0 = s2 ? x0.z : x0.x, h1 = s2 ? x0.w : x0.y, h2 = s2 ? x1.x : x0.z;
-        const uint32_t h3 = s2 ? x1.y : x0.w, h4 = s2 ? x1.z : x1.x, h5 = s2 ? x1.w : x1.y;
-        const uint32_t h6 = s2 ? x2.x : x1.z, h7 = s2 ? x2.y : x1.w, h8 = s2 ? x2.z : x2.x;
-        int32_t c[8];
-        c[0] = (int32_t)(s1 ? h1 : h0);
-        c[1] = (int32_t)(s1 ? h2 : h1);
-        c[2] = (int32_t)(s1 ? h3 : h2);
-        c[3] = (int32_t)(s1 ? h4 : h3);
-        c[4] = (int32_t)(s1 ? h5 : h4);
-        c[5] = (int32_t)(s1 ? h6 : h5);
-        c[6] = (int32_t)(s1 ? h7 : h6);
-        c[7] = (int32_t)(s1 ? h8 : h7);
-        uint64_t wd[8];
+    for (int32_t left = (int32_t)(e - b); left > 0; left -= 8, col += 8) {
+        const v4 x0 = *(const SS_G v4 *)col;
+        v4 x1 = {0u, 0u, 0u, 0u};
+        if (left > 4) x1 = *(const SS_G v4 *)(col + 4);
+        const uint32_t c[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+        uint32_t wd[8];
 #pragma unroll
-        for (int q = 0; q < 8; ++q) wd[q] = j + q < e ? cb[c[q] >> 6] : 0ull;
-        w.edges += (uint32_t)(e - j < 8 ? e - j : 8);
+        for (int q = 0; q < 8; ++q) wd[q] = q < left ? *(const SS_G uint32_t *)(cb + ((c[q] >> 3) & ~3u)) : 0u;
+        w.edges += (uint32_t)(left < 8 ? left : 8);
+        uint32_t hits = 0u;
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            if ((wd[q] >> (c[q] & 63)) & 1ull) {
-                if (first < 0) first = c[q];
-                ++k;
-                if (m < thr(V, C, k)) return true;
+        for (int q = 0; q < 8; ++q) hits |= ((wd[q] >> (c[q] & 31u)) & 1u) << q;
+        if (hits != 0u) {
+            if (hist && first < 0) {
+                const int f = __ffs(hits) - 1;
+#pragma unroll
+                for (int q = 0; q < 8; ++q) first = f == q ? (int32_t)c[q] : first;
             }
+            k += __popc(hits);
+            if (m < thr(V, C, k)) return true;
         }
     }
     return false;
@@ -501,7 +495,7 @@ __device__ __forceinline__ void light_tile(const TickView V, const LCold *C, int
             const int64_t i = begin + (sl & ~SS_QHIST);
             const int64_t b = V.row_ptr[i], e = V.row_ptr[i + 1];
             // with m = 0 the scan stops at the first infectious neighbour
-            const bool inf = scan_lane(V, C, b, e, Q.m[sec + q], first, w);
+            const bool inf = scan_lane(V, C, b, e, Q.m[sec + q], C->history != nullptr, first, w);
             if (!hist_only) Q.hit[sl] = inf ? 1 : 0;
             if (inf && C->history) ss_hist_append(C->history + i * SS_HIST_W, first);
             if (inf && !hist_only) dir_change(dir, V, V.s_code, V.s_target, e - b);
@@ -653,6 +647,19 @@ __device__ __forceinline__ void light_wide(const TickView V, const LCold *C, int
             if (any != 0u) st4(V.cnt + i0 + 8 * q, make_uint4(0u, 0u, 0u, (uint32_t)opaque(0)));
         }
     }
+    // A chunk whose rows all have du entries (most are: rows are sorted by
+    // degree) starts row i at row0 + (i - c0) du, so its scans skip the round
+    // trip to the row pointers.
+    int64_t row0 = -1;
+    uint32_t du = 0u;
+    if (pull) {
+        du = (uint32_t)__builtin_amdgcn_readfirstlane((int)(dg[0] & 0xFFu));
+        const uint32_t D = 0x01010101u * du;
+        uint32_t off = 0u;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) off |= (dg[q] ^ D) & (nl == 16 ? ~0u : byte_mask4((lmask >> (4 * q)) & 15u));
+        if (du != 255u && !__ballot(off != 0u)) row0 = V.row_ptr[c0];
+    }
     // states with a spontaneous transition, as a bit set over state codes 0..3
     uint32_t tbits = 0u;
 #pragma unroll
@@ -758,13 +765,13 @@ __device__ __forceinline__ void light_wide(const TickView V, const LCold *C, int
                 y = en.y;
                 const int64_t i = c0 + (y & 1023u);
                 const uint32_t d = y >> 16;
-                b = V.row_ptr[i];
+                b = row0 >= 0 ? row0 + (int64_t)((y & 1023u) * du) : V.row_ptr[i];
                 e = d == 255u ? V.row_ptr[i + 1] : b + (int64_t)d;
                 lng = e - b > SS_WIDE_SHORT;
             }
             bool inf = false;
             int32_t first = -1;
-            if (q < nsq && !lng) inf = scan_lane(V, C, b, e, m, first, w);
+            if (q < nsq && !lng) inf = scan_lane(V, C, b, e, m, C->history != nullptr, first, w);
             scan_rows(V, C, __ballot(lng), b, e, m, lane, inf, first, w);
             if (q < nsq && inf) {
                 const uint32_t slot = y & 1023u;
