@@ -108,6 +108,13 @@ int ss_set_seed(ss_ctx *ctx, int32_t rep, uint64_t seed);
 /* ---- state readback / upload: replace get_agent_property_value's slice
  *      .get() (model.py:422-450) and set_agent_property_value ---- */
 int ss_state_download(ss_ctx *ctx, int32_t rep, int8_t *out, int64_t n);
+/* The caller's agent order, for callers that relabelled the rows: slot[j] in
+ * [0, n_local) is the local slot of agent j.  Kept on the device (4 bytes an
+ * agent) until it is set again or the replica goes. */
+int ss_replica_set_order(ss_ctx *ctx, int32_t rep, const int32_t *slot, int64_t n_local);
+/* ss_state_download with the local agents in that order: out[j] = state of
+ * slot[j], then the ghost slots as they are. */
+int ss_state_download_ordered(ss_ctx *ctx, int32_t rep, int8_t *out, int64_t n);
 int ss_state_upload(ss_ctx *ctx, int32_t rep, const int8_t *in, int64_t n);
 int ss_history_download(ss_ctx *ctx, int32_t rep, int32_t *out, int64_t n_rows);
 

@@ -80,6 +80,8 @@ def step_lib():
     _proto(L, "ss_set_model", I, _P, _c_i32, ctypes.POINTER(SSModel))
     _proto(L, "ss_set_seed", I, _P, _c_i32, _c_u64)
     _proto(L, "ss_state_download", I, _P, _c_i32, _P, _c_i64)
+    _proto(L, "ss_replica_set_order", I, _P, _c_i32, _P, _c_i64)
+    _proto(L, "ss_state_download_ordered", I, _P, _c_i32, _P, _c_i64)
     _proto(L, "ss_state_upload", I, _P, _c_i32, _P, _c_i64)
     _proto(L, "ss_history_download", I, _P, _c_i32, _P, _c_i64)
     _proto(L, "ss_replica_save", I, _P, _c_i32, _P, _c_i64, _P)

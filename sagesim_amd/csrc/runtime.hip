@@ -49,6 +49,29 @@ void dfree(void *p) {
     if (p) (void)hipFree(p);
 }
 
+// The context's workspace, at least b bytes (256-byte aligned): kept for later
+// calls, replaced by a larger one when it is too small, freed with the context.
+// Every user runs on the context's stream and is done with it when it returns.
+hipError_t scratch(ss_ctx *ctx, size_t b, void **p) {
+    if (ctx->scratch_bytes < b) {
+        hipError_t e = hipStreamSynchronize(ctx->stream);
+        if (e != hipSuccess) return e;
+        dfree(ctx->scratch);
+        ctx->scratch = nullptr;
+        ctx->bytes -= ctx->scratch_bytes;
+        ctx->scratch_bytes = 0;
+        const size_t want = std::max<size_t>(b + b / 4, 1 << 16);
+        if ((e = hipMalloc(&ctx->scratch, want)) != hipSuccess) {
+            ctx->scratch = nullptr;
+            return e;
+        }
+        ctx->scratch_bytes = want;
+        ctx->bytes += want;
+    }
+    *p = ctx->scratch;
+    return hipSuccess;
+}
+
 // inf_T[k] = ceil(p_k * 2^23), p_k = 1 - q_k, q_k = q_{k-1} * (1 - beta),
 // for k = 0 .. min(max_deg, first k with p_k * 2^23 == 2^23).
 std::vector<uint32_t> threshold_table(double beta, int64_t max_deg) {
@@ -127,6 +150,7 @@ void free_replica(ss_replica &r) {
     dfree(r.ibits[0]); dfree(r.ibits[1]);
     dfree(r.history); dfree(r.init_history); dfree(r.inf_T);
     dfree(r.cnt[0]); dfree(r.cnt[1]); dfree(r.dec); dfree(r.acc);
+    dfree(r.order);
     dfree(r.map_keys); dfree(r.map_vals); dfree(r.halo_slots);
     for (auto &d : r.halo_dev) dfree(d);
     for (auto &d : r.halo_grp) dfree(d);
@@ -464,6 +488,7 @@ int ss_destroy(ss_ctx *ctx) {
     dfree(ctx->d_counters);
     dfree(ctx->d_work);
     dfree(ctx->d_stats);
+    dfree(ctx->scratch);
     if (ctx->t_start) (void)hipEventDestroy(ctx->t_start);
     if (ctx->t_stop) (void)hipEventDestroy(ctx->t_stop);
     if (ctx->h_reps) (void)hipHostFree(ctx->h_reps);
@@ -762,6 +787,45 @@ int ss_state_download(ss_ctx *ctx, int32_t rep, int8_t *out, int64_t n) {
     if (n != r.n_total) SS_FAIL(ctx, SS_ERR_INVALID, "n = %lld, replica has %lld slots", (long long)n, (long long)r.n_total);
     SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
     if (n) SS_HIP(ctx, hipMemcpy(out, r.state[r.tick & 1], (size_t)n, hipMemcpyDeviceToHost));
+    return SS_OK;
+}
+
+int ss_replica_set_order(ss_ctx *ctx, int32_t rep, const int32_t *slot, int64_t n) {
+    if (!valid_rep(ctx, rep) || (!slot && n)) SS_FAIL(ctx, SS_ERR_INVALID, "bad replica or NULL");
+    ss_replica &r = ctx->reps[rep];
+    if (n != r.n_local) SS_FAIL(ctx, SS_ERR_INVALID, "n = %lld, replica has %lld agents", (long long)n, (long long)r.n_local);
+    if (n == 0) return SS_OK;
+    SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (!r.order) SS_HIP(ctx, dalloc(ctx, &r, &r.order, (size_t)pad_agents(n)));
+    unsigned long long bad = ~0ull;
+    SS_HIP(ctx, hipMemcpy(r.order, slot, sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice));
+    SS_HIP(ctx, hipMemcpy(ctx->d_stats, &bad, sizeof bad, hipMemcpyHostToDevice));
+    SS_HIP(ctx, ss_launch_check_cols(r.order, n, n, ctx->d_stats, ctx->num_cus * 8, ctx->stream));
+    SS_HIP(ctx, hipMemcpyAsync(&bad, ctx->d_stats, sizeof bad, hipMemcpyDeviceToHost, ctx->stream));
+    SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (bad != ~0ull) {
+        dfree(r.order);
+        r.order = nullptr;
+        r.bytes -= sizeof(int32_t) * (size_t)pad_agents(n);
+        ctx->bytes -= sizeof(int32_t) * (size_t)pad_agents(n);
+        SS_FAIL(ctx, SS_ERR_RANGE, "slot[%llu] = %d outside [0, %lld)", bad, slot[bad], (long long)n);
+    }
+    return SS_OK;
+}
+
+int ss_state_download_ordered(ss_ctx *ctx, int32_t rep, int8_t *out, int64_t n) {
+    if (!valid_rep(ctx, rep) || (!out && n)) SS_FAIL(ctx, SS_ERR_INVALID, "bad replica or NULL");
+    ss_replica &r = ctx->reps[rep];
+    if (n != r.n_total) SS_FAIL(ctx, SS_ERR_INVALID, "n = %lld, replica has %lld slots", (long long)n, (long long)r.n_total);
+    if (!r.order) {
+        if (r.n_local) SS_FAIL(ctx, SS_ERR_STATE, "replica has no order (ss_replica_set_order)");
+        return ss_state_download(ctx, rep, out, n);
+    }
+    void *d = nullptr;
+    SS_HIP(ctx, scratch(ctx, (size_t)pad_agents(n), &d));
+    SS_HIP(ctx, ss_launch_order(r.state[r.tick & 1], r.order, (int8_t *)d, r.n_local, n, ctx->stream));
+    SS_HIP(ctx, hipMemcpyAsync(out, d, (size_t)n, hipMemcpyDeviceToHost, ctx->stream));
+    SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return SS_OK;
 }
 

@@ -51,6 +51,10 @@ hipError_t ss_launch_gather(const int8_t *st, const int32_t *slots, int8_t *out,
 // out[h / 4] bits 2 (h % 4).. = st[slots[h]] & 3
 hipError_t ss_launch_gather2(const int8_t *st, const int32_t *slots, uint8_t *out, int64_t n, hipStream_t s);
 hipError_t ss_launch_fill_i32(int32_t *p, int64_t n, int32_t v, hipStream_t s);
+// out[j] = st[slot[j]], j < n_local; out[j] = st[j] for the ghosts (slot and
+// out padded to whole groups of 16)
+hipError_t ss_launch_order(const int8_t *st, const int32_t *slot, int8_t *out, int64_t n_local, int64_t n_total,
+                           hipStream_t s);
 hipError_t ss_launch_copy(const void *src, void *dst, int64_t bytes, int grid, hipStream_t s);
 // n scattered 4-byte reads of src[0 .. n_words); out holds grid * 256 words
 hipError_t ss_launch_gather_probe(const uint32_t *src, int64_t n_words, int64_t n, uint32_t *out, int grid,
@@ -96,6 +100,7 @@ struct ss_replica {
     uint32_t *dec = nullptr;                   // push decisions [2] by tick parity
     unsigned long long *acc = nullptr;         // direction statistics [SS_ACC_WORDS]
     bool symmetric = false;                    // every entry (i, j) has its mirror (j, i)
+    int32_t *order = nullptr;                  // slot of every agent in the caller's order, or null
     // id -> slot map for ghosts
     unsigned long long *map_keys = nullptr;
     int32_t *map_vals = nullptr;
@@ -164,6 +169,8 @@ struct ss_ctx {
     hipEvent_t span_ev[2][SS_HALO_SPANS] = {};  // copy span s of group buffer b is on the device
     int64_t grp_pos = 0;                        // groups issued (buffer = grp_pos & 1)
     bool halo_fused = false;                    // this call's ticks fuse the next tick's halo refresh
+    void *scratch = nullptr;                    // workspace of one call at a time, on the context's stream
+    size_t scratch_bytes = 0;
     std::string err;
     size_t bytes = 0;
 };

@@ -160,6 +160,17 @@ class Engine:
         self._ck(self._L.ss_state_download(self._h, rep, ptr(out), n_total))
         return out
 
+    def set_order(self, rep, slots):
+        """The caller's agent order: slots[j] is the storage slot of agent j."""
+        slots = np.ascontiguousarray(slots, np.int32)
+        self._ck(self._L.ss_replica_set_order(self._h, rep, ptr(slots), slots.shape[0]))
+
+    def state_ordered(self, rep, n_total):
+        """The states with the local agents in the order of set_order."""
+        out = np.empty(n_total, np.int8)
+        self._ck(self._L.ss_state_download_ordered(self._h, rep, ptr(out), n_total))
+        return out
+
     def set_state(self, rep, st):
         st = np.ascontiguousarray(st, np.int8)
         self._ck(self._L.ss_state_upload(self._h, rep, ptr(st), st.shape[0]))
@@ -437,16 +448,18 @@ class Replica:
         self.n = data.n
         self.n_total = data.n_total
         self.n_ghost = self.n_total - self.n
+        self._order_set = False
         self.rep = engine.add_replica(data.graph.row_ptr, data.graph.col_idx, data.rng_key_id, data.state, model,
                                       seed, n_ghost=self.n_ghost, history=data.history, tick0=tick0,
                                       tick_limit=tick_limit)
 
     def states(self):
-        st = self.engine.state(self.rep, self.n_total)
-        out = np.empty_like(st)
-        out[self.perm] = st[:self.n]
-        out[self.n:] = st[self.n:]
-        return out
+        """The states in the caller's agent order (put in order on the device,
+        which keeps the order from the first call on)."""
+        if not self._order_set:
+            self.engine.set_order(self.rep, self.inv)
+            self._order_set = True
+        return self.engine.state_ordered(self.rep, self.n_total)
 
     def set_states(self, state):
         state = np.asarray(state, np.int8)
