@@ -294,6 +294,8 @@ int ss_timer_stop(ss_ctx *ctx, float *ms);
  * which includes "sagesim_rt.h" (the device runtime this library embeds). */
 typedef struct ss_prog ss_prog;
 int ss_prog_create(ss_ctx *ctx, int64_t n_agents, ss_prog **out);
+/* before or after its context: ss_destroy frees the device memory of the
+ * context's programs, whose calls return SS_ERR_STATE from then on */
 int ss_prog_destroy(ss_prog *prog);
 const char *ss_prog_last_error(const ss_prog *prog);
 int ss_prog_set_csr(ss_prog *prog, const int64_t *row_ptr, const int32_t *col_idx, int64_t nnz);

@@ -8,6 +8,7 @@
 // reference caches its generated module, model.py:843-865), loads it, and
 // runs the per-tick launch schedule followed by the write-back of
 // double-buffered arrays (model.py:2368-2408).
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -191,6 +192,11 @@ static thread_local std::string g_prog_err;
                    hipGetErrorString(_e));                                               \
     } while (0)
 
+#define P_LIVE(p)                                                                                  \
+    do {                                                                                           \
+        if ((p) && !(p)->ctx) P_FAIL(p, SS_ERR_STATE, "the context of this program has been destroyed"); \
+    } while (0)
+
 static void pfree(void *q) {
     if (q) (void)hipFree(q);
 }
@@ -253,6 +259,29 @@ static int write_back(ss_prog *p, hipStream_t st) {
     return SS_OK;
 }
 
+// The program's device resources; its context is alive.
+static void release(ss_prog *p) {
+    (void)hipStreamSynchronize(p->ctx->stream);
+    if (p->module) (void)hipModuleUnload(p->module);
+    pfree(p->d_args); pfree(p->agent_ids); pfree(p->logical_ids); pfree(p->breeds);
+    pfree(p->row_ptr); pfree(p->col_idx); pfree(p->globals); pfree(p->logical_ids64); pfree(p->order);
+    for (auto &q : p->props) {
+        if (q.w != q.r) pfree(q.w);
+        pfree(q.r);
+    }
+    for (auto &x : p->extras) pfree(x.d);
+    p->module = nullptr;
+    p->ctx = nullptr;
+}
+
+// Programs may be destroyed after their context (a garbage collector picks the
+// order): the context's end frees what they hold on its device, and they keep
+// no pointer to it.
+void ss_release_programs(ss_ctx *ctx) {
+    for (ss_prog *p : ctx->progs) release(p);
+    ctx->progs.clear();
+}
+
 extern "C" {
 
 const char *ss_prog_last_error(const ss_prog *p) { return p ? p->err.c_str() : g_prog_err.c_str(); }
@@ -278,26 +307,24 @@ int ss_prog_create(ss_ctx *ctx, int64_t n_agents, ss_prog **out) {
         delete p;
         return e == hipErrorOutOfMemory ? SS_ERR_OOM : SS_ERR_HIP;
     }
+    ctx->progs.push_back(p);
     *out = p;
     return SS_OK;
 }
 
 int ss_prog_destroy(ss_prog *p) {
     if (!p) return SS_OK;
-    (void)hipStreamSynchronize(p->ctx->stream);
-    if (p->module) (void)hipModuleUnload(p->module);
-    pfree(p->d_args); pfree(p->agent_ids); pfree(p->logical_ids); pfree(p->breeds);
-    pfree(p->row_ptr); pfree(p->col_idx); pfree(p->globals); pfree(p->logical_ids64); pfree(p->order);
-    for (auto &q : p->props) {
-        if (q.w != q.r) pfree(q.w);
-        pfree(q.r);
+    if (p->ctx) {
+        auto &v = p->ctx->progs;
+        v.erase(std::remove(v.begin(), v.end(), p), v.end());
+        release(p);
     }
-    for (auto &x : p->extras) pfree(x.d);
     delete p;
     return SS_OK;
 }
 
 int ss_prog_set_csr(ss_prog *p, const int64_t *row_ptr, const int32_t *col_idx, int64_t nnz) {
+    P_LIVE(p);
     if (!p || !row_ptr || (nnz && !col_idx)) P_FAIL(p, SS_ERR_INVALID, "NULL argument");
     if (row_ptr[0] != 0 || row_ptr[p->n] != nnz) P_FAIL(p, SS_ERR_INVALID, "row_ptr must start at 0 and end at nnz");
     for (int64_t i = 0; i < p->n; ++i)
@@ -321,6 +348,7 @@ int ss_prog_set_csr(ss_prog *p, const int64_t *row_ptr, const int32_t *col_idx, 
 
 int ss_prog_set_ids(ss_prog *p, const float *agent_ids, const float *logical_ids, const int64_t *logical_ids64,
                     const float *breeds) {
+    P_LIVE(p);
     if (!p || (p->n && (!agent_ids || !logical_ids || !logical_ids64 || !breeds)))
         P_FAIL(p, SS_ERR_INVALID, "NULL argument");
     if (p->n) {
@@ -334,6 +362,7 @@ int ss_prog_set_ids(ss_prog *p, const float *agent_ids, const float *logical_ids
 
 int ss_prog_add_array(ss_prog *p, int32_t elem_bytes, int64_t rows, int64_t width, int32_t double_buffered,
                       const void *init, int32_t *id) {
+    P_LIVE(p);
     if (!p || !id) P_FAIL(p, SS_ERR_INVALID, "NULL argument");
     if (elem_bytes != 1 && elem_bytes != 2 && elem_bytes != 4 && elem_bytes != 8)
         P_FAIL(p, SS_ERR_INVALID, "elem_bytes must be 1, 2, 4 or 8");
@@ -371,11 +400,13 @@ int ss_prog_add_array(ss_prog *p, int32_t elem_bytes, int64_t rows, int64_t widt
 
 int ss_prog_add_prop(ss_prog *p, int32_t elem_bytes, int64_t width, int32_t double_buffered, const void *init,
                      int32_t *id) {
+    P_LIVE(p);
     if (!p) P_FAIL(p, SS_ERR_INVALID, "NULL program");
     return ss_prog_add_array(p, elem_bytes, p->n, width, double_buffered, init, id);
 }
 
 int ss_prog_prop_upload(ss_prog *p, int32_t id, const void *data) {
+    P_LIVE(p);
     if (!p || id < 0 || id >= (int32_t)p->props.size() || !data) P_FAIL(p, SS_ERR_INVALID, "bad array or NULL");
     const ProgProp &q = p->props[id];
     const size_t nb = q.bytes();
@@ -388,6 +419,7 @@ int ss_prog_prop_upload(ss_prog *p, int32_t id, const void *data) {
 }
 
 int ss_prog_prop_download(ss_prog *p, int32_t id, void *out) {
+    P_LIVE(p);
     if (!p || id < 0 || id >= (int32_t)p->props.size() || !out) P_FAIL(p, SS_ERR_INVALID, "bad array or NULL");
     const ProgProp &q = p->props[id];
     P_HIP(p, hipStreamSynchronize(p->ctx->stream));
@@ -397,6 +429,7 @@ int ss_prog_prop_download(ss_prog *p, int32_t id, void *out) {
 }
 
 int ss_prog_set_globals(ss_prog *p, const double *values, int64_t count) {
+    P_LIVE(p);
     if (!p || (count && !values) || count < 0) P_FAIL(p, SS_ERR_INVALID, "bad globals");
     P_HIP(p, hipStreamSynchronize(p->ctx->stream));
     if (count != p->n_globals) {
@@ -413,6 +446,7 @@ int ss_prog_set_globals(ss_prog *p, const double *values, int64_t count) {
 // The reference keeps the seed as int32 (model.py:1104) and reduces it mod
 // 2^32 in the RNG (math_utils.py:108-111); the low 32 bits are what matter.
 int ss_prog_set_seed(ss_prog *p, int64_t seed) {
+    P_LIVE(p);
     if (!p) P_FAIL(p, SS_ERR_INVALID, "NULL program");
     P_HIP(p, hipStreamSynchronize(p->ctx->stream));
     p->seed = (int32_t)(uint32_t)(uint64_t)seed;
@@ -422,6 +456,7 @@ int ss_prog_set_seed(ss_prog *p, int64_t seed) {
 }
 
 int ss_prog_set_extra(ss_prog *p, int32_t slot, int64_t bytes, const void *data) {
+    P_LIVE(p);
     if (!p || slot < 0 || slot >= SS_MAXX_HOST || bytes < 0 || (bytes && !data))
         P_FAIL(p, SS_ERR_INVALID, "bad extra slot, size or NULL data");
     P_HIP(p, hipStreamSynchronize(p->ctx->stream));
@@ -438,6 +473,7 @@ int ss_prog_set_extra(ss_prog *p, int32_t slot, int64_t bytes, const void *data)
 }
 
 int ss_prog_get_extra(ss_prog *p, int32_t slot, int64_t bytes, void *out) {
+    P_LIVE(p);
     if (!p || slot < 0 || slot >= SS_MAXX_HOST || (bytes && !out)) P_FAIL(p, SS_ERR_INVALID, "bad extra slot or NULL");
     const Extra &x = p->extras[slot];
     if (!x.d || bytes != x.bytes) P_FAIL(p, SS_ERR_INVALID, "extra slot %d holds %lld bytes", slot, (long long)x.bytes);
@@ -447,6 +483,7 @@ int ss_prog_get_extra(ss_prog *p, int32_t slot, int64_t bytes, void *out) {
 }
 
 int ss_prog_compile(ss_prog *p, const char *source, const char *kernel_names, char *log, int64_t log_cap) {
+    P_LIVE(p);
     if (!p || !source || !kernel_names) P_FAIL(p, SS_ERR_INVALID, "NULL argument");
     if (log && log_cap > 0) log[0] = 0;
     const std::vector<std::string> opts_s = rtc_options();
@@ -528,12 +565,14 @@ int ss_prog_compile(ss_prog *p, const char *source, const char *kernel_names, ch
 }
 
 int ss_prog_cache_hit(ss_prog *p, int32_t *hit) {
+    P_LIVE(p);
     if (!p || !hit) P_FAIL(p, SS_ERR_INVALID, "NULL argument");
     *hit = p->cache_hit;
     return SS_OK;
 }
 
 int ss_prog_set_schedule(ss_prog *p, int32_t n, const int32_t *kernel, const int64_t *start, const int64_t *count) {
+    P_LIVE(p);
     if (!p || n < 0 || (n && (!kernel || !start || !count))) P_FAIL(p, SS_ERR_INVALID, "bad schedule");
     std::vector<Launch> s;
     for (int32_t i = 0; i < n; ++i) {
@@ -551,6 +590,7 @@ int ss_prog_set_schedule(ss_prog *p, int32_t n, const int32_t *kernel, const int
 }
 
 int ss_prog_set_order(ss_prog *p, const int32_t *order, int64_t n) {
+    P_LIVE(p);
     if (!p || n < 0 || (n && !order)) P_FAIL(p, SS_ERR_INVALID, "bad order");
     int64_t need = 0;
     for (const Launch &l : p->schedule) need += l.count;
@@ -584,6 +624,7 @@ int ss_prog_set_order(ss_prog *p, const int32_t *order, int64_t n) {
 // copy of every double-buffered array's write buffer into its read buffer
 // (model.py:2378-2406).
 int ss_prog_simulate(ss_prog *p, int64_t tick0, int64_t ticks) {
+    P_LIVE(p);
     if (!p || ticks < 0) P_FAIL(p, SS_ERR_INVALID, "bad arguments");
     if (!p->module) P_FAIL(p, SS_ERR_STATE, "no compiled step functions");
     hipStream_t st = p->ctx->stream;
@@ -613,6 +654,7 @@ int ss_prog_simulate(ss_prog *p, int64_t tick0, int64_t ticks) {
 static const uint64_t kProgMagic = 0x53534147455052ull;   // "SSAGEPR"
 
 int ss_prog_save(ss_prog *p, int64_t tick, void *buf, int64_t cap, int64_t *size) {
+    P_LIVE(p);
     if (!p || !size || cap < 0 || (cap && !buf)) P_FAIL(p, SS_ERR_INVALID, "bad arguments");
     int64_t need = 9 * 8 + 8 * p->n_globals;
     for (const ProgProp &q : p->props) need += 4 * 8 + (int64_t)((q.bytes() + 7) / 8 * 8);
@@ -639,6 +681,7 @@ int ss_prog_save(ss_prog *p, int64_t tick, void *buf, int64_t cap, int64_t *size
 }
 
 int ss_prog_restore(ss_prog *p, const void *buf, int64_t size, int64_t *tick) {
+    P_LIVE(p);
     if (!p || !buf || size < 9 * 8) P_FAIL(p, SS_ERR_INVALID, "bad arguments");
     const int64_t *h = static_cast<const int64_t *>(buf);
     if (h[0] != (int64_t)kProgMagic || h[1] != 1) P_FAIL(p, SS_ERR_INVALID, "not a program checkpoint");

@@ -480,6 +480,7 @@ int ss_destroy(ss_ctx *ctx) {
     (void)hipStreamSynchronize(ctx->stream);
     (void)hipStreamSynchronize(ctx->copy_stream);
     drop_graphs(ctx);
+    ss_release_programs(ctx);
     for (auto &r : ctx->reps) free_replica(r);
     dfree(ctx->d_reps);
     dfree(ctx->d_tiles);

@@ -81,6 +81,11 @@ hipError_t ss_launch_acc_init(const int8_t *st, const int64_t *row_ptr, int64_t 
 hipError_t ss_launch_symcheck(const int64_t *row_ptr, const int32_t *col_idx, int64_t n_rows,
                               unsigned long long *out, int grid, hipStream_t s);
 
+// Frees the device resources of every program of a context that is going
+// (rtc.hip); the programs themselves stay until ss_prog_destroy.
+struct ss_prog;
+void ss_release_programs(ss_ctx *ctx);
+
 // One replica's device allocations and host bookkeeping.
 struct ss_replica {
     bool live = false;
@@ -136,6 +141,7 @@ struct ss_ctx {
     hipStream_t stream = nullptr;
     hipStream_t copy_stream = nullptr;
     std::vector<ss_replica> reps;
+    std::vector<ss_prog *> progs;              // programs created on this context and not destroyed
     ss_rep_dev *d_reps = nullptr;              // device descriptor table
     ss_rep_dev *h_reps = nullptr;              // pinned host mirror
     int reps_cap = 0;
