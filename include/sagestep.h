@@ -339,6 +339,13 @@ int ss_prog_set_schedule(ss_prog *prog, int32_t n, const int32_t *kernel, const 
  * segment a permutation of its range), e.g. longest rows first so that the
  * threads of the longest rows start first; results do not depend on it. */
 int ss_prog_set_order(ss_prog *prog, const int32_t *order, int64_t n);
+/* After ss_prog_set_order: the first n_long[l] agents of launch l's order get
+ * a block each, with dynamic LDS for the longest of their rows (4 bytes an
+ * entry, at most 64 KB), before the blocks of the other agents; the launch's
+ * kernel then takes n_long as a sixth argument (long long).  n_launches
+ * entries, one per launch of the schedule; setting the schedule or the order
+ * clears it. */
+int ss_prog_set_long(ss_prog *prog, const int64_t *n_long, int32_t n_launches);
 /* Ticks tick0 .. tick0 + ticks - 1: the schedule, then write-back; waits. */
 int ss_prog_simulate(ss_prog *prog, int64_t tick0, int64_t ticks);
 /* Checkpoint of the program's state (replaces the pickle of Model.save /

@@ -66,6 +66,8 @@ struct Launch {
     int32_t kernel;
     int64_t start, count;
     int64_t order_off;          // first entry of this launch in the order array, -1: agents in index order
+    int64_t n_long = 0;         // agents at the front of the order that get a block each
+    int64_t long_deg = 0;       // entries of the longest of their rows
 };
 
 struct Extra {
@@ -167,7 +169,9 @@ struct ss_prog {
     hipModule_t module = nullptr;
     std::vector<hipFunction_t> kernels;
     std::vector<Launch> schedule;
+    std::vector<int64_t> h_row_ptr;             // row bounds, for the long rows' LDS
     int32_t *order = nullptr;                   // agent order of every launch (concatenated)
+    std::vector<int32_t> h_order;
     int64_t order_n = 0;
     int32_t seed = 0;
     int32_t cache_hit = 0;                      // the last compile came from the code-object cache
@@ -339,6 +343,8 @@ int ss_prog_set_csr(ss_prog *p, const int64_t *row_ptr, const int32_t *col_idx, 
     if (nnz) P_HIP(p, hipMemcpy(p->col_idx, col_idx, sizeof(int32_t) * nnz, hipMemcpyHostToDevice));
     P_HIP(p, hipMemcpy(p->row_ptr, row_ptr, sizeof(int64_t) * (p->n + 1), hipMemcpyHostToDevice));
     p->nnz = nnz;
+    p->h_row_ptr.assign(row_ptr, row_ptr + p->n + 1);
+    for (Launch &l : p->schedule) l.n_long = l.long_deg = 0;   // of the rows before
     p->csr_hash = fnv1a(fnv1a(1469598103934665603ull, row_ptr, sizeof(int64_t) * (size_t)(p->n + 1)), col_idx,
                         sizeof(int32_t) * (size_t)nnz);
     int rc = push_csr_globals(p);
@@ -608,6 +614,7 @@ int ss_prog_set_order(ss_prog *p, const int32_t *order, int64_t n) {
             seen[(size_t)a] = 1;
         }
         l.order_off = off;
+        l.n_long = l.long_deg = 0;
         off += l.count;
     }
     P_HIP(p, hipStreamSynchronize(p->ctx->stream));
@@ -616,6 +623,33 @@ int ss_prog_set_order(ss_prog *p, const int32_t *order, int64_t n) {
     P_HIP(p, hipMalloc((void **)&p->order, sizeof(int32_t) * (size_t)std::max<int64_t>(n, 1)));
     if (n) P_HIP(p, hipMemcpy(p->order, order, sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice));
     p->order_n = n;
+    p->h_order.assign(order, order + n);
+    return SS_OK;
+}
+
+int ss_prog_set_long(ss_prog *p, const int64_t *n_long, int32_t n_launches) {
+    P_LIVE(p);
+    if (!p || !n_long) P_FAIL(p, SS_ERR_INVALID, "NULL argument");
+    if (n_launches != (int32_t)p->schedule.size())
+        P_FAIL(p, SS_ERR_INVALID, "%d launches, the schedule has %zu", n_launches, p->schedule.size());
+    if (p->h_row_ptr.empty()) P_FAIL(p, SS_ERR_STATE, "no CSR");
+    std::vector<int64_t> deg(p->schedule.size(), 0);
+    for (size_t q = 0; q < p->schedule.size(); ++q) {
+        const Launch &l = p->schedule[q];
+        if (n_long[q] < 0 || n_long[q] > l.count || (n_long[q] > 0 && (l.order_off < 0 || !p->order)))
+            P_FAIL(p, SS_ERR_INVALID, "launch %zu: %lld long rows of %lld agents, or no order", q,
+                   (long long)n_long[q], (long long)l.count);
+        for (int64_t k = 0; k < n_long[q]; ++k) {
+            const int32_t i = p->h_order[(size_t)(l.order_off + k)];
+            deg[q] = std::max(deg[q], p->h_row_ptr[i + 1] - p->h_row_ptr[i]);
+        }
+        if (deg[q] * 4 > 65536) P_FAIL(p, SS_ERR_INVALID, "launch %zu: a row of %lld entries exceeds 64 KB of LDS", q,
+                                       (long long)deg[q]);
+    }
+    for (size_t q = 0; q < p->schedule.size(); ++q) {
+        p->schedule[q].n_long = n_long[q];
+        p->schedule[q].long_deg = deg[q];
+    }
     return SS_OK;
 }
 
@@ -635,9 +669,11 @@ int ss_prog_simulate(ss_prog *p, int64_t tick0, int64_t ticks) {
             const ProgArgsHost *a = p->d_args;
             long long start = l.start, count = l.count;
             const int32_t *ord = l.order_off >= 0 && p->order ? p->order + l.order_off : nullptr;
-            void *args[] = {(void *)&a, (void *)&tick, (void *)&start, (void *)&count, (void *)&ord};
-            const unsigned grid = (unsigned)((count + 255) / 256);
-            P_HIP(p, hipModuleLaunchKernel(p->kernels[l.kernel], grid, 1, 1, 256, 1, 1, 0, st, args, nullptr));
+            long long n_long = l.n_long;
+            void *args[] = {(void *)&a, (void *)&tick, (void *)&start, (void *)&count, (void *)&ord, (void *)&n_long};
+            const unsigned grid = (unsigned)(n_long + (count - n_long + 255) / 256);
+            P_HIP(p, hipModuleLaunchKernel(p->kernels[l.kernel], grid, 1, 1, 256, 1, 1, (unsigned)(4 * l.long_deg), st,
+                                           args, nullptr));
         }
         int rc = write_back(p, st);
         if (rc) return rc;

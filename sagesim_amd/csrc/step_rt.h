@@ -269,6 +269,29 @@ struct Locations {
     }
 };
 
+// The CSR as the step of an agent with a block to itself sees it: the running
+// agent's own row lies in the block's LDS.  Types of their own, so that no
+// flag has to be carried (and folded away) in the other agents' loops; both
+// convert to the plain ones, which read the same entries from memory.
+#define SS_RT_L __attribute__((address_space(3)))
+struct StagedRow {
+    const SS_RT_L int *l;
+    const int *p;
+    int n;
+    __device__ int operator[](long long j) const { return l[j]; }
+    __device__ operator NeighborRow() const { return NeighborRow{p, n}; }
+};
+__device__ inline int len(const StagedRow &row) { return row.n; }
+
+struct StagedLocations {
+    const long long *row_ptr;
+    const int *col_idx;
+    StagedRow own;
+    __device__ StagedRow operator[](const AgentIndex &) const { return own; }
+    __device__ NeighborRow operator[](long long i) const { return Locations{row_ptr, col_idx}[i]; }
+    __device__ operator Locations() const { return Locations{row_ptr, col_idx}; }
+};
+
 struct FloatArray {
     const float *p;
     __device__ float operator[](long long i) const { return ss_ld(p + i); }
@@ -279,6 +302,20 @@ struct GlobalArray {
     long long n;
     __device__ double operator[](long long i) const { return p[i]; }
 };
+
+// Copies the n entries at p to LDS by `width` threads, eight loads of a thread
+// in flight at a time.
+__device__ inline void ss_stage_row(const int *p, int n, SS_RT_L int *l, int me, int width) {
+#pragma clang loop unroll(disable)
+    for (int j = me; j < n; j += 8 * width) {
+        int x[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) x[q] = j + q * width < n ? ss_ld(p + j + q * width) : 0;
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+            if (j + q * width < n) l[j + q * width] = x[q];
+    }
+}
 
 // ---- helpers of utils.py:34-57 ----
 // The reference's step functions see the CSR as `neighbor_offsets` and
@@ -304,6 +341,8 @@ __device__ inline int get_neighbor(long long i, long long j, const NeighborOffse
 }
 __device__ inline int get_num_neighbors(long long i, const Locations &loc) { return loc[i].n; }
 __device__ inline int get_neighbor(long long i, long long j, const Locations &loc) { return loc[i][j]; }
+__device__ inline int get_num_neighbors(const AgentIndex &i, const StagedLocations &loc) { return loc[i].n; }
+__device__ inline int get_neighbor(const AgentIndex &i, long long j, const StagedLocations &loc) { return loc[i][j]; }
 template <class P>
 __device__ inline auto get_this_agent_data_from_tensor(long long i, const P &t) { return t[i]; }
 template <class P, class V>

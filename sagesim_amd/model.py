@@ -59,10 +59,76 @@ def build_csr_values_only(ragged_list, offsets):
 
 
 
-# Rows of the hipRTC path that start first (longest first): degree at least
-# _LONG_ROW_FACTOR times the priority group's mean and at least _LONG_ROW_MIN.
+# Agent order of the hipRTC path.  One thread runs an agent's step, so a tick
+# lasts as long as the longest row's walk: on BA(1M, 5), rows of up to 4076
+# entries, two dependent round trips for every 48 of them.  Long rows (degree at
+# least _LONG_ROW_FACTOR times the priority group's mean and at least
+# _LONG_ROW_MIN) start first, longest first, spread over the wavefronts so that
+# they do not share one's memory pipeline (109 -> 80 us a tick against 64 of them
+# to a wavefront).  Those of _STAGED_ROW_MIN to _STAGED_ROW_MAX entries get a
+# block each, which stages the row in LDS and so halves their round trips
+# (80 -> 70 us; the same for limits of 96 to 1024).
 _LONG_ROW_FACTOR = 8.0
 _LONG_ROW_MIN = 64.0
+_STAGED_ROW_MIN = 256
+_STAGED_ROW_MAX = 10_240          # 40 KB of LDS: four blocks per CU
+
+# Body of a wrapper whose first n_long agents have a block each.
+_LONG_ROW_KERNEL = """\
+    extern __shared__ int ss_row[];
+    if ((long long)blockIdx.x < n_long) {
+        const long long i = order[blockIdx.x];
+        const long long b = A->row_ptr[i];
+        int n = (int)(A->row_ptr[i + 1] - b);
+        ss_stage_row(A->col_idx + b, n, (SS_RT_L int *)ss_row, threadIdx.x, blockDim.x);
+        __syncthreads();
+        // a zero and a length the compiler takes for values of the lane: entries
+        // at uniform addresses would make the step's gathers scalar loads, one at
+        // a time, and a length it can take apart keeps some compiler versions
+        // from unrolling the step's loop
+        int lane = 0;
+        asm volatile("" : "+v"(lane), "+v"(n));
+        if (threadIdx.x == 0)
+            ss_step_@P@(A, tick, i, StagedLocations{A->row_ptr, A->col_idx,
+                                                  {(const SS_RT_L int *)ss_row + lane, A->col_idx + b, n}});
+        return;
+    }
+    const long long k = n_long + ((long long)blockIdx.x - n_long) * blockDim.x + threadIdx.x;
+    if (k >= count) return;
+    ss_step_@P@(A, tick, order[k], Locations{A->row_ptr, A->col_idx});
+}"""
+
+
+_NO_ROWS = np.zeros(0, np.int64)
+
+
+def _agent_order(deg, stage=True):
+    """Order of a priority group's agents (their degrees in buffer order) and
+    how many of the first get a block each (see above; none without `stage`)."""
+    if deg.size == 0:
+        return _NO_ROWS, 0
+    cut = max(_LONG_ROW_MIN, _LONG_ROW_FACTOR * float(deg.mean()))
+    staged = np.nonzero((deg >= max(cut, _STAGED_ROW_MIN)) & (deg <= _STAGED_ROW_MAX))[0] if stage else _NO_ROWS
+    staged = staged[np.argsort(-deg[staged], kind="stable")]
+    is_long = deg >= cut
+    is_long[staged] = False
+    spread = np.nonzero(is_long)[0]
+    spread = spread[np.argsort(-deg[spread], kind="stable")]
+    mine = np.ones(deg.size, bool)
+    mine[staged] = False
+    mine[spread] = False
+    m = deg.size - staged.size
+    waves = max(1, min(spread.size, m // 64))
+    body = np.empty(m, np.int64)
+    at = (np.arange(spread.size) % waves) * 64 + np.arange(spread.size) // waves
+    if spread.size and at.max() >= m:                  # too few agents to spread over
+        at = np.arange(spread.size)
+    taken = np.zeros(m, bool)
+    taken[at] = True
+    body[at] = spread
+    body[~taken] = np.nonzero(mine)[0]
+    return np.concatenate([staged, body]), int(staged.size)
+
 
 class _Program:
     """Owner of one ss_prog (general step functions)."""
@@ -518,12 +584,14 @@ class Model:
     def _no_double_buffer(self):
         return set().union(*(b.no_double_buffer_props for b in self._breeds)) if self._breeds else set()
 
-    def generate_source(self, groups=None):
+    def generate_source(self, groups=None, long_groups=()):
         """HIP source of the step kernels: the breeds' step functions plus one
         `ss_prio_<p>` wrapper per priority group that calls each breed's step
         function with the reference's argument order (model.py:2302-2337):
         tick, agent_index, globals, agent_ids, breeds, locations, properties
-        in registration order, then `array, idx_map` per breed-local array."""
+        in registration order, then `array, idx_map` per breed-local array.
+        The wrappers of the priority groups in long_groups give each of the
+        first n_long agents of their order a block."""
         if groups is None:
             _, groups = self._priority_groups()
         lines = []
@@ -588,17 +656,26 @@ class Model:
         for p, grp in enumerate(groups):
             kname = f"ss_prio_{p}"
             names.append(kname)
-            lines.append(f'extern "C" __global__ void {kname}(const SSProgArgs *__restrict__ A, long long tick, '
-                         f"long long start, long long count, const int *__restrict__ order) {{")
-            lines.append("    const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;")
-            lines.append("    if (k >= count) return;")
-            lines.append("    const long long i = order ? (long long)order[k] : start + k;")
+            head = (f'extern "C" __global__ void {kname}(const SSProgArgs *__restrict__ A, long long tick, '
+                    f"long long start, long long count, const int *__restrict__ order")
+            has_long = p in long_groups
+            if has_long:
+                # the step of agent i, called by the two kinds of blocks below
+                lines.append("template <class L>")
+                lines.append(f"static __device__ __forceinline__ void ss_step_{p}(const SSProgArgs *__restrict__ A, "
+                             "long long tick, long long i, const L &locations) {")
+            else:
+                lines.append(head + ") {")
+                lines.append("    const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;")
+                lines.append("    if (k >= count) return;")
+                lines.append("    const long long i = order ? (long long)order[k] : start + k;")
             lines.append("    const int breed = (int)A->breeds[i];")
             lines.append("    const AgentIndex agent_index{i, A->logical_ids[i], A->seed, A->logical_ids64[i]};")
             lines.append("    const long long _real_idx = i, thread_local_tick = tick; const int breed_id = breed;")
             lines.append("    (void)_real_idx; (void)thread_local_tick; (void)breed_id;")
             lines.append("    const FloatArray agent_ids{A->agent_ids}, breeds{A->breeds};")
-            lines.append("    const Locations locations{A->row_ptr, A->col_idx};")
+            if not has_long:
+                lines.append("    const Locations locations{A->row_ptr, A->col_idx};")
             lines += gdecl + pdecl + bdecl + xdecl
             for b, fn in grp.items():
                 args = ", ".join(["tick", "agent_index"] + gargs + ["agent_ids", "breeds", "locations"] + pargs
@@ -619,6 +696,9 @@ class Model:
                 lines.append("        return;")
                 lines.append("    }")
             lines.append("}")
+            if has_long:
+                lines.append(head + ", long long n_long) {")
+                lines += _LONG_ROW_KERNEL.replace("@P@", str(p)).splitlines()
             lines.append("")
         return "\n".join(lines), names
 
@@ -658,21 +738,10 @@ class Model:
             self._bla_ids.append((aid.value, xid.value, rows))
         self._prog = prog
         self._push_globals()
-        src, names = self.generate_source(groups)
-        if self._step_function_file_path:
-            with open(os.path.abspath(self._step_function_file_path), "w") as f:
-                f.write(src)
-        log = ctypes.create_string_buffer(1 << 16)
-        rc = L.ss_prog_compile(h, src.encode(), "\n".join(names).encode(), log, len(log))
-        if rc:
-            raise NativeError(rc, L.ss_prog_last_error(h).decode())
-        self._push_seed()
         # schedule: priority group p covers the breed-sorted range of its breeds
-        # (model.py:1051-1062); within it the long rows (see _LONG_ROW_FACTOR)
-        # start first, longest first, and the rest follow in buffer order, so
-        # that most threads read their agent's fields from consecutive slots
+        # (model.py:1051-1062), in the order of _agent_order
         deg = np.diff(np.asarray(rp, np.int64))
-        kern, start, count, segs = [], [], [], []
+        kern, start, count, orders = [], [], [], []
         for p, grp in enumerate(groups):
             lo, hi = n, 0
             for b in grp:
@@ -684,18 +753,34 @@ class Model:
             kern.append(p)
             start.append(lo)
             count.append(hi - lo)
-            d = deg[lo:hi]
-            cut = max(_LONG_ROW_MIN, _LONG_ROW_FACTOR * float(d.mean())) if d.size else 0.0
-            long_rows = np.nonzero(d >= cut)[0]
-            long_rows = long_rows[np.argsort(-d[long_rows], kind="stable")]
-            rest = np.nonzero(d < cut)[0]
-            segs.append(lo + np.concatenate([long_rows, rest]))
+            orders.append(_agent_order(deg[lo:hi]))
+        log = ctypes.create_string_buffer(1 << 16)
+
+        def compile_source():
+            src, names = self.generate_source(groups, [p for p, o in enumerate(orders) if o[1]])
+            return src, L.ss_prog_compile(h, src.encode(), "\n".join(names).encode(), log, len(log))
+        src, rc = compile_source()
+        if rc and any(o[1] for o in orders):
+            # a step that does not compile against the staged rows' types (say,
+            # one that assigns rows to each other) runs without them
+            orders = [_agent_order(deg[lo:lo + c], stage=False) for lo, c in zip(start, count)]
+            src, rc = compile_source()
+        if self._step_function_file_path:
+            with open(os.path.abspath(self._step_function_file_path), "w") as f:
+                f.write(src)
+        if rc:
+            raise NativeError(rc, L.ss_prog_last_error(h).decode())
+        self._push_seed()
         k = np.asarray(kern, np.int32)
         s = np.asarray(start, np.int64)
         c = np.asarray(count, np.int64)
         prog.ck(L.ss_prog_set_schedule(h, len(k), ptr(k), ptr(s), ptr(c)))
+        segs = [lo + o[0] for lo, o in zip(start, orders)]
         ordr = np.ascontiguousarray(np.concatenate(segs) if segs else np.zeros(0), np.int32)
         prog.ck(L.ss_prog_set_order(h, ptr(ordr), ordr.shape[0]))
+        nl = np.asarray([o[1] for o in orders], np.int64)
+        if nl.any():
+            prog.ck(L.ss_prog_set_long(h, ptr(nl), len(nl)))
 
     def _push_globals(self):
         if self._mode == "fused":
