@@ -320,6 +320,10 @@ int ss_prog_set_seed(ss_prog *prog, int64_t seed);
  * the wrapper kernels as SSProgArgs::extra[slot]; read back after a run */
 int ss_prog_set_extra(ss_prog *prog, int32_t slot, int64_t bytes, const void *data);
 int ss_prog_get_extra(ss_prog *prog, int32_t slot, int64_t bytes, void *out);
+/* How often the next compile unrolls the step functions' loops (1..128; 48
+ * when never called; SAGESIM_AMD_RTC_UNROLL overrides it): a count that fits
+ * the longest rows a thread walks.  Results do not depend on it. */
+int ss_prog_set_unroll(ss_prog *prog, int32_t count);
 /* Compile `source` for gfx950 and load the kernels named in `kernel_names`
  * ('\n'-separated); the hipRTC log is copied into `log` (may be NULL).  Code
  * objects are cached by a hash of the source, the runtime header and the
@@ -346,6 +350,11 @@ int ss_prog_set_order(ss_prog *prog, const int32_t *order, int64_t n);
  * entries, one per launch of the schedule; setting the schedule or the order
  * clears it. */
 int ss_prog_set_long(ss_prog *prog, const int64_t *n_long, int32_t n_launches);
+/* Small programs: kernel `kernel` (const SSProgArgs*, long long tick, long long
+ * ticks) runs whole ticks, schedule and write-back, on one block of `threads`
+ * threads; ss_prog_simulate then launches it once a call instead of the
+ * schedule.  -1: none (also after every compile). */
+int ss_prog_set_loop(ss_prog *prog, int32_t kernel, int32_t threads);
 /* Ticks tick0 .. tick0 + ticks - 1: the schedule, then write-back; waits. */
 int ss_prog_simulate(ss_prog *prog, int64_t tick0, int64_t ticks);
 /* Checkpoint of the program's state (replaces the pickle of Model.save /

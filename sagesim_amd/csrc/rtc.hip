@@ -86,14 +86,15 @@ uint64_t fnv1a(uint64_t h, const void *p, size_t n) {
 
 // Loops of unknown trip count (a step function's walk over its neighbour row)
 // are unrolled at run time, so one thread has several neighbour loads in
-// flight instead of one round trip per neighbour; SAGESIM_AMD_RTC_UNROLL
-// sets the count (1 disables it) and SAGESIM_AMD_RTC_UNROLL_THRESHOLD the
-// size the unrolled body may reach (LLVM lowers the count of a loop whose
-// body would grow past it: a heavy loop body unrolls less).
-std::vector<std::string> rtc_options() {
+// flight instead of one round trip per neighbour; entries beyond the last whole
+// round run one at a time, so the count has to fit the rows
+// (ss_prog_set_unroll; 48 by default).  SAGESIM_AMD_RTC_UNROLL overrides the
+// count (1 disables it) and SAGESIM_AMD_RTC_UNROLL_THRESHOLD the size the
+// unrolled body may reach (LLVM lowers the count of a loop whose body would
+// grow past it: a heavy loop body unrolls less).
+std::vector<std::string> rtc_options(int unroll) {
     std::vector<std::string> o = {"--offload-arch=gfx950", "-O3", "-std=c++20", "-ffp-contract=off",
                                   "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"};
-    int unroll = 48;
     std::string threshold = "1200";
     if (const char *u = std::getenv("SAGESIM_AMD_RTC_UNROLL")) unroll = std::atoi(u);
     if (const char *t = std::getenv("SAGESIM_AMD_RTC_UNROLL_THRESHOLD")) threshold = t;
@@ -139,13 +140,21 @@ void write_file_atomic(const std::string &dir, const std::string &name, const st
     std::rename(tmp.c_str(), (dir + "/" + name).c_str());
 }
 
-__global__ void writeback_kernel(const uint4 *__restrict__ src, uint4 *__restrict__ dst, int64_t n16,
-                                 const unsigned char *__restrict__ src_b, unsigned char *__restrict__ dst_b,
-                                 int64_t tail_from, int64_t n_bytes) {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// Write buffer -> read buffer of every double-buffered array, one launch:
+// block row y copies array y.  Bound by the launch at small sizes (2.2 us each,
+// a launch per array before) and by the copy at large ones.
+struct WriteBack {
+    const void *src[SS_MAXP_HOST];
+    void *dst[SS_MAXP_HOST];
+    int64_t bytes[SS_MAXP_HOST];
+};
+__global__ __launch_bounds__(256) void writeback_kernel(const WriteBack w) {
+    const int64_t nb = w.bytes[blockIdx.y], n16 = nb / 16;
+    const uint4 *src = (const uint4 *)w.src[blockIdx.y];
+    uint4 *dst = (uint4 *)w.dst[blockIdx.y];
+    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t i = g; i < n16; i += stride) dst[i] = src[i];
-    for (int64_t i = tail_from + g; i < n_bytes; i += stride) dst_b[i] = src_b[i];
+    for (int64_t i = n16 * 16 + g; i < nb; i += stride) ((unsigned char *)dst)[i] = ((const unsigned char *)src)[i];
 }
 
 }  // namespace
@@ -169,11 +178,14 @@ struct ss_prog {
     hipModule_t module = nullptr;
     std::vector<hipFunction_t> kernels;
     std::vector<Launch> schedule;
+    int32_t loop_kernel = -1;                   // kernel that runs whole ticks on one block, -1: none
+    int32_t loop_threads = 0;
     std::vector<int64_t> h_row_ptr;             // row bounds, for the long rows' LDS
     int32_t *order = nullptr;                   // agent order of every launch (concatenated)
     std::vector<int32_t> h_order;
     int64_t order_n = 0;
     int32_t seed = 0;
+    int32_t unroll = 48;                        // neighbour-loop unroll count of the next compile
     int32_t cache_hit = 0;                      // the last compile came from the code-object cache
     std::string err;
 };
@@ -251,15 +263,20 @@ static int push_seed(ss_prog *p) {
 
 // copy every double-buffered array's write buffer into its read buffer
 static int write_back(ss_prog *p, hipStream_t st) {
+    WriteBack w{};
+    int n = 0;
+    int64_t most = 0;
     for (const ProgProp &q : p->props) {
         if (!q.double_buffered || q.rows == 0) continue;
-        const int64_t nb = (int64_t)q.bytes();
-        const int64_t n16 = nb / 16;
-        int grid = (int)std::min<int64_t>(std::max<int64_t>((n16 + 255) / 256, 1), (int64_t)p->ctx->num_cus * 4);
-        hipLaunchKernelGGL(writeback_kernel, dim3(grid), dim3(256), 0, st, (const uint4 *)q.w, (uint4 *)q.r, n16,
-                           (const unsigned char *)q.w, (unsigned char *)q.r, n16 * 16, nb);
-        P_HIP(p, hipGetLastError());
+        w.src[n] = q.w;
+        w.dst[n] = q.r;
+        w.bytes[n] = (int64_t)q.bytes();
+        most = std::max(most, w.bytes[n++]);
     }
+    if (n == 0) return SS_OK;
+    const int grid = (int)std::min<int64_t>(std::max<int64_t>((most / 16 + 255) / 256, 1), (int64_t)p->ctx->num_cus * 4);
+    hipLaunchKernelGGL(writeback_kernel, dim3(grid, n), dim3(256), 0, st, w);
+    P_HIP(p, hipGetLastError());
     return SS_OK;
 }
 
@@ -488,11 +505,18 @@ int ss_prog_get_extra(ss_prog *p, int32_t slot, int64_t bytes, void *out) {
     return SS_OK;
 }
 
+int ss_prog_set_unroll(ss_prog *p, int32_t count) {
+    if (!p || count < 1 || count > 128) P_FAIL(p, SS_ERR_INVALID, "unroll count must be 1..128");
+    P_LIVE(p);
+    p->unroll = count;
+    return SS_OK;
+}
+
 int ss_prog_compile(ss_prog *p, const char *source, const char *kernel_names, char *log, int64_t log_cap) {
     P_LIVE(p);
     if (!p || !source || !kernel_names) P_FAIL(p, SS_ERR_INVALID, "NULL argument");
     if (log && log_cap > 0) log[0] = 0;
-    const std::vector<std::string> opts_s = rtc_options();
+    const std::vector<std::string> opts_s = rtc_options(p->unroll);
     std::vector<const char *> opts;
     for (const auto &o : opts_s) opts.push_back(o.c_str());
     uint64_t key = 1469598103934665603ull;
@@ -550,6 +574,7 @@ int ss_prog_compile(ss_prog *p, const char *source, const char *kernel_names, ch
         p->module = nullptr;
     }
     p->kernels.clear();
+    p->loop_kernel = -1;
     P_HIP(p, hipModuleLoadData(&p->module, code.data()));
     std::string names_s(kernel_names);
     size_t pos = 0;
@@ -653,6 +678,16 @@ int ss_prog_set_long(ss_prog *p, const int64_t *n_long, int32_t n_launches) {
     return SS_OK;
 }
 
+int ss_prog_set_loop(ss_prog *p, int32_t kernel, int32_t threads) {
+    if (!p) P_FAIL(p, SS_ERR_INVALID, "NULL argument");
+    P_LIVE(p);
+    if (kernel < -1 || kernel >= (int32_t)p->kernels.size() || threads < 64 || threads > 1024 || threads % 64)
+        P_FAIL(p, SS_ERR_INVALID, "kernel %d of %zu with %d threads", kernel, p->kernels.size(), threads);
+    p->loop_kernel = kernel;
+    p->loop_threads = threads;
+    return SS_OK;
+}
+
 // Every tick: the launches of the schedule in order (a kernel boundary
 // between priority groups is the grid barrier of model.py:2356-2366), then the
 // copy of every double-buffered array's write buffer into its read buffer
@@ -662,6 +697,18 @@ int ss_prog_simulate(ss_prog *p, int64_t tick0, int64_t ticks) {
     if (!p || ticks < 0) P_FAIL(p, SS_ERR_INVALID, "bad arguments");
     if (!p->module) P_FAIL(p, SS_ERR_STATE, "no compiled step functions");
     hipStream_t st = p->ctx->stream;
+    if (p->loop_kernel >= 0) {
+        // at most 4096 ticks (tens of milliseconds) a launch
+        for (int64_t k = 0; k < ticks; k += 4096) {
+            const ProgArgsHost *a = p->d_args;
+            long long tick = (long long)(tick0 + k), n_ticks = (long long)std::min<int64_t>(ticks - k, 4096);
+            void *args[] = {(void *)&a, (void *)&tick, (void *)&n_ticks};
+            P_HIP(p, hipModuleLaunchKernel(p->kernels[p->loop_kernel], 1, 1, 1, (unsigned)p->loop_threads, 1, 1, 0, st,
+                                           args, nullptr));
+        }
+        P_HIP(p, hipStreamSynchronize(st));
+        return SS_OK;
+    }
     for (int64_t k = 0; k < ticks; ++k) {
         long long tick = (long long)(tick0 + k);
         for (const Launch &l : p->schedule) {

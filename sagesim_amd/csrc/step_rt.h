@@ -317,6 +317,16 @@ __device__ inline void ss_stage_row(const int *p, int n, SS_RT_L int *l, int me,
     }
 }
 
+// Write buffer -> read buffer of one array by the block's threads.
+__device__ inline void ss_write_back(const void *w, void *r, long long bytes, int me, int width) {
+    const long long words = bytes / 4;
+#pragma clang loop unroll(disable)
+    for (long long k = me; k < words; k += width) ss_st((unsigned int *)r + k, ss_ld((const unsigned int *)w + k));
+#pragma clang loop unroll(disable)
+    for (long long k = 4 * words + me; k < bytes; k += width)
+        ss_st((unsigned char *)r + k, ss_ld((const unsigned char *)w + k));
+}
+
 // ---- helpers of utils.py:34-57 ----
 // The reference's step functions see the CSR as `neighbor_offsets` and
 // `neighbor_values` (model.py:1845-1900 renames `locations`), and its helpers

@@ -73,6 +73,23 @@ _LONG_ROW_MIN = 64.0
 _STAGED_ROW_MIN = 256
 _STAGED_ROW_MAX = 10_240          # 40 KB of LDS: four blocks per CU
 
+# Small models run whole ticks on one block, the loop over ticks inside the
+# kernel, instead of a launch per priority group and tick: both limits are
+# where one compute unit's work catches up with the launches (us a tick,
+# launches / one block: rows of 20, 1000 agents 10.0 / 6.9 and 2000 agents
+# 10.4 / 12.4; rows of 6, 2000 agents 7.6 / 5.9; two breeds at three
+# priorities, 1000 agents 18.5 / 8.2 and 2000 agents 14.2 / 13.2).
+_LOOP_AGENTS = 2048
+_LOOP_ENTRIES = 24_000
+# Neighbour loops unrolled, by the longest row a thread walks alone (up to the
+# first entry, up to the second, longer or staged): a round's loads are in
+# flight together, but what is left of a row after its last whole round goes one
+# entry at a time.  us a tick at 48 / 16 / 6: rows of 20, 1000 agents 7.1 / 4.7 /
+# 4.6; ER of mean 6, two breeds, 50k agents 21.3 / 20.5 / 15.2; ER of mean 12,
+# 300k agents 16.5 / 15.1 / 12.9; BA(3000, 5), two breeds 30.8 / 25.1 / 27.1;
+# BA(200k, 5), staged 27.7 / 32.3 / 45.9.
+_UNROLL_ROWS, _UNROLL = (64, 1024), (6, 16, 48)
+
 # Body of a wrapper whose first n_long agents have a block each.
 _LONG_ROW_KERNEL = """\
     extern __shared__ int ss_row[];
@@ -584,14 +601,16 @@ class Model:
     def _no_double_buffer(self):
         return set().union(*(b.no_double_buffer_props for b in self._breeds)) if self._breeds else set()
 
-    def generate_source(self, groups=None, long_groups=()):
+    def generate_source(self, groups=None, long_groups=(), loop=None):
         """HIP source of the step kernels: the breeds' step functions plus one
         `ss_prio_<p>` wrapper per priority group that calls each breed's step
         function with the reference's argument order (model.py:2302-2337):
         tick, agent_index, globals, agent_ids, breeds, locations, properties
         in registration order, then `array, idx_map` per breed-local array.
         The wrappers of the priority groups in long_groups give each of the
-        first n_long agents of their order a block."""
+        first n_long agents of their order a block.  loop, the (first agent,
+        agents) of every group, adds `ss_ticks`, which runs whole ticks on one
+        block."""
         if groups is None:
             _, groups = self._priority_groups()
         lines = []
@@ -659,8 +678,9 @@ class Model:
             head = (f'extern "C" __global__ void {kname}(const SSProgArgs *__restrict__ A, long long tick, '
                     f"long long start, long long count, const int *__restrict__ order")
             has_long = p in long_groups
-            if has_long:
-                # the step of agent i, called by the two kinds of blocks below
+            split = has_long or loop is not None
+            if split:
+                # the step of agent i, called by the kernels below
                 lines.append("template <class L>")
                 lines.append(f"static __device__ __forceinline__ void ss_step_{p}(const SSProgArgs *__restrict__ A, "
                              "long long tick, long long i, const L &locations) {")
@@ -674,7 +694,7 @@ class Model:
             lines.append("    const long long _real_idx = i, thread_local_tick = tick; const int breed_id = breed;")
             lines.append("    (void)_real_idx; (void)thread_local_tick; (void)breed_id;")
             lines.append("    const FloatArray agent_ids{A->agent_ids}, breeds{A->breeds};")
-            if not has_long:
+            if not split:
                 lines.append("    const Locations locations{A->row_ptr, A->col_idx};")
             lines += gdecl + pdecl + bdecl + xdecl
             for b, fn in grp.items():
@@ -699,8 +719,38 @@ class Model:
             if has_long:
                 lines.append(head + ", long long n_long) {")
                 lines += _LONG_ROW_KERNEL.replace("@P@", str(p)).splitlines()
+            elif split:
+                lines.append(head + ") {")
+                lines.append("    const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;")
+                lines.append("    if (k >= count) return;")
+                lines.append(f"    ss_step_{p}(A, tick, order ? (long long)order[k] : start + k, "
+                             "Locations{A->row_ptr, A->col_idx});")
+                lines.append("}")
             lines.append("")
+        if loop is not None:
+            names.append("ss_ticks")
+            lines += ['extern "C" __global__ __launch_bounds__(1024) void ss_ticks(const SSProgArgs *__restrict__ A, '
+                      "long long tick, long long ticks) {",
+                      "#pragma clang loop unroll(disable)",
+                      "    for (long long t = tick; t < tick + ticks; ++t) {"]
+            for p, (start, count) in enumerate(loop):
+                lines += ["#pragma clang loop unroll(disable)",
+                          f"        for (int k = threadIdx.x; k < {count}; k += blockDim.x)",
+                          f"            ss_step_{p}(A, t, {start}LL + k, Locations{{A->row_ptr, A->col_idx}});",
+                          "        __syncthreads();"]
+            for aid, nbytes in self._double_buffered():
+                lines.append(f"        ss_write_back(A->prop_w[{aid}], A->prop_r[{aid}], {nbytes}LL, threadIdx.x, "
+                             "blockDim.x);")
+            lines += ["        __syncthreads();", "    }", "}", ""]
         return "\n".join(lines), names
+
+    def _double_buffered(self):
+        """(array id, bytes) of every double-buffered property and breed-local array."""
+        nodb = self._no_double_buffer()
+        out = [(self._prop_index[name], self._host_props[name].nbytes) for name in self._prop_names[2:] if name not in nodb]
+        out += [(aid, rows * int(np.prod(bla["shape_per_agent"])) * 4)
+                for bla, (aid, _, rows) in zip(self._breed_local_arrays, self._bla_ids) if bla["name"] not in nodb]
+        return out
 
     def _setup_rtc(self, groups, rp, ci, order, logical):
         self._mode = "rtc"
@@ -756,14 +806,23 @@ class Model:
             orders.append(_agent_order(deg[lo:hi]))
         log = ctypes.create_string_buffer(1 << 16)
 
+        small = (n <= _LOOP_AGENTS and len(ci) <= _LOOP_ENTRIES and groups and not any(o[1] for o in orders))
+
         def compile_source():
-            src, names = self.generate_source(groups, [p for p, o in enumerate(orders) if o[1]])
+            src, names = self.generate_source(groups, [p for p, o in enumerate(orders) if o[1]],
+                                              list(zip(start, count)) if small else None)
             return src, L.ss_prog_compile(h, src.encode(), "\n".join(names).encode(), log, len(log))
+        def set_unroll():
+            longest = max(int(deg.max(initial=0)), _UNROLL_ROWS[-1] + 1 if any(o[1] for o in orders) else 0)
+            prog.ck(L.ss_prog_set_unroll(h, _UNROLL[sum(longest > r for r in _UNROLL_ROWS)]))
+        set_unroll()
         src, rc = compile_source()
-        if rc and any(o[1] for o in orders):
-            # a step that does not compile against the staged rows' types (say,
-            # one that assigns rows to each other) runs without them
+        if rc and (small or any(o[1] for o in orders)):
+            # what compiles only in a plain wrapper (a step that assigns rows to
+            # each other, whose staged rows have other types) runs in one
+            small = False
             orders = [_agent_order(deg[lo:lo + c], stage=False) for lo, c in zip(start, count)]
+            set_unroll()
             src, rc = compile_source()
         if self._step_function_file_path:
             with open(os.path.abspath(self._step_function_file_path), "w") as f:
@@ -775,9 +834,13 @@ class Model:
         s = np.asarray(start, np.int64)
         c = np.asarray(count, np.int64)
         prog.ck(L.ss_prog_set_schedule(h, len(k), ptr(k), ptr(s), ptr(c)))
-        segs = [lo + o[0] for lo, o in zip(start, orders)]
-        ordr = np.ascontiguousarray(np.concatenate(segs) if segs else np.zeros(0), np.int32)
-        prog.ck(L.ss_prog_set_order(h, ptr(ordr), ordr.shape[0]))
+        if any(not np.array_equal(o[0], np.arange(o[0].size)) for o in orders):
+            segs = [lo + o[0] for lo, o in zip(start, orders)]
+            ordr = np.ascontiguousarray(np.concatenate(segs), np.int32)
+            prog.ck(L.ss_prog_set_order(h, ptr(ordr), ordr.shape[0]))
+        if small:
+            threads = min(1024, max(64, -(-max(count) // 64) * 64))
+            prog.ck(L.ss_prog_set_loop(h, len(k), threads))
         nl = np.asarray([o[1] for o in orders], np.int64)
         if nl.any():
             prog.ck(L.ss_prog_set_long(h, ptr(nl), len(nl)))
