@@ -70,14 +70,42 @@ __device__ __forceinline__ int32_t map_find(const unsigned long long *__restrict
     return -1;
 }
 
-__global__ void map_lookup_kernel(const unsigned long long *__restrict__ keys, const int32_t *__restrict__ vals,
-                                  int64_t cap, const int64_t *__restrict__ ids, int32_t *__restrict__ out,
-                                  int64_t n, int32_t *misses) {
-    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= n) return;
-    const int32_t v = map_find(keys, vals, cap, ids[g]);
-    out[g] = v;
-    if (v < 0 && misses) atomicAdd(misses, 1);
+// counts[0] += lookups that found nothing, counts[1] = min of the slots found
+// (as unsigned words; LOWEST only).  One atomic per block and count: they run
+// one after another.
+template <bool LOWEST>
+__global__ __launch_bounds__(256) void map_lookup_kernel(const unsigned long long *__restrict__ keys,
+                                                         const int32_t *__restrict__ vals, int64_t cap,
+                                                         const int64_t *__restrict__ ids, int32_t *__restrict__ out,
+                                                         int64_t n, uint32_t *counts) {
+    __shared__ uint32_t miss, low;
+    if (threadIdx.x == 0) {
+        miss = 0u;
+        low = ~0u;
+    }
+    __syncthreads();
+    uint32_t m = 0u, lo = ~0u;
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < n; g += stride) {
+        const int32_t v = map_find(keys, vals, cap, ids[g]);
+        out[g] = v;
+        if (v < 0) ++m;
+        else if ((uint32_t)v < lo) lo = (uint32_t)v;
+    }
+    if (m) atomicAdd(&miss, m);
+    if (LOWEST && lo != ~0u) atomicMin(&low, lo);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        if (miss) atomicAdd(&counts[0], miss);
+        if (LOWEST && low != ~0u) atomicMin(&counts[1], low);
+    }
+}
+
+// rec[slot[h] - base] = the last record h of every slot (rec cleared to -1)
+__global__ __launch_bounds__(256) void halo_records_kernel(const int32_t *__restrict__ slot, int64_t n, int64_t base,
+                                                           int32_t *rec) {
+    const int64_t h = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (h < n && slot[h] >= 0) atomicMax(&rec[slot[h] - base], (int32_t)h);
 }
 
 __global__ void fill_i32_kernel(int32_t *p, int64_t n, int32_t v) {
@@ -340,10 +368,21 @@ hipError_t ss_launch_bits(const int8_t *st, uint64_t *bits, int64_t w0, int64_t 
 }
 
 hipError_t ss_launch_map_lookup(const unsigned long long *keys, const int32_t *vals, int64_t cap, const int64_t *ids,
-                                int32_t *out, int64_t n, int32_t *misses, hipStream_t s) {
+                                int32_t *out, int64_t n, uint32_t *counts, bool lowest, int num_cus, hipStream_t s) {
     if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(map_lookup_kernel, dim3(grid_for(n, 256)), dim3(256), 0, s, keys, vals, cap, ids, out, n,
-                       misses);
+    const unsigned grid = std::min(grid_for(n, 256), (unsigned)num_cus * 8u);
+    if (lowest)
+        hipLaunchKernelGGL(map_lookup_kernel<true>, dim3(grid), dim3(256), 0, s, keys, vals, cap, ids, out, n, counts);
+    else
+        hipLaunchKernelGGL(map_lookup_kernel<false>, dim3(grid), dim3(256), 0, s, keys, vals, cap, ids, out, n, counts);
+    return hipGetLastError();
+}
+
+hipError_t ss_launch_halo_records(const int32_t *slot, int64_t n, int64_t base, int32_t *rec, int64_t n_rec,
+                                  hipStream_t s) {
+    hipError_t e = ss_launch_fill_i32(rec, n_rec, -1, s);
+    if (e != hipSuccess || n <= 0) return e;
+    hipLaunchKernelGGL(halo_records_kernel, dim3(grid_for(n, 256)), dim3(256), 0, s, slot, n, base, rec);
     return hipGetLastError();
 }
 

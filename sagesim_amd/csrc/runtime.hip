@@ -50,8 +50,9 @@ void dfree(void *p) {
 }
 
 // The context's workspace, at least b bytes (256-byte aligned): kept for later
-// calls, replaced by a larger one when it is too small, freed with the context.
-// Every user runs on the context's stream and is done with it when it returns.
+// calls, replaced by a larger one when it is too small, freed with the context
+// (and by a Scratch guard's end when it is larger than what is worth keeping).  Every
+// user runs on the context's stream and is done with it when it returns.
 hipError_t scratch(ss_ctx *ctx, size_t b, void **p) {
     if (ctx->scratch_bytes < b) {
         hipError_t e = hipStreamSynchronize(ctx->stream);
@@ -71,6 +72,23 @@ hipError_t scratch(ss_ctx *ctx, size_t b, void **p) {
     *p = ctx->scratch;
     return hipSuccess;
 }
+
+const size_t kScratchKept = 256u << 20;
+
+struct Scratch {
+    ss_ctx *ctx;
+    explicit Scratch(ss_ctx *c) : ctx(c) {}
+    ~Scratch() {
+        if (ctx->scratch_bytes <= kScratchKept) return;
+        (void)hipStreamSynchronize(ctx->stream);
+        dfree(ctx->scratch);
+        ctx->scratch = nullptr;
+        ctx->bytes -= ctx->scratch_bytes;
+        ctx->scratch_bytes = 0;
+    }
+};
+
+inline size_t up256(size_t b) { return (b + 255) / 256 * 256; }
 
 // inf_T[k] = ceil(p_k * 2^23), p_k = 1 - q_k, q_k = q_{k-1} * (1 - beta),
 // for k = 0 .. min(max_deg, first k with p_k * 2^23 == 2^23).
@@ -151,7 +169,7 @@ void free_replica(ss_replica &r) {
     dfree(r.history); dfree(r.init_history); dfree(r.inf_T);
     dfree(r.cnt[0]); dfree(r.cnt[1]); dfree(r.dec); dfree(r.acc);
     dfree(r.order);
-    dfree(r.map_keys); dfree(r.map_vals); dfree(r.halo_slots);
+    dfree(r.map_keys); dfree(r.map_vals);
     for (auto &d : r.halo_dev) dfree(d);
     for (auto &d : r.halo_grp) dfree(d);
     dfree((void *)r.halo_ptrs);
@@ -977,12 +995,21 @@ int ss_simulate(ss_ctx *ctx, int64_t ticks) {
 
 // ---------------- ghosts ----------------
 
+// a pass without branches over blocks of entries, looked at one by one only
+// where something is wrong
 static int check_map_entries(ss_ctx *ctx, const ss_replica &r, const int64_t *ids, const int32_t *slots,
                              int64_t n) {
-    for (int64_t i = 0; i < n; ++i) {
-        if (ids[i] == -1 || ids[i] == -2) SS_FAIL(ctx, SS_ERR_RANGE, "ids -1 and -2 are reserved");
-        if (slots && (slots[i] < 0 || slots[i] >= r.n_total))
-            SS_FAIL(ctx, SS_ERR_RANGE, "slot %d outside the replica", slots[i]);
+    for (int64_t b = 0; b < n; b += 4096) {
+        const int64_t e = std::min<int64_t>(n, b + 4096);
+        uint32_t bad = 0;
+        for (int64_t i = b; i < e; ++i) bad |= (uint32_t)((uint64_t)ids[i] >= (uint64_t)-2ll);
+        if (slots)
+            for (int64_t i = b; i < e; ++i) bad |= (uint32_t)((uint64_t)(int64_t)slots[i] >= (uint64_t)r.n_total);
+        for (int64_t i = b; bad && i < e; ++i) {
+            if (ids[i] == -1 || ids[i] == -2) SS_FAIL(ctx, SS_ERR_RANGE, "ids -1 and -2 are reserved");
+            if (slots && (slots[i] < 0 || slots[i] >= r.n_total))
+                SS_FAIL(ctx, SS_ERR_RANGE, "slot %d outside the replica", slots[i]);
+        }
     }
     return SS_OK;
 }
@@ -1001,7 +1028,7 @@ struct MapBatch {
     }
 };
 
-static int alloc_map(ss_ctx *ctx, ss_replica &r, int64_t cap) {
+static int alloc_map(ss_ctx *ctx, ss_replica &r, int64_t cap, bool clear = true) {
     if (cap != r.map_cap || !r.map_keys) {
         if (r.map_keys) {
             const size_t b = (sizeof(unsigned long long) + sizeof(int32_t)) * (size_t)r.map_cap;
@@ -1014,7 +1041,7 @@ static int alloc_map(ss_ctx *ctx, ss_replica &r, int64_t cap) {
         SS_HIP(ctx, dalloc(ctx, &r, &r.map_vals, (size_t)cap));
         r.map_cap = cap;
     }
-    SS_HIP(ctx, ss_launch_map_clear(r.map_keys, r.map_vals, cap, ctx->stream));
+    if (clear) SS_HIP(ctx, ss_launch_map_clear(r.map_keys, r.map_vals, cap, ctx->stream));
     r.map_size = 0;
     return SS_OK;
 }
@@ -1045,34 +1072,24 @@ int ss_map_build(ss_ctx *ctx, int32_t rep, const int64_t *ids, const int32_t *sl
     if (rc) return rc;
     const int64_t cap = std::max<int64_t>(64, (int64_t)std::ceil((double)n / lf));
     SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    if ((rc = alloc_map(ctx, r, cap))) return rc;
+    Scratch guard(ctx);
+    const size_t b_ids = up256(sizeof(int64_t) * (size_t)n), b_vals = up256(sizeof(int32_t) * (size_t)n);
+    void *w = nullptr;
+    SS_HIP(ctx, scratch(ctx, b_ids + b_vals + sizeof(unsigned long long) * (size_t)cap, &w));
+    int64_t *d_ids = (int64_t *)w;
+    int32_t *d_vals = (int32_t *)((char *)w + b_ids);
+    if ((rc = alloc_map(ctx, r, cap, n == 0))) return rc;
     if (n > 0) {
-        MapBatch b;
-        int64_t *probe = nullptr;
-        int32_t *claim = nullptr;
-        hipError_t e = b.stage(ids, slots, n);
-        if (e == hipSuccess) e = hipMalloc((void **)&probe, sizeof(int64_t) * (size_t)n);
-        if (e == hipSuccess) e = hipMalloc((void **)&claim, sizeof(int32_t) * (size_t)cap);
-        if (e == hipSuccess) e = ss_launch_map_build_init(b.ids, n, cap, probe, claim, ctx->stream);
-        // rounds in batches of four between reads of the count left unplaced;
-        // every round places at least one entry, so n + cap rounds bound it
-        const int R = 4;
-        int64_t rounds = 0;
-        int32_t left = 1;
-        while (e == hipSuccess && left > 0 && rounds <= n + cap) {
-            e = hipMemsetAsync(ctx->d_counters, 0, R * sizeof(int32_t), ctx->stream);
-            for (int j = 0; j < R && e == hipSuccess; ++j)
-                e = ss_launch_map_build_round(r.map_keys, r.map_vals, cap, b.ids, b.vals, n, probe, claim,
-                                              ctx->d_counters + j, ctx->stream);
-            if (e == hipSuccess) e = hipMemcpyAsync(&left, ctx->d_counters + R - 1, sizeof(int32_t),
-                                                    hipMemcpyDeviceToHost, ctx->stream);
-            if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-            rounds += R;
-        }
-        dfree(probe);
-        dfree(claim);
+        hipError_t e = hipMemcpyAsync(d_ids, ids, sizeof(int64_t) * (size_t)n, hipMemcpyHostToDevice, ctx->stream);
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(d_vals, slots, sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice, ctx->stream);
+        if (e == hipSuccess)
+            e = ss_launch_map_build(r.map_keys, r.map_vals, cap, d_ids, d_vals, n,
+                                    (unsigned long long *)((char *)w + b_ids + b_vals), ctx->num_cus, ctx->stream);
+        if (e != hipSuccess) (void)ss_launch_map_clear(r.map_keys, r.map_vals, cap, ctx->stream);   // an empty table
+        const hipError_t e2 = hipStreamSynchronize(ctx->stream);
         SS_HIP(ctx, e);
-        if (left > 0) SS_FAIL(ctx, SS_ERR_FULL, "map build left %d entries unplaced", left);
+        SS_HIP(ctx, e2);
     }
     r.map_size = n;    // gpu_kernels.py:137 counts every entry, repeated ids included
     return SS_OK;
@@ -1154,18 +1171,17 @@ int ss_map_download(ss_ctx *ctx, int32_t rep, int64_t *keys, int32_t *vals, int6
     return SS_OK;
 }
 
-static int lookup_dev(ss_ctx *ctx, ss_replica &r, const int64_t *ids, int32_t *d_out, int64_t n, int64_t *n_missing) {
-    int64_t *d_ids = nullptr;
-    SS_HIP(ctx, hipMalloc((void **)&d_ids, sizeof(int64_t) * n));
-    int32_t zero = 0, miss = 0;
-    hipError_t e = hipMemcpy(d_ids, ids, sizeof(int64_t) * n, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(ctx->d_counters, &zero, sizeof(int32_t), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = ss_launch_map_lookup(r.map_keys, r.map_vals, r.map_cap, d_ids, d_out, n, ctx->d_counters, ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    if (e == hipSuccess) e = hipMemcpy(&miss, ctx->d_counters, sizeof(int32_t), hipMemcpyDeviceToHost);
-    dfree(d_ids);
-    SS_HIP(ctx, e);
-    if (n_missing) *n_missing = miss;
+// Lookups of n ids into d_out (device), with d_ids as their device copy;
+// counts: the misses and, with `lowest`, the smallest slot found.
+static int lookup_dev(ss_ctx *ctx, ss_replica &r, const int64_t *ids, int64_t *d_ids, int32_t *d_out, int64_t n,
+                      bool lowest, uint32_t counts[2]) {
+    uint32_t *d = (uint32_t *)ctx->d_counters;
+    SS_HIP(ctx, hipMemsetAsync(d, 0, sizeof(uint32_t), ctx->stream));
+    SS_HIP(ctx, hipMemsetAsync(d + 1, 0xFF, sizeof(uint32_t), ctx->stream));
+    SS_HIP(ctx, hipMemcpyAsync(d_ids, ids, sizeof(int64_t) * (size_t)n, hipMemcpyHostToDevice, ctx->stream));
+    SS_HIP(ctx, ss_launch_map_lookup(r.map_keys, r.map_vals, r.map_cap, d_ids, d_out, n, d, lowest, ctx->num_cus,
+                                     ctx->stream));
+    SS_HIP(ctx, hipMemcpyAsync(counts, d, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
     return SS_OK;
 }
 
@@ -1174,15 +1190,18 @@ int ss_map_lookup(ss_ctx *ctx, int32_t rep, const int64_t *ids, int32_t *out, in
     ss_replica &r = ctx->reps[rep];
     if (!r.map_keys) SS_FAIL(ctx, SS_ERR_STATE, "map not built");
     if (n == 0) { if (n_missing) *n_missing = 0; return SS_OK; }
-    int32_t *d_out = nullptr;
-    SS_HIP(ctx, hipMalloc((void **)&d_out, sizeof(int32_t) * n));
-    int rc = lookup_dev(ctx, r, ids, d_out, n, n_missing);
-    if (rc == SS_OK) {
-        hipError_t e = hipMemcpy(out, d_out, sizeof(int32_t) * n, hipMemcpyDeviceToHost);
-        if (e != hipSuccess) { dfree(d_out); SS_HIP(ctx, e); }
-    }
-    dfree(d_out);
-    return rc;
+    Scratch guard(ctx);
+    void *w = nullptr;
+    const size_t b_ids = up256(sizeof(int64_t) * (size_t)n);
+    SS_HIP(ctx, scratch(ctx, b_ids + sizeof(int32_t) * (size_t)n, &w));
+    int32_t *d_out = (int32_t *)((char *)w + b_ids);
+    uint32_t counts[2] = {0, 0};
+    int rc = lookup_dev(ctx, r, ids, (int64_t *)w, d_out, n, false, counts);
+    if (rc) return rc;
+    SS_HIP(ctx, hipMemcpyAsync(out, d_out, sizeof(int32_t) * (size_t)n, hipMemcpyDeviceToHost, ctx->stream));
+    SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (n_missing) *n_missing = counts[0];
+    return SS_OK;
 }
 
 int ss_halo_bind(ss_ctx *ctx, int32_t rep, const int64_t *ids, int64_t n, int64_t *n_missing) {
@@ -1190,34 +1209,58 @@ int ss_halo_bind(ss_ctx *ctx, int32_t rep, const int64_t *ids, int64_t n, int64_
     ss_replica &r = ctx->reps[rep];
     if (!r.map_keys) SS_FAIL(ctx, SS_ERR_STATE, "map not built");
     SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    dfree(r.halo_slots); dfree(r.halo_rec);
-    for (auto &d : r.halo_dev) { dfree(d); d = nullptr; }
-    for (auto &d : r.halo_grp) { dfree(d); d = nullptr; }
+    SS_HIP(ctx, hipStreamSynchronize(ctx->copy_stream));
+    // what the binding before held; its buffers of a tick's values are kept
+    // for one of as many records
+    const bool same = n == r.n_halo;
+    auto drop = [&](void *p, size_t b) {
+        if (!p) return;
+        dfree(p);
+        r.bytes -= b;
+        ctx->bytes -= b;
+    };
+    drop(r.halo_rec, sizeof(int32_t) * (size_t)r.halo_rec_n);
+    r.halo_rec = nullptr;
+    r.halo_rec_n = 0;
+    if (!same) for (auto &d : r.halo_dev) { drop(d, (size_t)std::max<int64_t>(r.n_halo, 1)); d = nullptr; }
+    for (auto &d : r.halo_grp) { drop(d, (size_t)r.halo_grp_bytes); d = nullptr; }
     r.halo_grp_bytes = 0;
-    r.halo_slots = nullptr; r.halo_rec = nullptr;
     r.n_halo = 0;
     if (n == 0) return SS_OK;
-    SS_HIP(ctx, dalloc(ctx, &r, &r.halo_slots, (size_t)n));
-    for (auto &d : r.halo_dev) SS_HIP(ctx, dalloc(ctx, &r, &d, (size_t)n));
-    int64_t miss = 0;
-    int rc = lookup_dev(ctx, r, ids, r.halo_slots, n, &miss);
-    if (rc) return rc;
+    auto unbound = [&](int rc) {                        // a binding that failed leaves no buffers behind
+        (void)hipStreamSynchronize(ctx->stream);
+        for (auto &d : r.halo_dev) { drop(d, (size_t)n); d = nullptr; }
+        return rc;
+    };
+    for (auto &d : r.halo_dev)
+        if (!d) {
+            hipError_t e = dalloc(ctx, &r, &d, (size_t)n);
+            if (e != hipSuccess) { d = nullptr; unbound(0); SS_HIP(ctx, e); }
+        }
+    Scratch guard(ctx);
+    void *w = nullptr;
+    const size_t b_ids = up256(sizeof(int64_t) * (size_t)n);
+    hipError_t e = scratch(ctx, b_ids + sizeof(int32_t) * (size_t)n, &w);
+    if (e != hipSuccess) { unbound(0); SS_HIP(ctx, e); }
+    int32_t *d_slots = (int32_t *)((char *)w + b_ids);
+    uint32_t counts[2] = {0, 0};
+    int rc = lookup_dev(ctx, r, ids, (int64_t *)w, d_slots, n, true, counts);
+    if (rc) return unbound(rc);
+    e = hipStreamSynchronize(ctx->stream);
     // the refresh runs in slot order: record of every slot from the first
-    // bound one (or the first ghost) on; a slot bound twice takes the later record
-    std::vector<int32_t> slots((size_t)n);
-    SS_HIP(ctx, hipMemcpy(slots.data(), r.halo_slots, sizeof(int32_t) * (size_t)n, hipMemcpyDeviceToHost));
-    int64_t lo = r.n_local;
-    for (int32_t s : slots)
-        if (s >= 0) lo = std::min<int64_t>(lo, s);
-    r.halo_base = lo / 64 * 64;
-    // padded to whole groups of sixteen slots (the refresh reads four records
-    // at once, a lane of the tick kernel's fused refresh sixteen)
-    std::vector<int32_t> rec((size_t)((r.n_total - r.halo_base + 15) / 16 * 16), -1);
-    for (int64_t h = 0; h < n; ++h)
-        if (slots[(size_t)h] >= 0) rec[(size_t)(slots[(size_t)h] - r.halo_base)] = (int32_t)h;
-    SS_HIP(ctx, dalloc(ctx, &r, &r.halo_rec, rec.size()));
-    SS_HIP(ctx, hipMemcpy(r.halo_rec, rec.data(), sizeof(int32_t) * rec.size(), hipMemcpyHostToDevice));
-    if (n_missing) *n_missing = miss;
+    // bound one (or the first ghost) on; a slot bound twice takes the later
+    // record.  Padded to whole groups of sixteen slots (the refresh reads four
+    // records at once, a lane of the tick kernel's fused refresh sixteen).
+    r.halo_base = std::min<int64_t>(r.n_local, (int64_t)counts[1]) / 64 * 64;
+    const int64_t n_rec = (r.n_total - r.halo_base + 15) / 16 * 16;
+    if (e == hipSuccess) e = dalloc(ctx, &r, &r.halo_rec, (size_t)n_rec);
+    if (e == hipSuccess) {
+        r.halo_rec_n = std::max<int64_t>(n_rec, 1);
+        e = ss_launch_halo_records(d_slots, n, r.halo_base, r.halo_rec, n_rec, ctx->stream);
+    }
+    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+    if (e != hipSuccess) { unbound(0); SS_HIP(ctx, e); }
+    if (n_missing) *n_missing = counts[0];
     r.n_halo = n;
     return SS_OK;
 }
@@ -1256,21 +1299,19 @@ int ss_halo_unpack_ids(ss_ctx *ctx, int32_t rep, const int64_t *ids, const int8_
     if (!r.map_keys) SS_FAIL(ctx, SS_ERR_STATE, "map not built");
     if (n == 0) { if (n_missing) *n_missing = 0; return SS_OK; }
     SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    int64_t *d_ids = nullptr;
-    int8_t *d_vals = nullptr;
-    SS_HIP(ctx, hipMalloc((void **)&d_ids, sizeof(int64_t) * n));
-    hipError_t e = hipMalloc((void **)&d_vals, (size_t)n);
-    if (e != hipSuccess) { dfree(d_ids); SS_HIP(ctx, e); }
-    int32_t zero = 0, miss = 0;
-    e = hipMemcpy(d_ids, ids, sizeof(int64_t) * n, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(d_vals, vals, (size_t)n, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(ctx->d_counters, &zero, sizeof(int32_t), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = ss_launch_halo_unpack_ids(r.map_keys, r.map_vals, r.map_cap, d_ids, d_vals, n, r.state[0], r.state[1], ctx->d_counters, ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    if (e == hipSuccess) e = hipMemcpy(&miss, ctx->d_counters, sizeof(int32_t), hipMemcpyDeviceToHost);
-    dfree(d_ids);
-    dfree(d_vals);
-    SS_HIP(ctx, e);
+    Scratch guard(ctx);
+    void *w = nullptr;
+    const size_t b_ids = up256(sizeof(int64_t) * (size_t)n);
+    SS_HIP(ctx, scratch(ctx, b_ids + (size_t)n, &w));
+    int8_t *d_vals = (int8_t *)w + b_ids;
+    int32_t miss = 0;
+    SS_HIP(ctx, hipMemsetAsync(ctx->d_counters, 0, sizeof(int32_t), ctx->stream));
+    SS_HIP(ctx, hipMemcpyAsync(w, ids, sizeof(int64_t) * (size_t)n, hipMemcpyHostToDevice, ctx->stream));
+    SS_HIP(ctx, hipMemcpyAsync(d_vals, vals, (size_t)n, hipMemcpyHostToDevice, ctx->stream));
+    SS_HIP(ctx, ss_launch_halo_unpack_ids(r.map_keys, r.map_vals, r.map_cap, (const int64_t *)w, d_vals, n, r.state[0],
+                                          r.state[1], ctx->d_counters, ctx->stream));
+    SS_HIP(ctx, hipMemcpyAsync(&miss, ctx->d_counters, sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
+    SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
     if (n_missing) *n_missing = miss;
     return refresh_ghost_bits(ctx, r);
 }
@@ -1278,25 +1319,24 @@ int ss_halo_unpack_ids(ss_ctx *ctx, int32_t rep, const int64_t *ids, const int8_
 static int halo_pack(ss_ctx *ctx, int32_t rep, const int32_t *slots, int64_t n, void *out, bool packed) {
     if (!valid_rep(ctx, rep) || (n && (!slots || !out))) SS_FAIL(ctx, SS_ERR_INVALID, "bad replica or NULL");
     ss_replica &r = ctx->reps[rep];
-    for (int64_t i = 0; i < n; ++i)
-        if (slots[i] < 0 || slots[i] >= r.n_total) SS_FAIL(ctx, SS_ERR_RANGE, "slot %d outside the replica", slots[i]);
+    for (int64_t b = 0; b < n; b += 4096) {             // without branches, one by one only where one is wrong
+        const int64_t e = std::min<int64_t>(n, b + 4096);
+        uint32_t bad = 0;
+        for (int64_t i = b; i < e; ++i) bad |= (uint32_t)((uint64_t)(int64_t)slots[i] >= (uint64_t)r.n_total);
+        for (int64_t i = b; bad && i < e; ++i)
+            if (slots[i] < 0 || slots[i] >= r.n_total) SS_FAIL(ctx, SS_ERR_RANGE, "slot %d outside the replica", slots[i]);
+    }
     if (n == 0) return SS_OK;
-    const size_t nb = (size_t)(packed ? (n + 3) / 4 : n);
+    const size_t nb = (size_t)(packed ? (n + 3) / 4 : n), b_slots = up256(sizeof(int32_t) * (size_t)n);
+    Scratch guard(ctx);
+    void *w = nullptr;
+    SS_HIP(ctx, scratch(ctx, b_slots + nb, &w));
+    int8_t *d_out = (int8_t *)w + b_slots;
+    SS_HIP(ctx, hipMemcpyAsync(w, slots, sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice, ctx->stream));
+    SS_HIP(ctx, packed ? ss_launch_gather2(r.state[r.tick & 1], (const int32_t *)w, (uint8_t *)d_out, n, ctx->stream)
+                       : ss_launch_gather(r.state[r.tick & 1], (const int32_t *)w, d_out, n, ctx->stream));
+    SS_HIP(ctx, hipMemcpyAsync(out, d_out, nb, hipMemcpyDeviceToHost, ctx->stream));
     SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    int32_t *d_slots = nullptr;
-    int8_t *d_out = nullptr;
-    SS_HIP(ctx, hipMalloc((void **)&d_slots, sizeof(int32_t) * n));
-    hipError_t e = hipMalloc((void **)&d_out, nb);
-    if (e != hipSuccess) { dfree(d_slots); SS_HIP(ctx, e); }
-    e = hipMemcpy(d_slots, slots, sizeof(int32_t) * n, hipMemcpyHostToDevice);
-    if (e == hipSuccess)
-        e = packed ? ss_launch_gather2(r.state[r.tick & 1], d_slots, (uint8_t *)d_out, n, ctx->stream)
-                   : ss_launch_gather(r.state[r.tick & 1], d_slots, d_out, n, ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    if (e == hipSuccess) e = hipMemcpy(out, d_out, nb, hipMemcpyDeviceToHost);
-    dfree(d_slots);
-    dfree(d_out);
-    SS_HIP(ctx, e);
     return SS_OK;
 }
 

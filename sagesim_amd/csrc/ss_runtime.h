@@ -37,7 +37,10 @@ hipError_t ss_occupancy_tick(int apl, int *blocks_per_cu);
 hipError_t ss_launch_bits(const int8_t *st, uint64_t *bits, int64_t w0, int64_t w1, int64_t n_total, int8_t inf,
                           hipStream_t s);
 hipError_t ss_launch_map_lookup(const unsigned long long *keys, const int32_t *vals, int64_t cap, const int64_t *ids,
-                                int32_t *out, int64_t n, int32_t *misses, hipStream_t s);
+                                int32_t *out, int64_t n, uint32_t *counts, bool lowest, int num_cus, hipStream_t s);
+// rec[slot[h] - base] = the last record h of every slot, -1 elsewhere
+hipError_t ss_launch_halo_records(const int32_t *slot, int64_t n, int64_t base, int32_t *rec, int64_t n_rec,
+                                  hipStream_t s);
 // ghost refresh from a bound halo: slot base + g <- vals[rec[g]] (rec -1: kept),
 // both buffers, and the bitmap words of [base, n_total) of the buffer `cur`;
 // packed: vals holds 2-bit codes, four records a byte
@@ -110,10 +113,10 @@ struct ss_replica {
     unsigned long long *map_keys = nullptr;
     int32_t *map_vals = nullptr;
     int64_t map_cap = 0, map_size = 0;
-    // bound halo: slot of every record of the per-tick halo buffer
-    int32_t *halo_slots = nullptr;
+    // bound halo: records of the per-tick halo buffer
     int64_t n_halo = 0;
     int32_t *halo_rec = nullptr;                // record of slot halo_base + g, -1 when not bound
+    int64_t halo_rec_n = 0;                     // entries allocated
     int64_t halo_base = 0;                      // first slot refreshed (a multiple of 64)
     int8_t *halo_dev[SS_HALO_RING] = {};       // device staging of halo values, a ring by tick
     int8_t *halo_grp[2] = {};                   // device staging of a group of ticks (page-locked input)

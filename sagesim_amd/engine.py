@@ -316,15 +316,17 @@ class Engine:
         this rank needs from r (ss_ghost_discover)."""
         nbr = np.ascontiguousarray(nbr_ids, np.int64)
         own = np.ascontiguousarray(owner, np.int32)
+        # one call into buffers that hold whatever it finds (their pages are
+        # touched only as far as they are filled), then cut to size
+        cap = max(1, min(nbr.shape[0], own.shape[0]))
         n = ctypes.c_int64()
-        self._ck(self._L.ss_ghost_discover(self._h, ptr(nbr), nbr.shape[0], ptr(own), own.shape[0], int(my_rank),
-                                           int(n_ranks), None, None, None, 0, ctypes.byref(n)))
-        ids = np.empty(n.value, np.int64)
+        ids = np.empty(cap, np.int64)
         offsets = np.empty(int(n_ranks) + 1, np.int32)
-        index = np.empty(n.value, np.int32)
+        index = np.empty(cap, np.int32)
         self._ck(self._L.ss_ghost_discover(self._h, ptr(nbr), nbr.shape[0], ptr(own), own.shape[0], int(my_rank),
-                                           int(n_ranks), ptr(ids), ptr(offsets), ptr(index), ids.shape[0],
-                                           ctypes.byref(n)))
+                                           int(n_ranks), ptr(ids), ptr(offsets), ptr(index), cap, ctypes.byref(n)))
+        ids.resize(n.value, refcheck=False)
+        index.resize(n.value, refcheck=False)
         return ids, offsets, index
 
     def halo_bind(self, rep, ids):

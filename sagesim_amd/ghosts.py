@@ -18,11 +18,10 @@ from .engine import Engine
 
 
 def _flat_ids(all_neighbors):
-    """Neighbour ids as int64, padding dropped (NaN and negative entries,
-    gpu_kernels.py:50-65)."""
+    """Neighbour ids as int64, padding (NaN and negative entries,
+    gpu_kernels.py:50-65) dropped or negative."""
     if isinstance(all_neighbors, np.ndarray) and all_neighbors.ndim == 1 and all_neighbors.dtype.kind in "iu":
-        flat = all_neighbors.astype(np.int64, copy=False)
-        return flat[flat >= 0]
+        return all_neighbors.astype(np.int64, copy=False)      # negative entries are skipped on the device
     if len(all_neighbors) == 0:
         return np.zeros(0, np.int64)
     if isinstance(all_neighbors[0], np.ndarray):

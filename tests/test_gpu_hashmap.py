@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from oracle.hashmap import RefHashMap, home_slot
-from sagesim_amd import Engine, graphs
+from sagesim_amd import Engine, Replica, graphs
 from sagesim_amd._lib import NativeError
 from sagesim_amd.engine import sir_model
 
@@ -139,3 +139,62 @@ def test_full_map_reports_no_slot(eng):
     got, miss = eng.map_lookup(rep, np.concatenate([ids, [5]]).astype(np.int64))
     assert miss == 0 and got[-1] == 0 and got[:5].tolist() == list(range(5))
     eng.remove_replica(rep)
+
+
+@pytest.mark.parametrize("n,load", [(1, 0.5), (2, 0.9), (57, 0.9), (58, 0.9), (64, 0.5), (900, 0.9), (4097, 0.9), (30_000, 0.9)])
+@pytest.mark.parametrize("kind", ["distinct", "repeats", "one home"])
+def test_build_places_as_the_rounds_do(n, load, kind):
+    """One launch of displacing proposals leaves the table the placement rounds
+    leave: near-full tables, ids repeated many times, and ids that all start at
+    one slot (chains as long as the table's entries)."""
+    print("[case] build", n, load, kind, flush=True)
+    rng = np.random.default_rng(n)
+    cap = max(64, int(np.ceil(n / load)))
+    if kind == "distinct":
+        ids = rng.choice(1 << 40, n, replace=False).astype(np.int64) - (1 << 39)
+        ids[(ids == -1) | (ids == -2)] = 5
+    elif kind == "repeats":
+        ids = rng.integers(0, max(1, n // 7), n).astype(np.int64)
+    else:
+        n = min(n, 900)
+        cap = max(64, int(np.ceil(n / load)))
+        ids = (np.arange(n, dtype=np.int64) * cap)[rng.permutation(n)]      # home = (id * odd) mod cap: all 0
+    g = graphs.from_edges(max(n, 2), np.arange(1), np.arange(1, 2))
+    slots = rng.permutation(max(n, 2))[:n].astype(np.int32)
+    ref = RefHashMap(cap)
+    ref.build_from_arrays(ids, slots)
+    with Engine(0) as e:
+        r = Replica(e, g, np.zeros(max(n, 2), np.int8), sir_model(0.1, 0.1), 1)
+        e.map_build(r.rep, ids, slots, load)
+        keys, vals = e.map_arrays(r.rep)
+        assert keys.shape[0] == cap
+        assert np.array_equal(keys, ref.keys) and np.array_equal(vals, ref.values)
+        out, miss = e.map_lookup(r.rep, np.concatenate([ids, [1 << 50, (1 << 50) + 1]]))
+        assert miss == 2 and out[-1] == out[-2] == -1
+        assert out[:n].tolist() == [ref.lookup_cpu(int(i)) for i in ids]
+
+
+def test_halo_bound_twice_and_low_slots():
+    """Records whose slots repeat (the later record counts) or lie among the
+    local agents, ids the map lacks, and a second binding of another order."""
+    print("[case] halo binding", flush=True)
+    rng = np.random.default_rng(8)
+    n, ghosts = 300, 333
+    rp = np.zeros(n + 1, np.int64)
+    g = graphs.CSRGraph(rp, np.zeros(0, np.int32), n_cols=n + ghosts)
+    ids = np.arange(1000, 1000 + n + ghosts, dtype=np.int64)
+    with Engine(0) as e:
+        r = Replica(e, g, np.zeros(n + ghosts, np.int8), sir_model(0.0, 0.0), 1, sort=False)
+        e.map_build(r.rep, ids, np.arange(n + ghosts, dtype=np.int32), 0.5)
+        for low in (n, 130):
+            for extra in (0, 7):
+                rec = np.concatenate([rng.permutation(ids[low:]), ids[low:low + 40], np.full(extra, 5)])
+                assert e.halo_bind(r.rep, rec) == extra
+                before = e.state(r.rep, n + ghosts)
+                vals = rng.integers(0, 3, rec.size).astype(np.int8)
+                e.halo_unpack(r.rep, vals)
+                want = before.copy()
+                for i, v in zip(rec, vals):
+                    if i >= 1000:
+                        want[i - 1000] = v
+                assert np.array_equal(e.state(r.rep, n + ghosts), want)
