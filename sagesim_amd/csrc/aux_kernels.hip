@@ -216,9 +216,14 @@ __global__ void gather2_kernel(const int8_t *__restrict__ st, const int32_t *__r
     const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (4 * j >= n) return;
     uint32_t b = 0u;
+    if (4 * j + 4 <= n) {                               // one load of the four slots
+        struct __attribute__((packed, aligned(4))) Four { int32_t s[4]; };
+        const Four f = *(const Four *)(slots + 4 * j);
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-        if (4 * j + q < n) b |= ((uint32_t)(uint8_t)st[slots[4 * j + q]] & 3u) << (2 * q);
+        for (int q = 0; q < 4; ++q) b |= ((uint32_t)(uint8_t)st[f.s[q]] & 3u) << (2 * q);
+    } else {
+        for (int q = 0; 4 * j + q < n; ++q) b |= ((uint32_t)(uint8_t)st[slots[4 * j + q]] & 3u) << (2 * q);
+    }
     out[j] = (uint8_t)b;
 }
 
@@ -308,6 +313,20 @@ __global__ __launch_bounds__(256) void order_kernel(const int8_t *__restrict__ s
         for (int h = 0; h < 4; ++h) w[q] |= (uint32_t)(uint8_t)st[x[h]] << (8 * h);
     }
     *(uint4 *)(out + j0) = make_uint4(w[0], w[1], w[2], w[3]);     // out is padded to whole groups of 16
+}
+
+// Page-locked host memory -> device by the compute units, for what the next
+// kernel waits for: bytes of src (W per lane) and a table of words2 8-byte
+// words.  Bound by the trip over the bus: 3.3 us for both, where the copy
+// engine's hand-over to the compute stream and back costs some 25 us beside
+// the 3 us of the copy, and the table took a copy of its own.
+template <class W>
+__global__ __launch_bounds__(256) void stage_kernel(const W *__restrict__ src, W *__restrict__ dst, int64_t n,
+                                                    const uint64_t *__restrict__ src2, uint64_t *__restrict__ dst2,
+                                                    int64_t words2) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) dst[i] = src[i];
+    if (i < words2) dst2[i] = src2[i];
 }
 
 // Plain streaming copy (16 B per lane per step): the known-size reference for
@@ -440,6 +459,26 @@ hipError_t ss_launch_order(const int8_t *st, const int32_t *slot, int8_t *out, i
     if (n_total <= 0) return hipSuccess;
     hipLaunchKernelGGL(order_kernel, dim3(grid_for(n_total, 16 * 256)), dim3(256), 0, s, st, slot, out, n_local,
                        n_total);
+    return hipGetLastError();
+}
+
+hipError_t ss_launch_stage(const void *src, void *dst, int64_t bytes, const uint64_t *src2, uint64_t *dst2,
+                           int64_t words2, hipStream_t s) {
+    // as wide as the start and the length allow (dst is an allocation's start)
+    const uintptr_t at = (uintptr_t)src | (uintptr_t)bytes;
+    const int64_t n = at % 16 == 0 ? bytes / 16 : at % 4 == 0 ? bytes / 4 : bytes;
+    const int64_t lanes = std::max(n, words2);
+    if (lanes <= 0) return hipSuccess;
+    const dim3 grid(grid_for(lanes, 256));
+    if (at % 16 == 0)
+        hipLaunchKernelGGL(stage_kernel<uint4>, grid, dim3(256), 0, s, (const uint4 *)src, (uint4 *)dst, n, src2, dst2,
+                           words2);
+    else if (at % 4 == 0)
+        hipLaunchKernelGGL(stage_kernel<uint32_t>, grid, dim3(256), 0, s, (const uint32_t *)src, (uint32_t *)dst, n,
+                           src2, dst2, words2);
+    else
+        hipLaunchKernelGGL(stage_kernel<uint8_t>, grid, dim3(256), 0, s, (const uint8_t *)src, (uint8_t *)dst, n, src2,
+                           dst2, words2);
     return hipGetLastError();
 }
 

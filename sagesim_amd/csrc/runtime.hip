@@ -375,8 +375,9 @@ int ensure_rep_table(ss_ctx *ctx) {
     return SS_OK;
 }
 
-// copy descriptors with tick window [tick, tick + ticks) clipped to each limit
-int push_descriptors(ss_ctx *ctx, int64_t ticks) {
+// the host's descriptors with tick window [tick, tick + ticks) clipped to each
+// limit; the compute stream is idle after it
+int fill_descriptors(ss_ctx *ctx, int64_t ticks) {
     int rc = ensure_rep_table(ctx);
     if (rc) return rc;
     SS_HIP(ctx, hipStreamSynchronize(ctx->stream));  // the mirror may still be in flight
@@ -394,6 +395,13 @@ int push_descriptors(ss_ctx *ctx, int64_t ticks) {
         }
         ctx->h_reps[i] = d;
     }
+    return SS_OK;
+}
+
+// the same, and their copy to the device
+int push_descriptors(ss_ctx *ctx, int64_t ticks) {
+    int rc = fill_descriptors(ctx, ticks);
+    if (rc) return rc;
     SS_HIP(ctx, hipMemcpyAsync(ctx->d_reps, ctx->h_reps, sizeof(ss_rep_dev) * ctx->reps.size(),
                                hipMemcpyHostToDevice, ctx->stream));
     return SS_OK;
@@ -512,6 +520,7 @@ int ss_destroy(ss_ctx *ctx) {
     if (ctx->t_stop) (void)hipEventDestroy(ctx->t_stop);
     if (ctx->h_reps) (void)hipHostFree(ctx->h_reps);
     if (ctx->h_stats) (void)hipHostFree(ctx->h_stats);
+    if (ctx->h_stage) (void)hipHostFree(ctx->h_stage);
     for (int i = 0; i < SS_HALO_RING; ++i) {
         if (ctx->h_halo_pin[i]) (void)hipHostFree(ctx->h_halo_pin[i]);
         if (ctx->halo_ev[i]) (void)hipEventDestroy(ctx->halo_ev[i]);
@@ -1328,6 +1337,19 @@ static int halo_pack(ss_ctx *ctx, int32_t rep, const int32_t *slots, int64_t n, 
     }
     if (n == 0) return SS_OK;
     const size_t nb = (size_t)(packed ? (n + 3) / 4 : n), b_slots = up256(sizeof(int32_t) * (size_t)n);
+    if (b_slots + nb <= (size_t)SS_STAGE_BYTES) {
+        // the kernel reads the slots from page-locked memory and writes the
+        // result there: no copy engine in the chain behind the tick
+        if (!ctx->h_stage) SS_HIP(ctx, hipHostMalloc(&ctx->h_stage, (size_t)SS_STAGE_BYTES, hipHostMallocDefault));
+        int8_t *h_out = (int8_t *)ctx->h_stage + b_slots;
+        std::memcpy(ctx->h_stage, slots, sizeof(int32_t) * (size_t)n);
+        const int32_t *h_slots = (const int32_t *)ctx->h_stage;
+        SS_HIP(ctx, packed ? ss_launch_gather2(r.state[r.tick & 1], h_slots, (uint8_t *)h_out, n, ctx->stream)
+                           : ss_launch_gather(r.state[r.tick & 1], h_slots, h_out, n, ctx->stream));
+        SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        std::memcpy(out, h_out, nb);
+        return SS_OK;
+    }
     Scratch guard(ctx);
     void *w = nullptr;
     SS_HIP(ctx, scratch(ctx, b_slots + nb, &w));
@@ -1493,6 +1515,26 @@ static int simulate_halo_groups(ss_ctx *ctx, ss_replica &r, int64_t ticks, const
     return SS_OK;
 }
 
+// One tick from page-locked memory (a live exchange): there is nothing to
+// overlap the halo's transfer with, so a kernel of the compute stream copies it
+// (and the descriptors), and no other queue is waited for.  The call returns
+// when the caller's buffer has been read.
+static int simulate_halo_one(ss_ctx *ctx, ss_replica &r, const int8_t *vals, int64_t n, bool packed) {
+    static_assert(sizeof(ss_rep_dev) % sizeof(uint64_t) == 0, "descriptors are copied in 8-byte words");
+    int rc = fill_descriptors(ctx, 1);
+    if (rc) return rc;
+    int8_t *staged = r.halo_dev[0];
+    SS_HIP(ctx, ss_launch_stage(vals, staged, n, (const uint64_t *)ctx->h_reps, (uint64_t *)ctx->d_reps,
+                                (int64_t)(sizeof(ss_rep_dev) / sizeof(uint64_t) * ctx->reps.size()), ctx->stream));
+    hipError_t e = hipEventRecord(ctx->halo_ev[0], ctx->stream);
+    if (e == hipSuccess) e = halo_tick(ctx, r, 0, staged, packed);
+    const hipError_t e2 = hipEventSynchronize(ctx->halo_ev[0]);
+    SS_HIP(ctx, e);
+    SS_HIP(ctx, e2);
+    advance_ticks(ctx, 1);
+    return SS_OK;
+}
+
 static int simulate_halo(ss_ctx *ctx, int32_t rep, int64_t ticks, const int8_t *vals, bool packed) {
     if (!valid_rep(ctx, rep) || (ticks > 0 && !vals)) SS_FAIL(ctx, SS_ERR_INVALID, "bad replica or NULL");
     if (ticks < 0 || ticks > INT32_MAX) SS_FAIL(ctx, SS_ERR_INVALID, "ticks out of range");
@@ -1504,12 +1546,15 @@ static int simulate_halo(ss_ctx *ctx, int32_t rep, int64_t ticks, const int8_t *
     if (ctx->tiles_dirty && (rc = build_tiles(ctx))) return rc;
     // values in page-locked memory are copied from where they are
     bool pinned = false;
+    const void *dev = nullptr;
     {
         hipPointerAttribute_t at;
         const hipError_t e = hipPointerGetAttributes(&at, vals);
         pinned = e == hipSuccess && at.type == hipMemoryTypeHost;
+        if (pinned) dev = at.devicePointer;
         if (e != hipSuccess) (void)hipGetLastError();   // pageable memory: not an error here
     }
+    if (dev && ticks == 1 && n <= SS_STAGE_BYTES) return simulate_halo_one(ctx, r, (const int8_t *)dev, n, packed);
     if (pinned) return simulate_halo_pinned(ctx, r, ticks, vals, n, packed);
     if ((rc = push_descriptors(ctx, ticks))) return rc;
     // pageable memory: staged tick by tick through a ring of page-locked buffers

@@ -17,6 +17,9 @@
 // page-locked halo input: ticks per group and device bytes per group buffer
 #define SS_HALO_GROUP 32
 #define SS_HALO_GROUP_BYTES (64ll << 20)
+// what the compute units copy from page-locked memory themselves (below this
+// the copy engine's signalling costs more than its bandwidth saves)
+#define SS_STAGE_BYTES (1ll << 20)
 #define SS_HALO_SPANS 8                         // copies per group: spans of 1, 1, 2, 4, ... ticks
 // work counters: S agents visited, draws, scans, CSR entries scanned,
 // counts pushed, replica-ticks taken in the push direction, agents of the
@@ -59,6 +62,10 @@ hipError_t ss_launch_fill_i32(int32_t *p, int64_t n, int32_t v, hipStream_t s);
 hipError_t ss_launch_order(const int8_t *st, const int32_t *slot, int8_t *out, int64_t n_local, int64_t n_total,
                            hipStream_t s);
 hipError_t ss_launch_copy(const void *src, void *dst, int64_t bytes, int grid, hipStream_t s);
+// bytes and a table of 8-byte words from page-locked host memory to device
+// memory, by one kernel
+hipError_t ss_launch_stage(const void *src, void *dst, int64_t bytes, const uint64_t *src2, uint64_t *dst2,
+                           int64_t words2, hipStream_t s);
 // n scattered 4-byte reads of src[0 .. n_words); out holds grid * 256 words
 hipError_t ss_launch_gather_probe(const uint32_t *src, int64_t n_words, int64_t n, uint32_t *out, int grid,
                                   hipStream_t s);
@@ -178,6 +185,7 @@ struct ss_ctx {
     hipEvent_t span_ev[2][SS_HALO_SPANS] = {};  // copy span s of group buffer b is on the device
     int64_t grp_pos = 0;                        // groups issued (buffer = grp_pos & 1)
     bool halo_fused = false;                    // this call's ticks fuse the next tick's halo refresh
+    void *h_stage = nullptr;                    // page-locked, SS_STAGE_BYTES: a small pack's slots and result
     void *scratch = nullptr;                    // workspace of one call at a time, on the context's stream
     size_t scratch_bytes = 0;
     std::string err;
