@@ -288,12 +288,14 @@ __global__ __launch_bounds__(256) void stats_kernel(const int8_t *__restrict__ s
 // as they are.  A thread makes 16 bytes of the result: four 16-byte loads of
 // slots (padded to whole groups of 16), 16 byte gathers, one 16-byte store.
 // Bound by the gathers (one cache line each, the states stay in the last-level
-// cache): 20 us for 10M agents, where scattering the downloaded states on the
-// host took 13 ms.
+// cache): 20 us for 10M agents into device memory, where scattering the
+// downloaded states on the host took 13 ms; a readback has it write the chunks
+// to page-locked memory, at the bus's rate.
 __global__ __launch_bounds__(256) void order_kernel(const int8_t *__restrict__ st, const int32_t *__restrict__ slot,
-                                                    int8_t *__restrict__ out, int64_t n_local, int64_t n_total) {
-    const int64_t j0 = 16 * ((int64_t)blockIdx.x * blockDim.x + threadIdx.x);
-    if (j0 >= n_total) return;
+                                                    int8_t *__restrict__ out, int64_t first, int64_t end,
+                                                    int64_t n_local) {
+    const int64_t j0 = first + 16 * ((int64_t)blockIdx.x * blockDim.x + threadIdx.x);
+    if (j0 >= end) return;
     uint32_t w[4] = {0u, 0u, 0u, 0u};
     const bool whole = j0 + 16 <= n_local;
 #pragma unroll
@@ -306,26 +308,29 @@ __global__ __launch_bounds__(256) void order_kernel(const int8_t *__restrict__ s
 #pragma unroll
             for (int h = 0; h < 4; ++h) {
                 const int64_t j = j0 + 4 * q + h;
-                x[h] = j < n_local ? slot[j] : j < n_total ? (int32_t)j : 0;
+                x[h] = j < n_local ? slot[j] : j < end ? (int32_t)j : 0;
             }
         }
 #pragma unroll
         for (int h = 0; h < 4; ++h) w[q] |= (uint32_t)(uint8_t)st[x[h]] << (8 * h);
     }
-    *(uint4 *)(out + j0) = make_uint4(w[0], w[1], w[2], w[3]);     // out is padded to whole groups of 16
+    *(uint4 *)(out + j0 - first) = make_uint4(w[0], w[1], w[2], w[3]);     // out is padded to whole groups of 16
 }
 
-// Page-locked host memory -> device by the compute units, for what the next
-// kernel waits for: bytes of src (W per lane) and a table of words2 8-byte
-// words.  Bound by the trip over the bus: 3.3 us for both, where the copy
-// engine's hand-over to the compute stream and back costs some 25 us beside
-// the 3 us of the copy, and the table took a copy of its own.
+// Page-locked host memory <-> device by the compute units, for what is waited
+// for: bytes of src (W per lane, one byte per lane of the rest) and a table of
+// words2 8-byte words.  Bound by the trip over the bus: 3.3 us for a halo and
+// the descriptors, where the copy engine's hand-over to the compute stream and
+// back costs some 25 us beside the 3 us of the copy, and the table took a copy
+// of its own.
 template <class W>
-__global__ __launch_bounds__(256) void stage_kernel(const W *__restrict__ src, W *__restrict__ dst, int64_t n,
+__global__ __launch_bounds__(256) void stage_kernel(const char *__restrict__ src, char *__restrict__ dst, int64_t bytes,
                                                     const uint64_t *__restrict__ src2, uint64_t *__restrict__ dst2,
                                                     int64_t words2) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) dst[i] = src[i];
+    const int64_t n = bytes / (int64_t)sizeof(W), rest = n * (int64_t)sizeof(W) + (i - n);
+    if (i < n) ((W *)dst)[i] = ((const W *)src)[i];
+    else if (rest < bytes) dst[rest] = src[rest];
     if (i < words2) dst2[i] = src2[i];
 }
 
@@ -454,31 +459,24 @@ hipError_t ss_launch_stats(const int8_t *st, const uint8_t *deg8, const int64_t 
     return hipGetLastError();
 }
 
-hipError_t ss_launch_order(const int8_t *st, const int32_t *slot, int8_t *out, int64_t n_local, int64_t n_total,
-                           hipStream_t s) {
-    if (n_total <= 0) return hipSuccess;
-    hipLaunchKernelGGL(order_kernel, dim3(grid_for(n_total, 16 * 256)), dim3(256), 0, s, st, slot, out, n_local,
-                       n_total);
+hipError_t ss_launch_order(const int8_t *st, const int32_t *slot, int8_t *out, int64_t first, int64_t end,
+                           int64_t n_local, hipStream_t s) {
+    if (end <= first) return hipSuccess;
+    hipLaunchKernelGGL(order_kernel, dim3(grid_for(end - first, 16 * 256)), dim3(256), 0, s, st, slot, out, first, end,
+                       n_local);
     return hipGetLastError();
 }
 
 hipError_t ss_launch_stage(const void *src, void *dst, int64_t bytes, const uint64_t *src2, uint64_t *dst2,
                            int64_t words2, hipStream_t s) {
-    // as wide as the start and the length allow (dst is an allocation's start)
-    const uintptr_t at = (uintptr_t)src | (uintptr_t)bytes;
-    const int64_t n = at % 16 == 0 ? bytes / 16 : at % 4 == 0 ? bytes / 4 : bytes;
-    const int64_t lanes = std::max(n, words2);
+    // as wide as the pointers allow
+    const uintptr_t at = (uintptr_t)src | (uintptr_t)dst;
+    const int64_t w = at % 16 == 0 ? 16 : at % 4 == 0 ? 4 : 1;
+    const int64_t lanes = std::max(bytes / w + bytes % w, words2);
     if (lanes <= 0) return hipSuccess;
-    const dim3 grid(grid_for(lanes, 256));
-    if (at % 16 == 0)
-        hipLaunchKernelGGL(stage_kernel<uint4>, grid, dim3(256), 0, s, (const uint4 *)src, (uint4 *)dst, n, src2, dst2,
-                           words2);
-    else if (at % 4 == 0)
-        hipLaunchKernelGGL(stage_kernel<uint32_t>, grid, dim3(256), 0, s, (const uint32_t *)src, (uint32_t *)dst, n,
-                           src2, dst2, words2);
-    else
-        hipLaunchKernelGGL(stage_kernel<uint8_t>, grid, dim3(256), 0, s, (const uint8_t *)src, (uint8_t *)dst, n, src2,
-                           dst2, words2);
+    auto kernel = w == 16 ? stage_kernel<uint4> : w == 4 ? stage_kernel<uint32_t> : stage_kernel<uint8_t>;
+    hipLaunchKernelGGL(kernel, dim3(grid_for(lanes, 256)), dim3(256), 0, s, (const char *)src, (char *)dst, bytes, src2,
+                       dst2, words2);
     return hipGetLastError();
 }
 

@@ -136,9 +136,9 @@ extern "C" int ss_ghost_discover(ss_ctx *ctx, const int64_t *nbr_ids, int64_t nn
     if (e == hipSuccess) e = s.get(&d_cnt, (size_t)n_words + 1);
     if (e == hipSuccess) e = s.get(&d_pos, (size_t)n_words + 1);
     if (e == hipSuccess) e = s.get(&d_misc, 1);
-    if (e == hipSuccess && nnz) e = hipMemcpyAsync(d_nbr, nbr_ids, sizeof(int64_t) * nnz, hipMemcpyHostToDevice, st);
+    if (e == hipSuccess && nnz) e = ss_copy_in(ctx, d_nbr, nbr_ids, sizeof(int64_t) * (size_t)nnz);
     if (e == hipSuccess && n_owner)
-        e = hipMemcpyAsync(d_owner, owner, sizeof(int32_t) * n_owner, hipMemcpyHostToDevice, st);
+        e = ss_copy_in(ctx, d_owner, owner, sizeof(int32_t) * (size_t)n_owner);
     if (e == hipSuccess) e = hipMemsetAsync(d_bits, 0, sizeof(uint32_t) * (size_t)std::max<int64_t>(n_words, 1), st);
     if (e == hipSuccess) e = hipMemsetAsync(d_cnt, 0, sizeof(int32_t) * (size_t)(n_words + 1), st);
     if (e == hipSuccess) e = hipMemsetAsync(d_misc, 0, sizeof(int32_t), st);
@@ -204,9 +204,8 @@ extern "C" int ss_ghost_discover(ss_ctx *ctx, const int64_t *nbr_ids, int64_t nn
     if (e == hipSuccess) e = hipMemcpyAsync(&bad, d_misc, sizeof(int32_t), hipMemcpyDeviceToHost, st);
     if (e == hipSuccess)
         e = hipMemcpyAsync(recv_offsets, d_off, sizeof(int32_t) * ((size_t)n_ranks + 1), hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess && total) e = hipMemcpyAsync(ghost_ids, d_ids, sizeof(int64_t) * total, hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess && total)
-        e = hipMemcpyAsync(recv_index, d_idx2, sizeof(int32_t) * total, hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = ss_copy_out(ctx, ghost_ids, d_ids, sizeof(int64_t) * (size_t)total);
+    if (e == hipSuccess) e = ss_copy_out(ctx, recv_index, d_idx2, sizeof(int32_t) * (size_t)total);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     if (e != hipSuccess) {
         char b[256];

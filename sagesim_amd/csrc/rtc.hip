@@ -357,8 +357,8 @@ int ss_prog_set_csr(ss_prog *p, const int64_t *row_ptr, const int32_t *col_idx, 
     pfree(p->col_idx);
     p->col_idx = nullptr;
     P_HIP(p, hipMalloc((void **)&p->col_idx, sizeof(int32_t) * (size_t)std::max<int64_t>(nnz, 1)));
-    if (nnz) P_HIP(p, hipMemcpy(p->col_idx, col_idx, sizeof(int32_t) * nnz, hipMemcpyHostToDevice));
-    P_HIP(p, hipMemcpy(p->row_ptr, row_ptr, sizeof(int64_t) * (p->n + 1), hipMemcpyHostToDevice));
+    P_HIP(p, ss_copy_in(p->ctx, p->col_idx, col_idx, sizeof(int32_t) * (size_t)nnz));
+    P_HIP(p, ss_copy_in(p->ctx, p->row_ptr, row_ptr, sizeof(int64_t) * (size_t)(p->n + 1)));
     p->nnz = nnz;
     p->h_row_ptr.assign(row_ptr, row_ptr + p->n + 1);
     for (Launch &l : p->schedule) l.n_long = l.long_deg = 0;   // of the rows before
@@ -407,9 +407,10 @@ int ss_prog_add_array(ss_prog *p, int32_t elem_bytes, int64_t rows, int64_t widt
     const size_t nb = q.bytes();
     hipError_t e = hipSuccess;
     if (nb) {
-        if (init) e = hipMemcpy(q.r, init, nb, hipMemcpyHostToDevice);
-        else e = hipMemset(q.r, 0, nb);
-        if (e == hipSuccess && q.w != q.r) e = hipMemcpy(q.w, q.r, nb, hipMemcpyDeviceToDevice);
+        if (init) e = ss_copy_in(p->ctx, q.r, init, nb);
+        else e = hipMemsetAsync(q.r, 0, nb, p->ctx->stream);
+        if (e == hipSuccess && q.w != q.r) e = hipMemcpyAsync(q.w, q.r, nb, hipMemcpyDeviceToDevice, p->ctx->stream);
+        if (e != hipSuccess) (void)hipStreamSynchronize(p->ctx->stream);
     }
     if (e != hipSuccess) {
         if (q.w != q.r) pfree(q.w);
@@ -435,8 +436,8 @@ int ss_prog_prop_upload(ss_prog *p, int32_t id, const void *data) {
     const size_t nb = q.bytes();
     P_HIP(p, hipStreamSynchronize(p->ctx->stream));
     if (nb) {
-        P_HIP(p, hipMemcpy(q.r, data, nb, hipMemcpyHostToDevice));
-        if (q.w != q.r) P_HIP(p, hipMemcpy(q.w, data, nb, hipMemcpyHostToDevice));
+        P_HIP(p, ss_copy_in(p->ctx, q.r, data, nb));
+        if (q.w != q.r) P_HIP(p, hipMemcpyAsync(q.w, q.r, nb, hipMemcpyDeviceToDevice, p->ctx->stream));
     }
     return SS_OK;
 }
@@ -445,9 +446,7 @@ int ss_prog_prop_download(ss_prog *p, int32_t id, void *out) {
     P_LIVE(p);
     if (!p || id < 0 || id >= (int32_t)p->props.size() || !out) P_FAIL(p, SS_ERR_INVALID, "bad array or NULL");
     const ProgProp &q = p->props[id];
-    P_HIP(p, hipStreamSynchronize(p->ctx->stream));
-    const size_t nb = q.bytes();
-    if (nb) P_HIP(p, hipMemcpy(out, q.r, nb, hipMemcpyDeviceToHost));
+    P_HIP(p, ss_copy_out(p->ctx, out, q.r, q.bytes()));
     return SS_OK;
 }
 
@@ -491,7 +490,7 @@ int ss_prog_set_extra(ss_prog *p, int32_t slot, int64_t bytes, const void *data)
         P_HIP(p, hipMalloc(&x.d, (size_t)std::max<int64_t>(bytes, 16)));
         x.bytes = bytes;
     }
-    if (bytes) P_HIP(p, hipMemcpy(x.d, data, (size_t)bytes, hipMemcpyHostToDevice));
+    P_HIP(p, ss_copy_in(p->ctx, x.d, data, (size_t)bytes));
     return push_args(p);
 }
 
@@ -500,8 +499,7 @@ int ss_prog_get_extra(ss_prog *p, int32_t slot, int64_t bytes, void *out) {
     if (!p || slot < 0 || slot >= SS_MAXX_HOST || (bytes && !out)) P_FAIL(p, SS_ERR_INVALID, "bad extra slot or NULL");
     const Extra &x = p->extras[slot];
     if (!x.d || bytes != x.bytes) P_FAIL(p, SS_ERR_INVALID, "extra slot %d holds %lld bytes", slot, (long long)x.bytes);
-    P_HIP(p, hipStreamSynchronize(p->ctx->stream));
-    if (bytes) P_HIP(p, hipMemcpy(out, x.d, (size_t)bytes, hipMemcpyDeviceToHost));
+    P_HIP(p, ss_copy_out(p->ctx, out, x.d, (size_t)bytes));
     return SS_OK;
 }
 

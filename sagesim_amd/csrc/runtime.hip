@@ -505,6 +505,7 @@ int ss_destroy(ss_ctx *ctx) {
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
     (void)hipStreamSynchronize(ctx->copy_stream);
+    ss_stager_close(ctx);
     drop_graphs(ctx);
     ss_release_programs(ctx);
     for (auto &r : ctx->reps) free_replica(r);
@@ -646,10 +647,10 @@ int ss_replica_create(ss_ctx *ctx, const ss_replica_spec *sp, int32_t *rep_out) 
         if (nl > 0) std::memcpy(rp.data(), sp->row_ptr, sizeof(int64_t) * (nl + 1));
         else rp[0] = 0;
         for (int64_t i = nl + 1; i <= nt; ++i) rp[i] = nnz;  // ghost rows are empty
-        R_HIP(hipMemcpy(r.row_ptr, rp.data(), sizeof(int64_t) * rp.size(), hipMemcpyHostToDevice));
+        R_HIP(ss_copy_in(ctx, r.row_ptr, rp.data(), sizeof(int64_t) * rp.size()));
     }
     if (nnz) {
-        R_HIP(hipMemcpy(r.col_idx, sp->col_idx, sizeof(int32_t) * nnz, hipMemcpyHostToDevice));
+        R_HIP(ss_copy_in(ctx, r.col_idx, sp->col_idx, sizeof(int32_t) * (size_t)nnz));
         unsigned long long first_bad = ~0ull;
         R_HIP(hipMemcpy(ctx->d_stats, &first_bad, sizeof first_bad, hipMemcpyHostToDevice));
         R_HIP(ss_launch_check_cols(r.col_idx, nnz, nt, ctx->d_stats, ctx->num_cus * 8, ctx->stream));
@@ -673,14 +674,14 @@ int ss_replica_create(ss_ctx *ctx, const ss_replica_spec *sp, int32_t *rep_out) 
             kh = (kh ^ (uint64_t)sp->rng_key_id[i]) * 1099511628211ull;
         }
         r.key_hash = kh;
-        if (nl) R_HIP(hipMemcpy(r.rng_lo, lo.data(), sizeof(uint32_t) * nl, hipMemcpyHostToDevice));
+        R_HIP(ss_copy_in(ctx, r.rng_lo, lo.data(), sizeof(uint32_t) * (size_t)nl));
         std::vector<uint8_t> d8((size_t)std::max<int64_t>(nl, 1));
         for (int64_t i = 0; i < nl; ++i)
             d8[i] = (uint8_t)std::min<int64_t>(sp->row_ptr[i + 1] - sp->row_ptr[i], 255);
-        if (nl) R_HIP(hipMemcpy(r.deg8, d8.data(), nl, hipMemcpyHostToDevice));
-        if (need_hi) R_HIP(hipMemcpy(r.rng_hi, hi.data(), sizeof(uint32_t) * nl, hipMemcpyHostToDevice));
+        R_HIP(ss_copy_in(ctx, r.deg8, d8.data(), (size_t)nl));
+        if (need_hi) R_HIP(ss_copy_in(ctx, r.rng_hi, hi.data(), sizeof(uint32_t) * (size_t)nl));
     }
-    if (nt) R_HIP(hipMemcpy(r.init_state, sp->state, (size_t)nt, hipMemcpyHostToDevice));
+    R_HIP(ss_copy_in(ctx, r.init_state, sp->state, (size_t)nt));
     // the push direction needs every entry's mirror (a neighbour's row then
     // lists the agent) and no ghosts (ghost rows are empty)
     r.symmetric = nnz == 0;
@@ -695,7 +696,7 @@ int ss_replica_create(ss_ctx *ctx, const ss_replica_spec *sp, int32_t *rep_out) 
         r.csr_hash[1] = h[1];
     }
     if (sp->history)
-        R_HIP(hipMemcpy(r.init_history, sp->history, sizeof(int32_t) * nl * SS_HISTORY_WIDTH, hipMemcpyHostToDevice));
+        R_HIP(ss_copy_in(ctx, r.init_history, sp->history, sizeof(int32_t) * (size_t)nl * SS_HISTORY_WIDTH));
     r.dev = ss_rep_dev{};
     r.dev.row_ptr = r.row_ptr;
     r.dev.col_idx = r.col_idx;
@@ -813,8 +814,7 @@ int ss_state_download(ss_ctx *ctx, int32_t rep, int8_t *out, int64_t n) {
     if (!valid_rep(ctx, rep) || (!out && n)) SS_FAIL(ctx, SS_ERR_INVALID, "bad replica or NULL");
     ss_replica &r = ctx->reps[rep];
     if (n != r.n_total) SS_FAIL(ctx, SS_ERR_INVALID, "n = %lld, replica has %lld slots", (long long)n, (long long)r.n_total);
-    SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    if (n) SS_HIP(ctx, hipMemcpy(out, r.state[r.tick & 1], (size_t)n, hipMemcpyDeviceToHost));
+    SS_HIP(ctx, ss_copy_out(ctx, out, r.state[r.tick & 1], (size_t)n));
     return SS_OK;
 }
 
@@ -826,7 +826,7 @@ int ss_replica_set_order(ss_ctx *ctx, int32_t rep, const int32_t *slot, int64_t 
     SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
     if (!r.order) SS_HIP(ctx, dalloc(ctx, &r, &r.order, (size_t)pad_agents(n)));
     unsigned long long bad = ~0ull;
-    SS_HIP(ctx, hipMemcpy(r.order, slot, sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice));
+    SS_HIP(ctx, ss_copy_in(ctx, r.order, slot, sizeof(int32_t) * (size_t)n));
     SS_HIP(ctx, hipMemcpy(ctx->d_stats, &bad, sizeof bad, hipMemcpyHostToDevice));
     SS_HIP(ctx, ss_launch_check_cols(r.order, n, n, ctx->d_stats, ctx->num_cus * 8, ctx->stream));
     SS_HIP(ctx, hipMemcpyAsync(&bad, ctx->d_stats, sizeof bad, hipMemcpyDeviceToHost, ctx->stream));
@@ -849,9 +849,16 @@ int ss_state_download_ordered(ss_ctx *ctx, int32_t rep, int8_t *out, int64_t n) 
         if (r.n_local) SS_FAIL(ctx, SS_ERR_STATE, "replica has no order (ss_replica_set_order)");
         return ss_state_download(ctx, rep, out, n);
     }
+    const int8_t *st = r.state[r.tick & 1];
+    if (!ss_known_to_hip(out)) {
+        SS_HIP(ctx, ss_stage_out(ctx, out, (size_t)n, [&](size_t at, size_t len, void *slot) {
+            return ss_launch_order(st, r.order, (int8_t *)slot, (int64_t)at, (int64_t)(at + len), r.n_local, ctx->stream);
+        }));
+        return SS_OK;
+    }
     void *d = nullptr;
     SS_HIP(ctx, scratch(ctx, (size_t)pad_agents(n), &d));
-    SS_HIP(ctx, ss_launch_order(r.state[r.tick & 1], r.order, (int8_t *)d, r.n_local, n, ctx->stream));
+    SS_HIP(ctx, ss_launch_order(st, r.order, (int8_t *)d, 0, n, r.n_local, ctx->stream));
     SS_HIP(ctx, hipMemcpyAsync(out, d, (size_t)n, hipMemcpyDeviceToHost, ctx->stream));
     SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return SS_OK;
@@ -864,8 +871,8 @@ int ss_state_upload(ss_ctx *ctx, int32_t rep, const int8_t *in, int64_t n) {
     SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
     const int par = (int)(r.tick & 1);
     if (n) {
-        SS_HIP(ctx, hipMemcpy(r.state[par], in, (size_t)n, hipMemcpyHostToDevice));
-        SS_HIP(ctx, hipMemcpy(r.state[par ^ 1], in, (size_t)n, hipMemcpyHostToDevice));
+        SS_HIP(ctx, ss_copy_in(ctx, r.state[par], in, (size_t)n));
+        SS_HIP(ctx, hipMemcpyAsync(r.state[par ^ 1], r.state[par], (size_t)n, hipMemcpyDeviceToDevice, ctx->stream));
     }
     int rc = rebuild_bits(ctx, r, par, 0, r.n_words);
     if (rc) return rc;
@@ -878,8 +885,7 @@ int ss_history_download(ss_ctx *ctx, int32_t rep, int32_t *out, int64_t n_rows) 
     ss_replica &r = ctx->reps[rep];
     if (!r.history) SS_FAIL(ctx, SS_ERR_STATE, "replica has no history property");
     if (n_rows != r.n_local) SS_FAIL(ctx, SS_ERR_INVALID, "n_rows must equal n_local");
-    SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    SS_HIP(ctx, hipMemcpy(out, r.history, sizeof(int32_t) * n_rows * SS_HISTORY_WIDTH, hipMemcpyDeviceToHost));
+    SS_HIP(ctx, ss_copy_out(ctx, out, r.history, sizeof(int32_t) * (size_t)n_rows * SS_HISTORY_WIDTH));
     return SS_OK;
 }
 
@@ -1089,9 +1095,8 @@ int ss_map_build(ss_ctx *ctx, int32_t rep, const int64_t *ids, const int32_t *sl
     int32_t *d_vals = (int32_t *)((char *)w + b_ids);
     if ((rc = alloc_map(ctx, r, cap, n == 0))) return rc;
     if (n > 0) {
-        hipError_t e = hipMemcpyAsync(d_ids, ids, sizeof(int64_t) * (size_t)n, hipMemcpyHostToDevice, ctx->stream);
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(d_vals, slots, sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice, ctx->stream);
+        hipError_t e = ss_copy_in(ctx, d_ids, ids, sizeof(int64_t) * (size_t)n);
+        if (e == hipSuccess) e = ss_copy_in(ctx, d_vals, slots, sizeof(int32_t) * (size_t)n);
         if (e == hipSuccess)
             e = ss_launch_map_build(r.map_keys, r.map_vals, cap, d_ids, d_vals, n,
                                     (unsigned long long *)((char *)w + b_ids + b_vals), ctx->num_cus, ctx->stream);
@@ -1187,7 +1192,7 @@ static int lookup_dev(ss_ctx *ctx, ss_replica &r, const int64_t *ids, int64_t *d
     uint32_t *d = (uint32_t *)ctx->d_counters;
     SS_HIP(ctx, hipMemsetAsync(d, 0, sizeof(uint32_t), ctx->stream));
     SS_HIP(ctx, hipMemsetAsync(d + 1, 0xFF, sizeof(uint32_t), ctx->stream));
-    SS_HIP(ctx, hipMemcpyAsync(d_ids, ids, sizeof(int64_t) * (size_t)n, hipMemcpyHostToDevice, ctx->stream));
+    SS_HIP(ctx, ss_copy_in(ctx, d_ids, ids, sizeof(int64_t) * (size_t)n));
     SS_HIP(ctx, ss_launch_map_lookup(r.map_keys, r.map_vals, r.map_cap, d_ids, d_out, n, d, lowest, ctx->num_cus,
                                      ctx->stream));
     SS_HIP(ctx, hipMemcpyAsync(counts, d, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
@@ -1207,7 +1212,7 @@ int ss_map_lookup(ss_ctx *ctx, int32_t rep, const int64_t *ids, int32_t *out, in
     uint32_t counts[2] = {0, 0};
     int rc = lookup_dev(ctx, r, ids, (int64_t *)w, d_out, n, false, counts);
     if (rc) return rc;
-    SS_HIP(ctx, hipMemcpyAsync(out, d_out, sizeof(int32_t) * (size_t)n, hipMemcpyDeviceToHost, ctx->stream));
+    SS_HIP(ctx, ss_copy_out(ctx, out, d_out, sizeof(int32_t) * (size_t)n));
     SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
     if (n_missing) *n_missing = counts[0];
     return SS_OK;
@@ -1315,8 +1320,8 @@ int ss_halo_unpack_ids(ss_ctx *ctx, int32_t rep, const int64_t *ids, const int8_
     int8_t *d_vals = (int8_t *)w + b_ids;
     int32_t miss = 0;
     SS_HIP(ctx, hipMemsetAsync(ctx->d_counters, 0, sizeof(int32_t), ctx->stream));
-    SS_HIP(ctx, hipMemcpyAsync(w, ids, sizeof(int64_t) * (size_t)n, hipMemcpyHostToDevice, ctx->stream));
-    SS_HIP(ctx, hipMemcpyAsync(d_vals, vals, (size_t)n, hipMemcpyHostToDevice, ctx->stream));
+    SS_HIP(ctx, ss_copy_in(ctx, w, ids, sizeof(int64_t) * (size_t)n));
+    SS_HIP(ctx, ss_copy_in(ctx, d_vals, vals, (size_t)n));
     SS_HIP(ctx, ss_launch_halo_unpack_ids(r.map_keys, r.map_vals, r.map_cap, (const int64_t *)w, d_vals, n, r.state[0],
                                           r.state[1], ctx->d_counters, ctx->stream));
     SS_HIP(ctx, hipMemcpyAsync(&miss, ctx->d_counters, sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
@@ -1354,11 +1359,10 @@ static int halo_pack(ss_ctx *ctx, int32_t rep, const int32_t *slots, int64_t n, 
     void *w = nullptr;
     SS_HIP(ctx, scratch(ctx, b_slots + nb, &w));
     int8_t *d_out = (int8_t *)w + b_slots;
-    SS_HIP(ctx, hipMemcpyAsync(w, slots, sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice, ctx->stream));
+    SS_HIP(ctx, ss_copy_in(ctx, w, slots, sizeof(int32_t) * (size_t)n));
     SS_HIP(ctx, packed ? ss_launch_gather2(r.state[r.tick & 1], (const int32_t *)w, (uint8_t *)d_out, n, ctx->stream)
                        : ss_launch_gather(r.state[r.tick & 1], (const int32_t *)w, d_out, n, ctx->stream));
-    SS_HIP(ctx, hipMemcpyAsync(out, d_out, nb, hipMemcpyDeviceToHost, ctx->stream));
-    SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    SS_HIP(ctx, ss_copy_out(ctx, out, d_out, nb));
     return SS_OK;
 }
 

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <functional>
 #include <map>
 #include <string>
 #include <vector>
@@ -57,12 +58,27 @@ hipError_t ss_launch_gather(const int8_t *st, const int32_t *slots, int8_t *out,
 // out[h / 4] bits 2 (h % 4).. = st[slots[h]] & 3
 hipError_t ss_launch_gather2(const int8_t *st, const int32_t *slots, uint8_t *out, int64_t n, hipStream_t s);
 hipError_t ss_launch_fill_i32(int32_t *p, int64_t n, int32_t v, hipStream_t s);
-// out[j] = st[slot[j]], j < n_local; out[j] = st[j] for the ghosts (slot and
-// out padded to whole groups of 16)
-hipError_t ss_launch_order(const int8_t *st, const int32_t *slot, int8_t *out, int64_t n_local, int64_t n_total,
-                           hipStream_t s);
+// out[j - first] = st[slot[j]], j < n_local; st[j] for the ghosts; for
+// first <= j < end (slot and out padded to whole groups of 16, first a multiple)
+hipError_t ss_launch_order(const int8_t *st, const int32_t *slot, int8_t *out, int64_t first, int64_t end,
+                           int64_t n_local, hipStream_t s);
 hipError_t ss_launch_copy(const void *src, void *dst, int64_t bytes, int grid, hipStream_t s);
-// bytes and a table of 8-byte words from page-locked host memory to device
+// ---- staging.hip: copies of ordinary host memory on the context's stream ----
+// Up: the caller's memory is read when it returns, the device has it for what
+// follows on the stream.  Down: the caller has it when it returns.
+#define SS_STAGE_LANES 4
+struct ss_ctx;
+struct ss_stager;
+hipError_t ss_copy_in(ss_ctx *ctx, void *dev, const void *host, size_t bytes);
+hipError_t ss_copy_out(ss_ctx *ctx, void *host, const void *dev, size_t bytes);
+// down, of what issue(at, len, slot) writes into page-locked memory: bytes
+// [at, at + len) of the result to slot, enqueued on the context's stream, by any of its threads
+typedef std::function<hipError_t(size_t at, size_t len, void *slot)> ss_stage_issue;
+hipError_t ss_stage_out(ss_ctx *ctx, void *host, size_t bytes, const ss_stage_issue &issue);
+bool ss_known_to_hip(const void *p);            // page-locked or device memory
+void ss_stager_close(ss_ctx *ctx);
+
+// bytes and a table of 8-byte words between page-locked host memory and device
 // memory, by one kernel
 hipError_t ss_launch_stage(const void *src, void *dst, int64_t bytes, const uint64_t *src2, uint64_t *dst2,
                            int64_t words2, hipStream_t s);
@@ -185,6 +201,7 @@ struct ss_ctx {
     hipEvent_t span_ev[2][SS_HALO_SPANS] = {};  // copy span s of group buffer b is on the device
     int64_t grp_pos = 0;                        // groups issued (buffer = grp_pos & 1)
     bool halo_fused = false;                    // this call's ticks fuse the next tick's halo refresh
+    ss_stager *stager = nullptr;                // page-locked chunks and threads of large copies (staging.hip)
     void *h_stage = nullptr;                    // page-locked, SS_STAGE_BYTES: a small pack's slots and result
     void *scratch = nullptr;                    // workspace of one call at a time, on the context's stream
     size_t scratch_bytes = 0;
