@@ -19,31 +19,132 @@ __device__ __forceinline__ uint64_t mix64(uint64_t x) {
 
 // Symmetry of a CSR as a multiset test: the sums of two independent hashes
 // over all entries (i, j) equal those over the mirrored entries (j, i) when
-// every entry has its mirror.  One thread per row.
-__global__ void symcheck_kernel(const int64_t *__restrict__ row_ptr, const int32_t *__restrict__ col, int64_t n,
-                                unsigned long long *out) {
-    unsigned long long a0 = 0, a1 = 0, b0 = 0, b1 = 0;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t b = row_ptr[i], e = row_ptr[i + 1];
-#pragma unroll 4
-        for (int64_t j = b; j < e; ++j) {
-            const uint64_t c = (uint32_t)col[j];
+// every entry has its mirror.
+// Row b of part (SS_STATS_ROW words, page-locked) gets block b's words 0 .. 3:
+// the sums, and 4: the complement of the first entry outside [0, n_total), 0 if
+// all are inside.  A thread takes 16 entries at a time (64 bytes) wherever its rows begin,
+// and finds the row of the first by halving, so that a hub's row is shared by as
+// many threads as it has entries for.  Bound by the 64-bit products (eight an
+// entry) and the halving's chain of loads, once for 16 entries: 36 us for the
+// 6.8M entries of a BA(851k), where a row to a thread took 1033 us, the longest
+// row's walk.  Rows that do not ascend only give sums that nobody uses.
+__device__ __forceinline__ int64_t row_of(const int64_t *__restrict__ row_ptr, int64_t j, int64_t lo, int64_t hi) {
+    while (hi - lo > 1) {                               // the last row in [lo, hi) that begins at or before j
+        const int64_t mid = (lo + hi) >> 1;
+        if (row_ptr[mid] <= j) lo = mid;
+        else hi = mid;
+    }
+    return lo;
+}
+
+__global__ __launch_bounds__(256) void entries_kernel(const int64_t *__restrict__ row_ptr,
+                                                      const int32_t *__restrict__ col, int64_t n, int64_t nnz,
+                                                      int64_t n_total, unsigned long long *part) {
+    unsigned long long h[5] = {0, 0, 0, 0, 0};
+    const int64_t stride = 16 * (int64_t)gridDim.x * blockDim.x;
+    for (int64_t j0 = 16 * ((int64_t)blockIdx.x * blockDim.x + threadIdx.x); j0 < nnz; j0 += stride) {
+        int64_t i = row_of(row_ptr, j0, 0, n), next = row_ptr[i + 1];
+        auto entry = [&](int64_t j, int32_t e) {
+            if (j >= next && i + 1 < n) {
+                next = row_ptr[++i + 1];
+                if (j >= next) {                        // past empty rows
+                    i = row_of(row_ptr, j, i, n);
+                    next = row_ptr[i + 1];
+                }
+            }
+            if ((e < 0 || (int64_t)e >= n_total) && ~(unsigned long long)j > h[4]) h[4] = ~(unsigned long long)j;
+            const uint64_t c = (uint32_t)e;
             const uint64_t fwd = ((uint64_t)i << 32) | c, bwd = (c << 32) | (uint64_t)i;
-            a0 += mix64(fwd ^ 0x9E3779B97F4A7C15ull);
-            a1 += mix64(fwd * 0xD6E8FEB86659FD93ull + 0x2545F4914F6CDD1Dull);
-            b0 += mix64(bwd ^ 0x9E3779B97F4A7C15ull);
-            b1 += mix64(bwd * 0xD6E8FEB86659FD93ull + 0x2545F4914F6CDD1Dull);
+            h[0] += mix64(fwd ^ 0x9E3779B97F4A7C15ull);
+            h[1] += mix64(fwd * 0xD6E8FEB86659FD93ull + 0x2545F4914F6CDD1Dull);
+            h[2] += mix64(bwd ^ 0x9E3779B97F4A7C15ull);
+            h[3] += mix64(bwd * 0xD6E8FEB86659FD93ull + 0x2545F4914F6CDD1Dull);
+        };
+        if (j0 + 16 <= nnz) {
+            int4 v[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[q] = *(const int4 *)(col + j0 + 4 * q);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                entry(j0 + 4 * q, v[q].x);
+                entry(j0 + 4 * q + 1, v[q].y);
+                entry(j0 + 4 * q + 2, v[q].z);
+                entry(j0 + 4 * q + 3, v[q].w);
+            }
+        } else {
+            for (int64_t j = j0; j < nnz; ++j) entry(j, col[j]);
         }
     }
+    __shared__ unsigned long long red[4][5];
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
-        a0 += __shfl_down(a0, off); a1 += __shfl_down(a1, off);
-        b0 += __shfl_down(b0, off); b1 += __shfl_down(b1, off);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) h[q] += __shfl_down(h[q], off);
+        const unsigned long long o = __shfl_down(h[4], off);
+        h[4] = o > h[4] ? o : h[4];
     }
-    if ((threadIdx.x & 63) == 0) {
-        atomicAdd(&out[0], a0); atomicAdd(&out[1], a1);
-        atomicAdd(&out[2], b0); atomicAdd(&out[3], b1);
+    if ((threadIdx.x & 63) == 0)
+        for (int q = 0; q < 5; ++q) red[threadIdx.x >> 6][q] = h[q];
+    __syncthreads();
+    if (threadIdx.x < 5) {
+        unsigned long long t = red[0][threadIdx.x];
+        for (int w = 1; w < 4; ++w) {
+            const unsigned long long o = red[w][threadIdx.x];
+            t = threadIdx.x < 4 ? t + o : o > t ? o : t;
+        }
+        part[SS_STATS_ROW * blockIdx.x + threadIdx.x] = t;
     }
+}
+
+// What a replica keeps by agent, from its rows and key ids, in one pass: degrees
+// in a byte, the key ids' low words, the entries before every 64th agent, the
+// empty rows of the ghosts (nnz each).  Row b of part gets words 5: the
+// complement of the first row that is negative (0: none), 6: the longest row,
+// 7: the high words of the key ids or'ed.  Bound by the 21 bytes an agent.
+__global__ __launch_bounds__(256) void agents_kernel(int64_t *__restrict__ row_ptr, const int64_t *__restrict__ ids,
+                                                     int64_t n, int64_t n_total, int64_t nnz, uint8_t *__restrict__ deg8,
+                                                     uint32_t *__restrict__ lo, int64_t *__restrict__ edge64,
+                                                     unsigned long long *part) {
+    unsigned long long w[3] = {0, 0, 0};
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i <= n_total; i += stride) {
+        const int64_t b = i <= n && n > 0 ? row_ptr[i] : nnz;
+        if (i > n || n == 0) row_ptr[i] = nnz;
+        if (i % 64 == 0 && i < n_total) edge64[i / 64] = b;
+        if (i >= n) continue;
+        const int64_t d = row_ptr[i + 1] - b;
+        deg8[i] = (uint8_t)(d < 0 ? 0 : d < 255 ? d : 255);
+        if (d < 0) w[0] = ~(unsigned long long)i > w[0] ? ~(unsigned long long)i : w[0];
+        else w[1] = (unsigned long long)d > w[1] ? (unsigned long long)d : w[1];
+        const uint64_t id = (uint64_t)ids[i];
+        lo[i] = (uint32_t)id;
+        w[2] |= id >> 32;
+    }
+    __shared__ unsigned long long red[4][3];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const unsigned long long o = __shfl_down(w[q], off);
+            w[q] = q == 2 ? w[q] | o : o > w[q] ? o : w[q];
+        }
+    if ((threadIdx.x & 63) == 0)
+        for (int q = 0; q < 3; ++q) red[threadIdx.x >> 6][q] = w[q];
+    __syncthreads();
+    if (threadIdx.x < 3) {
+        unsigned long long t = red[0][threadIdx.x];
+        for (int v = 1; v < 4; ++v) {
+            const unsigned long long o = red[v][threadIdx.x];
+            t = threadIdx.x == 2 ? t | o : o > t ? o : t;
+        }
+        part[SS_STATS_ROW * blockIdx.x + 5 + threadIdx.x] = t;
+    }
+}
+
+__global__ __launch_bounds__(256) void high_words_kernel(const int64_t *__restrict__ ids, int64_t n,
+                                                         uint32_t *__restrict__ hi) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) hi[i] = (uint32_t)((uint64_t)ids[i] >> 32);
 }
 
 // Rebuild bitmap words [w0, w1) of one state buffer.
@@ -375,11 +476,27 @@ inline unsigned grid_for(int64_t n, int b) { return (unsigned)((n + b - 1) / b);
 }  // namespace
 
 // ---- launchers (host) ----
-hipError_t ss_launch_symcheck(const int64_t *row_ptr, const int32_t *col_idx, int64_t n_rows,
-                              unsigned long long *out, int grid, hipStream_t s) {
-    if (n_rows <= 0) return hipSuccess;
-    int g = (int)std::min<int64_t>(grid, (int64_t)grid_for(n_rows, 256));
-    hipLaunchKernelGGL(symcheck_kernel, dim3(g), dim3(256), 0, s, row_ptr, col_idx, n_rows, out);
+hipError_t ss_launch_entries(const int64_t *row_ptr, const int32_t *col_idx, int64_t n_rows, int64_t nnz,
+                             int64_t n_total, unsigned long long *part, int max_blocks, int *blocks, hipStream_t s) {
+    *blocks = 0;
+    if (nnz <= 0 || n_rows <= 0) return hipSuccess;
+    *blocks = (int)std::min<int64_t>(max_blocks, (int64_t)grid_for(nnz, 16 * 256));
+    hipLaunchKernelGGL(entries_kernel, dim3(*blocks), dim3(256), 0, s, row_ptr, col_idx, n_rows, nnz, n_total, part);
+    return hipGetLastError();
+}
+
+hipError_t ss_launch_agents(int64_t *row_ptr, const int64_t *ids, int64_t n, int64_t n_total, int64_t nnz,
+                            uint8_t *deg8, uint32_t *lo, int64_t *edge64, unsigned long long *part, int max_blocks,
+                            int *blocks, hipStream_t s) {
+    *blocks = (int)std::min<int64_t>(max_blocks, (int64_t)grid_for(n_total + 1, 256));
+    hipLaunchKernelGGL(agents_kernel, dim3(*blocks), dim3(256), 0, s, row_ptr, ids, n, n_total, nnz, deg8, lo, edge64,
+                       part);
+    return hipGetLastError();
+}
+
+hipError_t ss_launch_high_words(const int64_t *ids, int64_t n, uint32_t *hi, hipStream_t s) {
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(high_words_kernel, dim3(grid_for(n, 256)), dim3(256), 0, s, ids, n, hi);
     return hipGetLastError();
 }
 

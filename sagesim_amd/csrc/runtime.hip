@@ -4,6 +4,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <thread>
 #include <string>
 
 #include "../../include/sagestep.h"
@@ -142,7 +143,7 @@ int apply_model(ss_ctx *ctx, ss_replica &r, const ss_model *m) {
     dfree(r.inf_T);
     r.inf_T = nullptr;
     SS_HIP(ctx, dalloc(ctx, &r, &r.inf_T, T.size()));
-    SS_HIP(ctx, hipMemcpy(r.inf_T, T.data(), T.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+    SS_HIP(ctx, ss_copy_in(ctx, r.inf_T, T.data(), T.size() * sizeof(uint32_t)));
     r.dev.inf_T = r.inf_T;
     r.dev.inf_T_last = (int32_t)T.size() - 1;
     for (int s = 0; s < 4; ++s) {
@@ -562,6 +563,38 @@ int64_t ss_replica_footprint(int64_t n_local, int64_t n_ghost, int64_t nnz, int3
     return b;
 }
 
+// Hash of the RNG key ids (checkpoint identity): a product chain of some five
+// cycles an id, so a long one runs on a thread of its own beside the uploads
+// (1.2 ms of 850k agents).
+struct KeyHash {
+    const int64_t *ids;
+    int64_t n;
+    uint64_t h = 1469598103934665603ull;
+    std::thread t;
+    bool ready = false;
+    void run() {
+        uint64_t v = h;
+        for (int64_t i = 0; i < n; ++i) v = (v ^ (uint64_t)ids[i]) * 1099511628211ull;
+        h = v;
+    }
+    KeyHash(const int64_t *ids_, int64_t n_) : ids(ids_), n(n_) {
+        if (n < 100000) return;
+        try {
+            t = std::thread([this] { run(); });
+        } catch (...) {                                 // no thread: get() does it
+        }
+    }
+    uint64_t get() {
+        if (t.joinable()) t.join();
+        else if (!ready) run();
+        ready = true;
+        return h;
+    }
+    ~KeyHash() {
+        if (t.joinable()) t.join();
+    }
+};
+
 int ss_replica_create(ss_ctx *ctx, const ss_replica_spec *sp, int32_t *rep_out) {
     if (!ctx || !sp || !rep_out) SS_FAIL(ctx, SS_ERR_INVALID, "NULL argument");
     (void)hipSetDevice(ctx->device);
@@ -569,34 +602,24 @@ int ss_replica_create(ss_ctx *ctx, const ss_replica_spec *sp, int32_t *rep_out) 
     if (nl < 0 || ng < 0 || nnz < 0 || nt > INT32_MAX) SS_FAIL(ctx, SS_ERR_RANGE, "slot counts out of range");
     if ((nl > 0 && (!sp->row_ptr || !sp->rng_key_id)) || (nt > 0 && !sp->state) || (nnz > 0 && !sp->col_idx))
         SS_FAIL(ctx, SS_ERR_INVALID, "missing arrays");
-    // shape checks on the host before anything reaches a kernel
-    int64_t max_deg = 0;
     if (nl > 0) {
         if (sp->row_ptr[0] != 0 || sp->row_ptr[nl] != nnz) SS_FAIL(ctx, SS_ERR_INVALID, "row_ptr[0] must be 0 and row_ptr[n_local] == nnz");
-        for (int64_t i = 0; i < nl; ++i) {
-            int64_t d = sp->row_ptr[i + 1] - sp->row_ptr[i];
-            if (d < 0) SS_FAIL(ctx, SS_ERR_INVALID, "row_ptr decreases at row %lld", (long long)i);
-            max_deg = std::max(max_deg, d);
-        }
     } else if (nnz != 0) {
         SS_FAIL(ctx, SS_ERR_INVALID, "nnz must be 0 without local rows");
     }
-    // col_idx is range-checked on the device right after its upload (below),
-    // before any kernel indexes with it.
+    // the rows and entries are checked on the device right after their upload
+    // (below), before any kernel indexes with them
     int rc = check_model(ctx, &sp->model);
-    if (rc) return rc;
-    bool need_hi = false;
-    for (int64_t i = 0; i < nl; ++i)
-        if ((uint64_t)sp->rng_key_id[i] >> 32) { need_hi = true; break; }
+    if (rc) {
+        for (int64_t i = 0; i < nl; ++i)
+            if (sp->row_ptr[i + 1] < sp->row_ptr[i])
+                SS_FAIL(ctx, SS_ERR_INVALID, "row_ptr decreases at row %lld", (long long)i);
+        return rc;
+    }
 
     ss_replica r;
     r.n_local = nl; r.n_ghost = ng; r.n_total = nt; r.nnz = nnz;
     r.n_words = (nt + 63) / 64;
-    r.max_deg = max_deg;
-    // CSR entries before agents 0, 64, 128, ... and before n_total (light tile sizes)
-    r.edge64.resize((size_t)((nt + 63) / 64 + 1));
-    for (int64_t j = 0; j * 64 < nt; ++j) r.edge64[(size_t)j] = nl > 0 ? sp->row_ptr[std::min(j * 64, nl)] : 0;
-    r.edge64.back() = nnz;
     // heavy prefix lengths for the tiling thresholds the autotuner may pick
     for (int32_t thr : SS_THRESHOLDS) {
         int64_t H = 0;
@@ -620,11 +643,10 @@ int ss_replica_create(ss_ctx *ctx, const ss_replica_spec *sp, int32_t *rep_out) 
     R_HIP(dalloc(ctx, &r, &r.row_ptr, (size_t)nt + 1));
     // a lane's scan reads its row eight entries at a time
     R_HIP(dalloc(ctx, &r, &r.col_idx, (size_t)nnz + SS_COL_PAD));
-    R_HIP(hipMemset(r.col_idx + nnz, 0, sizeof(int32_t) * SS_COL_PAD));
+    R_HIP(hipMemsetAsync(r.col_idx + nnz, 0, sizeof(int32_t) * SS_COL_PAD, ctx->stream));
     // per-agent arrays the light tiles read as 16-agent vectors are padded
     R_HIP(dalloc(ctx, &r, &r.rng_lo, (size_t)pad_agents(nl)));
     R_HIP(dalloc(ctx, &r, &r.deg8, (size_t)pad_agents(nl)));
-    if (need_hi) R_HIP(dalloc(ctx, &r, &r.rng_hi, (size_t)nl));
     for (int b = 0; b < 2; ++b) {
         R_HIP(dalloc(ctx, &r, &r.state[b], (size_t)pad_agents(nt)));
         R_HIP(dalloc(ctx, &r, &r.ibits[b], (size_t)r.n_words));
@@ -635,66 +657,72 @@ int ss_replica_create(ss_ctx *ctx, const ss_replica_spec *sp, int32_t *rep_out) 
         R_HIP(dalloc(ctx, &r, &r.cnt[0], (size_t)pad_agents(nl)));
         R_HIP(dalloc(ctx, &r, &r.cnt[1], (size_t)pad_agents(nl)));
         R_HIP(dalloc(ctx, &r, &r.dec, (size_t)2));
-        R_HIP(hipMemset(r.dec, 0, 2 * sizeof(uint32_t)));
+        R_HIP(hipMemsetAsync(r.dec, 0, 2 * sizeof(uint32_t), ctx->stream));
     }
     if (sp->history) {
         R_HIP(dalloc(ctx, &r, &r.history, (size_t)nl * SS_HISTORY_WIDTH));
         R_HIP(dalloc(ctx, &r, &r.init_history, (size_t)nl * SS_HISTORY_WIDTH));
     }
-    // uploads (synchronous: host arrays are borrowed only for this call)
-    {
-        std::vector<int64_t> rp((size_t)nt + 1);
-        if (nl > 0) std::memcpy(rp.data(), sp->row_ptr, sizeof(int64_t) * (nl + 1));
-        else rp[0] = 0;
-        for (int64_t i = nl + 1; i <= nt; ++i) rp[i] = nnz;  // ghost rows are empty
-        R_HIP(ss_copy_in(ctx, r.row_ptr, rp.data(), sizeof(int64_t) * rp.size()));
-    }
-    if (nnz) {
-        R_HIP(ss_copy_in(ctx, r.col_idx, sp->col_idx, sizeof(int32_t) * (size_t)nnz));
-        unsigned long long first_bad = ~0ull;
-        R_HIP(hipMemcpy(ctx->d_stats, &first_bad, sizeof first_bad, hipMemcpyHostToDevice));
-        R_HIP(ss_launch_check_cols(r.col_idx, nnz, nt, ctx->d_stats, ctx->num_cus * 8, ctx->stream));
-        R_HIP(hipStreamSynchronize(ctx->stream));
-        R_HIP(hipMemcpy(&first_bad, ctx->d_stats, sizeof first_bad, hipMemcpyDeviceToHost));
-        if (first_bad != ~0ull) {
-            char b[200];
-            std::snprintf(b, sizeof b, "col_idx[%llu] = %d outside [0, %lld)", first_bad,
-                          sp->col_idx[first_bad], (long long)nt);
-            ctx->err = b;
-            return fail(SS_ERR_RANGE);
-        }
-    }
-    {
-        std::vector<uint32_t> lo((size_t)std::max<int64_t>(nl, 1)), hi;
-        if (need_hi) hi.resize((size_t)nl);
-        uint64_t kh = 1469598103934665603ull;
-        for (int64_t i = 0; i < nl; ++i) {
-            lo[i] = (uint32_t)sp->rng_key_id[i];
-            if (need_hi) hi[i] = (uint32_t)((uint64_t)sp->rng_key_id[i] >> 32);
-            kh = (kh ^ (uint64_t)sp->rng_key_id[i]) * 1099511628211ull;
-        }
-        r.key_hash = kh;
-        R_HIP(ss_copy_in(ctx, r.rng_lo, lo.data(), sizeof(uint32_t) * (size_t)nl));
-        std::vector<uint8_t> d8((size_t)std::max<int64_t>(nl, 1));
-        for (int64_t i = 0; i < nl; ++i)
-            d8[i] = (uint8_t)std::min<int64_t>(sp->row_ptr[i + 1] - sp->row_ptr[i], 255);
-        R_HIP(ss_copy_in(ctx, r.deg8, d8.data(), (size_t)nl));
-        if (need_hi) R_HIP(ss_copy_in(ctx, r.rng_hi, hi.data(), sizeof(uint32_t) * (size_t)nl));
-    }
+    // uploads (the host arrays are borrowed only for this call), and one wait
+    // for everything the device finds out about them
+    KeyHash keys(sp->rng_key_id, nl);
+    Scratch guard(ctx);
+    void *w = nullptr;
+    const int64_t n64 = (nt + 63) / 64;
+    const size_t b_ids = up256(sizeof(int64_t) * (size_t)nl);
+    R_HIP(scratch(ctx, b_ids + sizeof(int64_t) * (size_t)(n64 + 1), &w));
+    int64_t *d_ids = (int64_t *)w, *d_edge64 = (int64_t *)((char *)w + b_ids);
+    int ab = 0, eb = 0;
+    const int max_blocks = 4 * ctx->num_cus;
+    if (nl) R_HIP(ss_copy_in(ctx, r.row_ptr, sp->row_ptr, sizeof(int64_t) * (size_t)(nl + 1)));
+    R_HIP(ss_copy_in(ctx, d_ids, sp->rng_key_id, sizeof(int64_t) * (size_t)nl));
+    R_HIP(ss_launch_agents(r.row_ptr, d_ids, nl, nt, nnz, r.deg8, r.rng_lo, d_edge64, ctx->h_stats, max_blocks, &ab,
+                           ctx->stream));
+    R_HIP(ss_copy_in(ctx, r.col_idx, sp->col_idx, sizeof(int32_t) * (size_t)nnz));
+    R_HIP(ss_launch_entries(r.row_ptr, r.col_idx, nl, nnz, nt, ctx->h_stats, max_blocks, &eb, ctx->stream));
     R_HIP(ss_copy_in(ctx, r.init_state, sp->state, (size_t)nt));
+    // CSR entries before agents 0, 64, 128, ... and before n_total (light tile sizes)
+    r.edge64.resize((size_t)(n64 + 1));
+    R_HIP(ss_copy_out(ctx, r.edge64.data(), d_edge64, sizeof(int64_t) * (size_t)n64));
+    r.edge64.back() = nnz;
+    R_HIP(hipStreamSynchronize(ctx->stream));
+    unsigned long long h[4] = {0, 0, 0, 0}, bad_col = 0, bad_row = 0, longest = 0, high = 0;
+    for (int b = 0; b < std::max(ab, eb); ++b) {
+        const unsigned long long *q = ctx->h_stats + SS_STATS_ROW * b;
+        if (b < eb) {
+            for (int i = 0; i < 4; ++i) h[i] += q[i];
+            bad_col = std::max(bad_col, q[4]);
+        }
+        if (b < ab) {
+            bad_row = std::max(bad_row, q[5]);
+            longest = std::max(longest, q[6]);
+            high |= q[7];
+        }
+    }
+    if (bad_row) {
+        char b[100];
+        std::snprintf(b, sizeof b, "row_ptr decreases at row %llu", ~bad_row);
+        ctx->err = b;
+        return fail(SS_ERR_INVALID);
+    }
+    if (bad_col) {
+        char b[200];
+        std::snprintf(b, sizeof b, "col_idx[%llu] = %d outside [0, %lld)", ~bad_col, sp->col_idx[~bad_col],
+                      (long long)nt);
+        ctx->err = b;
+        return fail(SS_ERR_RANGE);
+    }
+    const int64_t max_deg = r.max_deg = (int64_t)longest;
+    if (high) {
+        R_HIP(dalloc(ctx, &r, &r.rng_hi, (size_t)nl));
+        R_HIP(ss_launch_high_words(d_ids, nl, r.rng_hi, ctx->stream));
+    }
     // the push direction needs every entry's mirror (a neighbour's row then
     // lists the agent) and no ghosts (ghost rows are empty)
-    r.symmetric = nnz == 0;
-    if (nnz > 0) {
-        unsigned long long h[4] = {0, 0, 0, 0};
-        R_HIP(hipMemcpy(ctx->d_stats, h, sizeof h, hipMemcpyHostToDevice));
-        R_HIP(ss_launch_symcheck(r.row_ptr, r.col_idx, nl, ctx->d_stats, ctx->num_cus * 8, ctx->stream));
-        R_HIP(hipStreamSynchronize(ctx->stream));
-        R_HIP(hipMemcpy(h, ctx->d_stats, sizeof h, hipMemcpyDeviceToHost));
-        r.symmetric = h[0] == h[2] && h[1] == h[3];
-        r.csr_hash[0] = h[0];
-        r.csr_hash[1] = h[1];
-    }
+    r.symmetric = h[0] == h[2] && h[1] == h[3];
+    r.csr_hash[0] = h[0];
+    r.csr_hash[1] = h[1];
+    r.key_hash = keys.get();
     if (sp->history)
         R_HIP(ss_copy_in(ctx, r.init_history, sp->history, sizeof(int32_t) * (size_t)nl * SS_HISTORY_WIDTH));
     r.dev = ss_rep_dev{};
@@ -826,8 +854,8 @@ int ss_replica_set_order(ss_ctx *ctx, int32_t rep, const int32_t *slot, int64_t 
     SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
     if (!r.order) SS_HIP(ctx, dalloc(ctx, &r, &r.order, (size_t)pad_agents(n)));
     unsigned long long bad = ~0ull;
+    SS_HIP(ctx, hipMemsetAsync(ctx->d_stats, 0xFF, sizeof bad, ctx->stream));
     SS_HIP(ctx, ss_copy_in(ctx, r.order, slot, sizeof(int32_t) * (size_t)n));
-    SS_HIP(ctx, hipMemcpy(ctx->d_stats, &bad, sizeof bad, hipMemcpyHostToDevice));
     SS_HIP(ctx, ss_launch_check_cols(r.order, n, n, ctx->d_stats, ctx->num_cus * 8, ctx->stream));
     SS_HIP(ctx, hipMemcpyAsync(&bad, ctx->d_stats, sizeof bad, hipMemcpyDeviceToHost, ctx->stream));
     SS_HIP(ctx, hipStreamSynchronize(ctx->stream));

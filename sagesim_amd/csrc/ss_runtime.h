@@ -103,9 +103,18 @@ hipError_t ss_launch_dec_demote(uint32_t *dec, hipStream_t s);
 // direction statistics of the state buffer st into statistics slot `slot` (zeroed first by the caller)
 hipError_t ss_launch_acc_init(const int8_t *st, const int64_t *row_ptr, int64_t n_local, int8_t s_code, int8_t inf_code,
                               unsigned long long *acc, int slot, int grid, hipStream_t s);
-// sums of two 64-bit hashes of every entry (i, j) and of its mirror (j, i): out[0..1] and out[2..3]
-hipError_t ss_launch_symcheck(const int64_t *row_ptr, const int32_t *col_idx, int64_t n_rows,
-                              unsigned long long *out, int grid, hipStream_t s);
+// Rows of part (SS_STATS_ROW words, one a block): words 0 .. 3, the sums of two
+// 64-bit hashes of every entry (i, j) and of its mirror (j, i); 4: ~(first entry
+// outside [0, n_total)), 0 if none.  Rows that do not ascend are safe, their sums mean nothing
+hipError_t ss_launch_entries(const int64_t *row_ptr, const int32_t *col_idx, int64_t n_rows, int64_t nnz,
+                             int64_t n_total, unsigned long long *part, int max_blocks, int *blocks, hipStream_t s);
+// Degrees in a byte, low words of the key ids, entries before agents 0, 64, ...,
+// row_ptr of the ghosts' empty rows; words 5 of part: ~(first row of negative
+// length), 0 if none; 6: the longest row; 7: the high words or'ed
+hipError_t ss_launch_agents(int64_t *row_ptr, const int64_t *ids, int64_t n, int64_t n_total, int64_t nnz,
+                            uint8_t *deg8, uint32_t *lo, int64_t *edge64, unsigned long long *part, int max_blocks,
+                            int *blocks, hipStream_t s);
+hipError_t ss_launch_high_words(const int64_t *ids, int64_t n, uint32_t *hi, hipStream_t s);
 
 // Frees the device resources of every program of a context that is going
 // (rtc.hip); the programs themselves stay until ss_prog_destroy.
