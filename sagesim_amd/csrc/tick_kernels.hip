@@ -554,15 +554,29 @@ __device__ __forceinline__ void put_bits(SS_G uint64_t *nb, int64_t word, uint64
 // full wavefronts whatever the mix of states; the rows that must be scanned
 // are packed again (in place) and scanned one per lane, long rows by the
 // whole wavefront.  Results return through a byte per chunk slot.
+// Bound where few agents scan by the vector units (busy 50 to 56 % of the time,
+// 1340 instructions a chunk of which 250 agents draw) and by memory (147 MB a
+// tick of 10M agents, the rows' lines most of it), at an epidemic's peak by the
+// gathers' trips to L2.  Hence states as bit planes (nine instructions for 16
+// bytes) instead of compares, queueing without branches where many draw and
+// agent by agent where few do (push), states and counts read again where they
+// are drawn for rather than carried.  Ticks before and after: BA(10M, 5) 200
+// 8.73 and 8.19 ms, 48 scenarios (18M agents) 100 12.35 and 11.65, BA(1M, 5) 200
+// 2.61 and 2.44, WS(100k, 10) SEIR 100 1.26 and 1.20, G(10k) 100 0.965 and 0.945.
+// No gain: a fifth block on each CU (30 KB of LDS, 96 registers), the next
+// tile's first loads ahead of time, tags looked at by each wavefront, draws
+// straight from registers in chunks where most agents draw.
 #define SS_WIDE_A 16
 #define SS_WIDE_CHUNK (64 * SS_WIDE_A)
 #define SS_WIDE_SHORT 512        // rows longer than this are scanned by the whole wavefront
 struct alignas(16) WideQueue {
-    // draw entry: x = RNG key (pull) or infectious-neighbour count (push);
-    //   y = slot | transition << 10 | (state & 3) << 11 | deg8 << 16 (deg8 only on pull)
-    // scan entry: x = draw; y = slot | history-only << 10 | deg8 << 16
-    uint2 e[SS_BLOCK / 64][SS_WIDE_CHUNK];
-    uint8_t res[SS_BLOCK / 64][SS_WIDE_CHUNK];   // next state by chunk slot (queued agents only)
+    struct Part {                                // one wavefront's
+        // draw entry: x = RNG key, y = slot | deg8 << 16; on push only y = slot
+        // scan entry: x = draw; y = slot | history-only << 10 | deg8 << 16
+        // the last 64 of each take what is not queued
+        uint32_t x[SS_WIDE_CHUNK + 64], y[SS_WIDE_CHUNK + 64];
+        uint8_t st[SS_WIDE_CHUNK];               // state by chunk slot, then next state
+    } part[SS_BLOCK / 64];
 };
 
 // 0xFF in byte b of the result for every set bit b of n (n < 16).
@@ -586,6 +600,37 @@ __device__ __forceinline__ int64_t deg_of(const TickView &V, int64_t i, uint32_t
     return d8 == 255u ? V.row_ptr[i + 1] - V.row_ptr[i] : (int64_t)d8;
 }
 
+// Bits set in B below this lane's.
+__device__ __forceinline__ uint32_t rank_in(uint64_t B) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(B >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)B, 0u));
+}
+
+// Bit j set where byte j of the sixteen in v has a bit of the one-bit mask
+// whose copies fill m: the bytes' weights 1, 2, 4, ... are summed four at a time.
+__device__ __forceinline__ uint32_t plane16(const uint4 v, uint32_t m, int shift) {
+    const uint32_t lo = __builtin_amdgcn_udot4(
+        v.y & m, 0x80402010u, __builtin_amdgcn_udot4(v.x & m, 0x08040201u, 0u, false), false);
+    const uint32_t hi = __builtin_amdgcn_udot4(
+        v.w & m, 0x80402010u, __builtin_amdgcn_udot4(v.z & m, 0x08040201u, 0u, false), false);
+    return (lo | hi << 8) >> shift;
+}
+
+// The sixteen bytes' codes 0..3 as two bit planes, and which bytes are codes.
+struct Codes {
+    uint32_t b0, b1, ok;
+    __device__ __forceinline__ explicit Codes(const uint4 v)
+        : b0(plane16(v, 0x01010101u, 0)), b1(plane16(v, 0x02020202u, 1)), ok(0xFFFFu) {
+        const uint32_t f = 0xFCFCFCFCu;
+        if (__ballot(((v.x | v.y | v.z | v.w) & f) != 0u))        // wave-uniform, other values than codes
+            ok = eq_bytes4(v.x & f, 0u) | eq_bytes4(v.y & f, 0u) << 4 | eq_bytes4(v.z & f, 0u) << 8 |
+                 eq_bytes4(v.w & f, 0u) << 12;
+    }
+    // bit j set where byte j is c (0..3)
+    __device__ __forceinline__ uint32_t is(uint32_t c) const {
+        return (b0 ^ ((c & 1u) - 1u)) & (b1 ^ ((c >> 1 & 1u) - 1u)) & ok;
+    }
+};
+
 template <bool HALO>
 __device__ __forceinline__ void light_wide(const TickView V, const LCold *C, int64_t begin, int64_t end, Work &w,
                                            Dir &dir, WideQueue &Q) {
@@ -598,9 +643,7 @@ __device__ __forceinline__ void light_wide(const TickView V, const LCold *C, int
     const int64_t c0 = begin + (int64_t)wv * chunk;
     if (c0 >= end) return;                                        // wave-uniform: no block barrier below
     if (end > c0 + chunk) end = c0 + chunk;
-    uint2 *const E = Q.e[wv];
-    uint8_t *const res = Q.res[wv];
-    const uint64_t below = (1ull << lane) - 1ull;
+    WideQueue::Part &E = Q.part[wv];
     const int64_t i0 = c0 + 16 * lane;
     const int nv = (int)(end - i0 < 0 ? 0 : end - i0 > 16 ? 16 : end - i0);           // agents of the lane
     const int nl = (int)(V.n_local - i0 < 0 ? 0 : V.n_local - i0 > nv ? nv : V.n_local - i0);   // local rows
@@ -611,19 +654,26 @@ __device__ __forceinline__ void light_wide(const TickView V, const LCold *C, int
     uint4 sv = make_uint4(0u, 0u, 0u, 0u);
     if (nv > 0) sv = ld4(V.cur + i0);
     uint32_t a[16];
-    uint32_t dg[4];
+    uint32_t dg[4], hot[2] = {0u, 0u};               // pull: degrees; push: whether the lane's counts 0-7, 8-15 are not all 0
+    uint32_t cmask = 0u;                             // candidates: with neighbours, or with counts
 #pragma unroll
     for (int q = 0; q < 16; ++q) a[q] = 0u;
 #pragma unroll
     for (int q = 0; q < 4; ++q) dg[q] = 0u;
     if (nl > 0) {
         if (!pull) {
+            typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+            const u16x2 one = {1, 1};
+            const uint4 x = ld4(V.cnt + i0), y = ld4(V.cnt + i0 + 8);
+            const uint32_t wd[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+            hot[0] = wd[0] | wd[1] | wd[2] | wd[3];
+            hot[1] = wd[4] | wd[5] | wd[6] | wd[7];
+            if (__ballot((hot[0] | hot[1]) != 0u)) {
+                uint32_t acc = 0u;                   // count 2h: bit 2h, count 2h + 1: bit 16 + 2h
 #pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                const uint4 x = ld4(V.cnt + i0 + 8 * q);
-                const uint32_t wd[4] = {x.x, x.y, x.z, x.w};
-#pragma unroll
-                for (int h = 0; h < 8; ++h) a[8 * q + h] = (wd[h >> 1] >> (16 * (h & 1))) & 0xFFFFu;
+                for (int h = 0; h < 8; ++h)
+                    acc |= __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, wd[h]), one)) << (2 * h);
+                cmask = (acc & 0x5555u) | ((acc >> 15) & 0xAAAAu);
             }
         } else {
 #pragma unroll
@@ -635,16 +685,11 @@ __device__ __forceinline__ void light_wide(const TickView V, const LCold *C, int
                 const uint4 x = ld4(V.deg8 + i0);
                 dg[0] = x.x; dg[1] = x.y; dg[2] = x.z; dg[3] = x.w;
             }
-        }
-    }
-    if (!pull && nl > 0) {
-        // counts are cleared as they are read, ready for the tick after next
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            uint32_t any = 0u;
-#pragma unroll
-            for (int h = 0; h < 8; ++h) any |= a[8 * q + h];
-            if (any != 0u) st4(V.cnt + i0 + 8 * q, make_uint4(0u, 0u, 0u, (uint32_t)opaque(0)));
+            for (int q = 0; q < 4; ++q) {
+                const uint32_t z = ((((dg[q] & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | dg[q]) >> 7) & 0x01010101u;
+                cmask |= __builtin_amdgcn_udot4(z, 0x08040201u, 0u, false) << (4 * q);
+            }
         }
     }
     // A chunk whose rows all have du entries (most are: rows are sorted by
@@ -660,97 +705,97 @@ __device__ __forceinline__ void light_wide(const TickView V, const LCold *C, int
         for (int q = 0; q < 4; ++q) off |= (dg[q] ^ D) & (nl == 16 ? ~0u : byte_mask4((lmask >> (4 * q)) & 15u));
         if (du != 255u && !__ballot(off != 0u)) row0 = V.row_ptr[c0];
     }
-    // states with a spontaneous transition, as a bit set over state codes 0..3
-    uint32_t tbits = 0u;
+    // susceptible agents, and agents in a state with a spontaneous transition
+    const Codes now(sv);
+    const uint32_t smask = now.is((uint32_t)(uint8_t)V.s_code) & lmask;
+    uint32_t tmask = 0u;
 #pragma unroll
-    for (int s = 0; s < 4; ++s) tbits |= (C->tT[s] != 0u ? 1u : 0u) << s;
-    uint32_t smask = 0u, tmask = 0u, cmask = 0u;     // susceptible, transition, candidate
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-        const uint32_t s = (u4_word(sv, j >> 2) >> (8 * (j & 3))) & 0xFFu;
-        const bool is_s = (int8_t)s == V.s_code;
-        smask |= (is_s ? 1u : 0u) << j;
-        tmask |= (!is_s && s < 4u && ((tbits >> s) & 1u) ? 1u : 0u) << j;
-        const uint32_t nz = pull ? ((dg[j >> 2] >> (8 * (j & 3))) & 0xFFu) : a[j];
-        cmask |= (nz != 0u ? 1u : 0u) << j;
-    }
-    smask &= lmask;
-    tmask &= lmask;
+    for (uint32_t c = 0; c < 4; ++c)
+        if (__builtin_amdgcn_readfirstlane((int)C->tT[c]) != 0) tmask |= now.is(c);
+    tmask &= lmask & ~smask;
     const uint32_t enq = (smask & cmask) | tmask;
     w.s_agents += (uint32_t)__popc(smask);
     // the lane's queue position: exclusive prefix over lanes of popc(enq) (<= 16)
     const uint32_t ne = (uint32_t)__popc(enq);
     uint32_t pos = 0u, nq = 0u;
+    if (__ballot(ne != 0u)) {
 #pragma unroll
-    for (int b = 0; b < 5; ++b) {
-        const uint64_t B = __ballot((ne >> b) & 1u);
-        pos += (uint32_t)__popcll(B & below) << b;
-        nq += (uint32_t)__popcll(B) << b;
-    }
-    if (enq) {
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            if ((enq >> j) & 1u) {
-                const uint32_t s = (u4_word(sv, j >> 2) >> (8 * (j & 3))) & 3u;
-                const uint32_t d = pull ? ((dg[j >> 2] >> (8 * (j & 3))) & 0xFFu) : 0u;
-                E[pos] = make_uint2(a[j], (uint32_t)(16 * lane + j) | ((tmask >> j) & 1u) << 10 | s << 11 | d << 16);
-                ++pos;
-            }
+        for (int b = 0; b < 5; ++b) {
+            const uint64_t B = __ballot((ne >> b) & 1u);
+            pos += rank_in(B) << b;
+            nq += (uint32_t)__popcll(B) << b;
         }
     }
-    bool busy = false;                               // the tile must run next tick
+    bool busy = tmask != 0u;                         // the tile must run next tick
     uint32_t nsq = 0u;                               // wave-uniform scan-queue length
     if (nq > 0u) {                                   // wave-uniform
+        *(uint4 *)(E.st + 16 * lane) = sv;
+        if (pull) {
+            // many draw: without branches, an agent that is not queued goes past the end
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                const uint32_t bit = (enq >> j) & 1u;
+                const uint32_t at = bit != 0u ? pos : (uint32_t)(SS_WIDE_CHUNK + lane);
+                E.x[at] = a[j];
+                E.y[at] = (uint32_t)(16 * lane + j) | ((dg[j >> 2] >> (8 * (j & 3))) & 0xFFu) << 16;
+                pos += bit;
+            }
+        } else {
+            // few do: one after another
+            for (uint32_t rest = enq; rest != 0u; rest &= rest - 1u)
+                E.y[pos++] = (uint32_t)(16 * lane + __ffs(rest) - 1);
+        }
         wave_sync();
         // draws, a full wavefront of queued agents per round; the rows to scan
         // are packed over the entries already read
+        const SS_L uint32_t *const lim = (const SS_L uint32_t *)C;   // T, then tT
         for (uint32_t r0 = 0; r0 < nq; r0 += 64) {
             const uint32_t q = r0 + (uint32_t)lane;
             bool sc = false;
-            uint2 se = make_uint2(0u, 0u);
+            uint32_t m = 0u, y = 0u;
             if (q < nq) {
-                const uint2 en = E[q];
-                const uint32_t slot = en.y & 1023u;
-                const bool trans = ((en.y >> 10) & 1u) != 0u;
+                y = E.y[q];
+                const uint32_t slot = y & 1023u;
                 const int64_t i = c0 + slot;
-                const uint32_t key = pull ? en.x : V.rng_lo[i];
+                const uint32_t s = E.st[slot];
+                const bool trans = (int8_t)s != V.s_code;
+                const uint32_t key = pull ? E.x[q] : V.rng_lo[i];
+                const uint32_t k0 = pull ? y >> 16 : (uint32_t)V.cnt[i];
                 const uint32_t khi = V.rng_hi ? V.rng_hi[i] : 0u;
                 ++w.draws;
-                const uint32_t m = draw_key(V, key, khi);
-                int8_t s, ns;
-                if (trans) {
-                    s = (int8_t)((en.y >> 11) & 3u);
-                    ns = m < C->tT[s] ? trans_next(C, s) : s;
-                } else {
-                    s = ns = V.s_code;
-                    if (!pull) {
-                        if (m < thr(V, C, (int64_t)en.x)) {
-                            ns = V.s_target;
-                            if (C->history) {
-                                // the history's first infectious neighbour (draw 0 stops the scan there)
-                                sc = true;
-                                se = make_uint2(0u, slot | 1u << 10 | (uint32_t)V.deg8[i] << 16);
-                            }
-                        }
+                m = draw_key(V, key, khi);
+                // pull: the bound of all neighbours; a capped degree (255) bounds with the last table entry
+                const uint32_t last = (uint32_t)V.last;
+                const uint32_t kk = k0 > last || (pull && k0 == 255u) ? last : k0;
+                uint32_t t = lim[trans ? SS_TLDS + s : kk < SS_TLDS ? kk : 0u];
+                if (!trans && kk >= SS_TLDS) t = ((const SS_G uint32_t *)C->inf_T)[kk];
+                if (m < t) {
+                    if (!trans && pull) {
+                        sc = true;
+                        ++w.scans;
                     } else {
-                        const uint32_t d = en.y >> 16;
-                        // a capped degree (255) bounds with the last table entry
-                        if (m < thr(V, C, d == 255u ? (int64_t)V.last : (int64_t)d)) {
+                        const int8_t ns = trans ? trans_next(C, (int8_t)s) : V.s_target;
+                        dir_change(dir, V, (int8_t)s, ns, deg_of(V, i, pull ? y >> 16 : (uint32_t)V.deg8[i]));
+                        E.st[slot] = (uint8_t)ns;
+                        busy = true;
+                        if (!trans && C->history) {
+                            // the history's first infectious neighbour (draw 0 stops the scan there)
                             sc = true;
-                            se = make_uint2(m, slot | d << 16);
-                            ++w.scans;
+                            m = 0u;
+                            y = slot | 1u << 10 | (uint32_t)V.deg8[i] << 16;
                         }
                     }
                 }
-                if (ns != s)
-                    dir_change(dir, V, s, ns, deg_of(V, i, pull ? en.y >> 16 : (uint32_t)V.deg8[i]));
-                busy |= ns != s || ns == V.inf_code || trans_thr(C, ns) != 0u;
-                res[slot] = (uint8_t)ns;
             }
             const uint64_t sm = __ballot(sc);
-            if (sc) E[nsq + (uint32_t)__popcll(sm & below)] = se;
+            if (sc) {
+                const uint32_t at = nsq + rank_in(sm);
+                E.x[at] = m;
+                E.y[at] = y;
+            }
             nsq += (uint32_t)__popcll(sm);
         }
+        busy |= V.inf_code == V.s_code && enq != 0u;
     }
     if (nsq > 0u) {                                  // wave-uniform
         wave_sync();
@@ -760,9 +805,8 @@ __device__ __forceinline__ void light_wide(const TickView V, const LCold *C, int
             int64_t b = 0, e = 0;
             uint32_t m = 0u, y = 0u;
             if (q < nsq) {
-                const uint2 en = E[q];
-                m = en.x;
-                y = en.y;
+                m = E.x[q];
+                y = E.y[q];
                 const int64_t i = c0 + (y & 1023u);
                 const uint32_t d = y >> 16;
                 b = row0 >= 0 ? row0 + (int64_t)((y & 1023u) * du) : V.row_ptr[i];
@@ -777,7 +821,7 @@ __device__ __forceinline__ void light_wide(const TickView V, const LCold *C, int
                 const uint32_t slot = y & 1023u;
                 const int64_t i = c0 + slot;
                 if (((y >> 10) & 1u) == 0u) {
-                    res[slot] = (uint8_t)V.s_target;
+                    E.st[slot] = (uint8_t)V.s_target;
                     dir_change(dir, V, V.s_code, V.s_target, e - b);
                     busy = true;
                 }
@@ -785,19 +829,15 @@ __device__ __forceinline__ void light_wide(const TickView V, const LCold *C, int
             }
         }
     }
-    // next states: the queued agents' from LDS, the others unchanged
+    // counts are cleared once read, ready for the tick after next
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+        if (hot[q] != 0u) st4(V.cnt + i0 + 8 * q, make_uint4(0u, 0u, 0u, (uint32_t)opaque(0)));
+    // next states
     uint4 nsv = sv;
     if (nq > 0u) {
         wave_sync();
-        if (enq) {
-            const uint4 r = *(const uint4 *)(res + 16 * lane);
-            const uint32_t m0 = byte_mask4(enq & 15u), m1 = byte_mask4((enq >> 4) & 15u);
-            const uint32_t m2 = byte_mask4((enq >> 8) & 15u), m3 = byte_mask4(enq >> 12);
-            nsv.x = (r.x & m0) | (sv.x & ~m0);
-            nsv.y = (r.y & m1) | (sv.y & ~m1);
-            nsv.z = (r.z & m2) | (sv.z & ~m2);
-            nsv.w = (r.w & m3) | (sv.w & ~m3);
-        }
+        nsv = *(const uint4 *)(E.st + 16 * lane);
     }
     // fused halo refresh: the lane's ghost slots take the next step's halo
     // (what the refresh kernel would write before that step); a lane with
@@ -838,9 +878,7 @@ __device__ __forceinline__ void light_wide(const TickView V, const LCold *C, int
     // infectious bits of the lane's agents; lanes 4g .. 4g+3 fill bitmap word g
     // of a chunk of whole words, otherwise each lane sets and clears its own 16
     // bits of a word it shares (chunk is wave-uniform)
-    const uint32_t X = 0x01010101u * (uint32_t)(uint8_t)V.inf_code;
-    const uint32_t ib = (eq_bytes4(nsv.x, X) | eq_bytes4(nsv.y, X) << 4 | eq_bytes4(nsv.z, X) << 8 |
-                         eq_bytes4(nsv.w, X) << 12) & vmask;
+    const uint32_t ib = Codes(nsv).is((uint32_t)(uint8_t)V.inf_code) & vmask;
     if (chunk & 63) {
         if (nv > 0) {
             const int sh = (int)(i0 & 63);
@@ -874,16 +912,18 @@ __device__ __forceinline__ void light_wide(const TickView V, const LCold *C, int
         // of BA(1M, 5) 2.89 -> 2.77.
         const uint32_t np1 = (uint32_t)__popc(pend);
         uint32_t pp = 0u, np = 0u;
+        if (__ballot(np1 != 0u)) {
 #pragma unroll
-        for (int b = 0; b < 5; ++b) {
-            const uint64_t B = __ballot((np1 >> b) & 1u);
-            pp += (uint32_t)__popcll(B & below) << b;
-            np += (uint32_t)__popcll(B) << b;
+            for (int b = 0; b < 5; ++b) {
+                const uint64_t B = __ballot((np1 >> b) & 1u);
+                pp += rank_in(B) << b;
+                np += (uint32_t)__popcll(B) << b;
+            }
         }
         if (np > 0u) {                               // wave-uniform
             wave_sync();
             while (pend != 0u) {
-                E[pp++].x = (uint32_t)(16 * lane + __ffs(pend) - 1);
+                E.x[pp++] = (uint32_t)(16 * lane + __ffs(pend) - 1);
                 pend &= pend - 1u;
             }
             wave_sync();
@@ -891,7 +931,7 @@ __device__ __forceinline__ void light_wide(const TickView V, const LCold *C, int
             for (uint32_t r0 = 0; r0 < np; r0 += 64) {
                 int64_t b = 0, e = 0;
                 if (r0 + lane < np) {
-                    const int64_t i = c0 + E[r0 + lane].x;
+                    const int64_t i = c0 + E.x[r0 + lane];
                     b = V.row_ptr[i];
                     e = V.row_ptr[i + 1];
                     w.pushed += (uint32_t)(e - b);
