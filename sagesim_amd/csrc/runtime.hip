@@ -190,25 +190,36 @@ int64_t heavy_prefix(const ss_replica &r, int32_t thr) {
     return -1;
 }
 
-// Direction state of the replica's current tick t: statistics of t in slot
-// t % 3 (the other slots cleared), the push decision for t and, when it
-// pushes, the infectious-neighbour counts of t from the infectious bitmap.
-int init_acc(ss_ctx *ctx, ss_replica &r) {
-    SS_HIP(ctx, hipMemsetAsync(r.acc, 0, sizeof(unsigned long long) * SS_ACC_WORDS, ctx->stream));
-    const int slot = (int)((uint64_t)r.tick % 3u);
-    SS_HIP(ctx, ss_launch_acc_init(r.state[r.tick & 1], r.row_ptr, r.n_local, r.dev.s_code, r.dev.inf_code, r.acc,
-                                   slot, ctx->num_cus * 8, ctx->stream));
-    if (r.cnt[0]) {
-        const int par = (int)(r.tick & 1);
-        const uint32_t num = r.dev.push_ok ? ctx->push_num : 0u;
-        for (int b = 0; b < 2; ++b)
-            SS_HIP(ctx, hipMemsetAsync(r.cnt[b], 0, sizeof(uint16_t) * (size_t)pad_agents(r.n_local), ctx->stream));
-        SS_HIP(ctx, ss_launch_count_init(r.row_ptr, r.col_idx, r.ibits[par], r.n_local, heavy_prefix(r, 64),
-                                         r.cnt[par], r.dec + par, r.acc + slot * (SS_ACC_SLOTS * 2), num,
-                                         ctx->num_cus * 8, ctx->stream));
-    }
+// Direction state of the replica's current tick t from the states src: statistics
+// of t in slot t % 3 (the other slots cleared), the push decision for t and,
+// when it pushes, the infectious-neighbour counts of t; and, where asked for,
+// copies of the states and both bitmaps.
+int begin_tick(ss_ctx *ctx, ss_replica &r, const int8_t *src, int8_t *dst0 = nullptr, int8_t *dst1 = nullptr,
+               uint64_t *bits0 = nullptr, uint64_t *bits1 = nullptr) {
+    const int par = (int)(r.tick & 1);
+    ss_begin q{};
+    q.row_ptr = r.row_ptr;
+    q.col_idx = r.col_idx;
+    q.deg8 = r.deg8;
+    q.bits = r.ibits[par];
+    q.cnt[0] = r.cnt[0];
+    q.cnt[1] = r.cnt[1];
+    q.cnt_now = r.cnt[par];
+    q.dec = r.dec ? r.dec + par : nullptr;
+    q.acc = r.acc;
+    q.part = ctx->d_part;
+    q.n_local = r.n_local;
+    q.n_total = r.n_total;
+    q.heavy = r.cnt[0] ? heavy_prefix(r, 64) : 0;
+    q.slot = (int32_t)((uint64_t)r.tick % 3u);
+    q.push_num = r.dev.push_ok ? ctx->push_num : 0u;
+    q.s_code = r.dev.s_code;
+    q.inf_code = r.dev.inf_code;
+    SS_HIP(ctx, ss_launch_begin(src, dst0, dst1, bits0, bits1, q, ctx->num_cus, ctx->stream));
     return SS_OK;
 }
+
+int init_acc(ss_ctx *ctx, ss_replica &r) { return begin_tick(ctx, r, r.state[r.tick & 1]); }
 
 void drop_graphs(ss_ctx *ctx) {
     for (auto &kv : ctx->graphs) (void)hipGraphExecDestroy(kv.second);
@@ -487,6 +498,7 @@ int ss_create(int device, ss_ctx **out) {
         (e = hipMalloc((void **)&ctx->d_work, SS_WORK_N * sizeof(unsigned long long))) != hipSuccess ||
         (e = hipMalloc((void **)&ctx->d_stats, 8 * sizeof(unsigned long long))) != hipSuccess ||
         (e = hipMemset(ctx->d_work, 0, SS_WORK_N * sizeof(unsigned long long))) != hipSuccess ||
+        (e = hipMalloc((void **)&ctx->d_part, 2 * sizeof(unsigned long long) * SS_BEGIN_PARTS(prop.multiProcessorCount))) != hipSuccess ||
         (e = hipMalloc((void **)&ctx->d_counters, 64 * sizeof(int32_t))) != hipSuccess ||
         (e = hipHostMalloc((void **)&ctx->h_stats,
                            sizeof(unsigned long long) * SS_STATS_ROW * 4 * prop.multiProcessorCount,
@@ -517,6 +529,7 @@ int ss_destroy(ss_ctx *ctx) {
     dfree(ctx->d_counters);
     dfree(ctx->d_work);
     dfree(ctx->d_stats);
+    dfree(ctx->d_part);
     dfree(ctx->scratch);
     if (ctx->t_start) (void)hipEventDestroy(ctx->t_start);
     if (ctx->t_stop) (void)hipEventDestroy(ctx->t_stop);
@@ -556,7 +569,7 @@ int ss_device_info(ss_ctx *ctx, int32_t *num_cus, int64_t *total_mem, int64_t *c
 int64_t ss_replica_footprint(int64_t n_local, int64_t n_ghost, int64_t nnz, int32_t with_history, int64_t max_deg) {
     int64_t n_total = n_local + n_ghost;
     int64_t words = (n_total + 63) / 64;
-    int64_t b = 8 * (n_total + 1) + 4 * (nnz + SS_COL_PAD) + 6 * pad_agents(n_local) + 2 * pad_agents(n_total) + n_total +
+    int64_t b = 8 * (n_total + 1) + 4 * (nnz + SS_COL_PAD) + 6 * pad_agents(n_local) + 3 * pad_agents(n_total) +
                 2 * 8 * words + 4 * (std::min<int64_t>(max_deg, 1 << 24) + 1) + 8 * SS_ACC_WORDS +
                 (n_ghost == 0 ? 4 * pad_agents(n_local) + 8 : 0);
     if (with_history) b += 2 * 4 * n_local * SS_HISTORY_WIDTH;
@@ -651,7 +664,7 @@ int ss_replica_create(ss_ctx *ctx, const ss_replica_spec *sp, int32_t *rep_out) 
         R_HIP(dalloc(ctx, &r, &r.state[b], (size_t)pad_agents(nt)));
         R_HIP(dalloc(ctx, &r, &r.ibits[b], (size_t)r.n_words));
     }
-    R_HIP(dalloc(ctx, &r, &r.init_state, (size_t)nt));
+    R_HIP(dalloc(ctx, &r, &r.init_state, (size_t)pad_agents(nt)));
     R_HIP(dalloc(ctx, &r, &r.acc, (size_t)SS_ACC_WORDS));
     if (ng == 0 && nl > 0) {
         R_HIP(dalloc(ctx, &r, &r.cnt[0], (size_t)pad_agents(nl)));
@@ -778,18 +791,10 @@ int ss_replica_reset(ss_ctx *ctx, int32_t rep) {
     if (!valid_rep(ctx, rep)) SS_FAIL(ctx, SS_ERR_INVALID, "no live replica %d", rep);
     ss_replica &r = ctx->reps[rep];
     r.tick = r.tick_init;
-    const int par = (int)(r.tick & 1);
-    if (r.n_total) {
-        SS_HIP(ctx, hipMemcpyAsync(r.state[par], r.init_state, (size_t)r.n_total, hipMemcpyDeviceToDevice, ctx->stream));
-        SS_HIP(ctx, hipMemcpyAsync(r.state[par ^ 1], r.init_state, (size_t)r.n_total, hipMemcpyDeviceToDevice, ctx->stream));
-    }
     if (r.history)
         SS_HIP(ctx, hipMemcpyAsync(r.history, r.init_history, sizeof(int32_t) * r.n_local * SS_HISTORY_WIDTH,
                                    hipMemcpyDeviceToDevice, ctx->stream));
-    int rc = rebuild_bits(ctx, r, par, 0, r.n_words);
-    if (rc) return rc;
-    if ((rc = rebuild_bits(ctx, r, par ^ 1, 0, r.n_words))) return rc;
-    return init_acc(ctx, r);
+    return begin_tick(ctx, r, r.init_state, r.state[0], r.state[1], r.ibits[0], r.ibits[1]);
 }
 
 int ss_replica_tick(ss_ctx *ctx, int32_t rep, int64_t *tick) {
@@ -802,15 +807,12 @@ int ss_replica_set_tick(ss_ctx *ctx, int32_t rep, int64_t tick, int64_t tick_lim
     if (!valid_rep(ctx, rep) || tick < 0) SS_FAIL(ctx, SS_ERR_INVALID, "bad replica or tick");
     ss_replica &r = ctx->reps[rep];
     SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    if ((tick & 1) != (r.tick & 1) && r.n_total) {
-        // keep "tick t reads state[t & 1]": move the live buffer
-        const int from = (int)(r.tick & 1);
-        SS_HIP(ctx, hipMemcpyAsync(r.state[from ^ 1], r.state[from], (size_t)r.n_total, hipMemcpyDeviceToDevice, ctx->stream));
-        int rc = rebuild_bits(ctx, r, from ^ 1, 0, r.n_words);
-        if (rc) return rc;
-    }
+    const int from = (int)(r.tick & 1);
     r.tick = tick;
     r.tick_limit = tick_limit > 0 ? tick_limit : INT64_MAX;
+    // keep "tick t reads state[t & 1]": move the live buffer
+    if ((tick & 1) != from)
+        return begin_tick(ctx, r, r.state[from], r.state[from ^ 1], nullptr, r.ibits[from ^ 1]);
     return init_acc(ctx, r);
 }
 
@@ -827,8 +829,7 @@ int ss_set_model(ss_ctx *ctx, int32_t rep, const ss_model *m) {
     int rc = apply_model(ctx, r, m);
     if (rc) return rc;
     const int par = (int)(r.tick & 1);
-    if ((rc = rebuild_bits(ctx, r, par, 0, r.n_words))) return rc;
-    return init_acc(ctx, r);
+    return begin_tick(ctx, r, r.state[par], nullptr, nullptr, r.ibits[par]);
 }
 
 int ss_set_seed(ss_ctx *ctx, int32_t rep, uint64_t seed) {
@@ -898,14 +899,8 @@ int ss_state_upload(ss_ctx *ctx, int32_t rep, const int8_t *in, int64_t n) {
     if (n != r.n_total) SS_FAIL(ctx, SS_ERR_INVALID, "n = %lld, replica has %lld slots", (long long)n, (long long)r.n_total);
     SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
     const int par = (int)(r.tick & 1);
-    if (n) {
-        SS_HIP(ctx, ss_copy_in(ctx, r.state[par], in, (size_t)n));
-        SS_HIP(ctx, hipMemcpyAsync(r.state[par ^ 1], r.state[par], (size_t)n, hipMemcpyDeviceToDevice, ctx->stream));
-    }
-    int rc = rebuild_bits(ctx, r, par, 0, r.n_words);
-    if (rc) return rc;
-    if ((rc = rebuild_bits(ctx, r, par ^ 1, 0, r.n_words))) return rc;
-    return init_acc(ctx, r);
+    SS_HIP(ctx, ss_copy_in(ctx, r.state[par], in, (size_t)n));
+    return begin_tick(ctx, r, r.state[par], r.state[par ^ 1], nullptr, r.ibits[0], r.ibits[1]);
 }
 
 int ss_history_download(ss_ctx *ctx, int32_t rep, int32_t *out, int64_t n_rows) {

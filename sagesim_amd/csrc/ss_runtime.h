@@ -93,16 +93,28 @@ hipError_t ss_launch_check_cols(const int32_t *col, int64_t nnz, int64_t n_total
 #define SS_STATS_ROW 8
 hipError_t ss_launch_stats(const int8_t *st, const uint8_t *deg8, const int64_t *row_ptr, int64_t n_local,
                            int8_t s_code, unsigned long long *part, int max_blocks, int *blocks, hipStream_t s);
-// push decision of the current tick from its statistics acc_t, then (when
-// pushing) its infectious-neighbour counts (cleared before) from the bitmap
-hipError_t ss_launch_count_init(const int64_t *row_ptr, const int32_t *col_idx, const uint64_t *bits,
-                                int64_t n_local, int64_t heavy, uint16_t *cnt, uint32_t *dec,
-                                const unsigned long long *acc_t, uint32_t push_num, int grid, hipStream_t s);
+// The start of a replica's current tick from the states src: copies into dst0 and
+// dst1, bitmaps bits0 and bits1 (null: left alone), direction statistics, the
+// push decision and, when it pushes, the infectious-neighbour counts along the
+// rows of the bitmap `bits`.  part: 2 words for each of SS_BEGIN_PARTS blocks
+#define SS_BEGIN_PARTS(num_cus) (4 * (num_cus))
+struct ss_begin {
+    const int64_t *row_ptr;
+    const int32_t *col_idx;
+    const uint8_t *deg8;
+    const uint64_t *bits;                       // this tick's, written before or by bits0 / bits1
+    uint16_t *cnt[2], *cnt_now;                 // null without push arrays
+    uint32_t *dec;                              // this tick's decision
+    unsigned long long *acc, *part;
+    int64_t n_local, n_total, heavy;
+    int32_t slot;                               // statistics slot of this tick
+    uint32_t push_num;                          // 0: pull only
+    int8_t s_code, inf_code;
+};
+hipError_t ss_launch_begin(const int8_t *src, int8_t *dst0, int8_t *dst1, uint64_t *bits0, uint64_t *bits1,
+                           const ss_begin &q, int num_cus, hipStream_t s);
 // a push decision with tile tags (1) becomes "push, every tile runs" (2)
 hipError_t ss_launch_dec_demote(uint32_t *dec, hipStream_t s);
-// direction statistics of the state buffer st into statistics slot `slot` (zeroed first by the caller)
-hipError_t ss_launch_acc_init(const int8_t *st, const int64_t *row_ptr, int64_t n_local, int8_t s_code, int8_t inf_code,
-                              unsigned long long *acc, int slot, int grid, hipStream_t s);
 // Rows of part (SS_STATS_ROW words, one a block): words 0 .. 3, the sums of two
 // 64-bit hashes of every entry (i, j) and of its mirror (j, i); 4: ~(first entry
 // outside [0, n_total)), 0 if none.  Rows that do not ascend are safe, their sums mean nothing
@@ -197,6 +209,7 @@ struct ss_ctx {
     int32_t *d_counters = nullptr;              // misc device counters (misses, overflow)
     unsigned long long *d_work = nullptr;       // [SS_WORK_N] tick-kernel work counters
     unsigned long long *d_stats = nullptr;      // [8] results of the checks at replica creation
+    unsigned long long *d_part = nullptr;       // parts of a tick's start, 2 words a block
     unsigned long long *h_stats = nullptr;      // census rows, page-locked, 4 blocks per CU
     bool counting = false;
     uint32_t push_num = 4;                      // direction rule, 16 * ratio (0: pull only); ratio 0.25

@@ -1350,14 +1350,116 @@ __global__ __launch_bounds__(SS_BLOCK) __attribute__((amdgpu_waves_per_eu(4))) v
     if constexpr (CNT) flush_work(counters, w);
 }
 
-// Infectious-neighbour counts of the current tick of one replica (cleared
-// before), pushed along the rows of its infectious agents, when *dec is set.
-// Rows [0, heavy) (the rows of degree >= 64 of a degree-sorted replica) are
-// walked by a wavefront each, the others by a thread.
-__global__ void count_init_kernel(const int64_t *__restrict__ row_ptr, const int32_t *__restrict__ col,
-                                  const uint64_t *__restrict__ bits, int64_t n_local, int64_t heavy,
-                                  uint16_t *cnt, const uint32_t *dec) {
-    if (*dec == 0u) return;
+// The start of a replica's current tick from a state buffer, a lane 16 agents at
+// a time: the other copies of the states and the bitmaps of both buffers (null:
+// left alone), both count arrays cleared, and each block's part of the direction
+// statistics, part[2 b] the degrees of infectious agents, part[2 b + 1] the
+// susceptible ones.  Bound by its launch below a million agents (one of two,
+// where a reset took ten: resets of 48 replicas 1376 and 369 us, calls included)
+// and by the 9 bytes an agent above.
+__global__ __launch_bounds__(256) void begin_kernel(const SS_G int8_t *src, SS_G int8_t *dst0, SS_G int8_t *dst1,
+                                                    uint64_t *bits0, uint64_t *bits1, SS_G uint16_t *cnt0,
+                                                    SS_G uint16_t *cnt1, const SS_G uint8_t *deg8,
+                                                    const int64_t *row_ptr, int64_t n_local, int64_t n_total,
+                                                    uint32_t s_code, uint32_t inf, unsigned long long *part) {
+    unsigned long long d = 0, c = 0;
+    const int64_t stride = 16 * (int64_t)gridDim.x * blockDim.x;
+    // whole wavefronts: the lanes past the end take part with no agents
+    for (int64_t w0 = 16 * ((int64_t)blockIdx.x * blockDim.x + (threadIdx.x & ~63u)); w0 < n_total; w0 += stride) {
+        const int64_t i0 = w0 + 16 * (threadIdx.x & 63u);
+        const int nv = (int)(n_total - i0 < 0 ? 0 : n_total - i0 > 16 ? 16 : n_total - i0);
+        const int nl = (int)(n_local - i0 < 0 ? 0 : n_local - i0 > nv ? nv : n_local - i0);
+        uint4 sv = make_uint4(0u, 0u, 0u, 0u), dg = sv;
+        if (nv > 0) sv = ld4(src + i0);                  // the arrays are padded to whole groups of 64
+        if (nl > 0) dg = ld4(deg8 + i0);
+        const Codes now(sv);
+        const uint32_t ib = now.is(inf) & ((1u << nv) - 1u), lmask = (1u << nl) - 1u;
+        c += (unsigned long long)__popc(now.is(s_code) & lmask);
+        for (uint32_t rest = ib & lmask; rest != 0u; rest &= rest - 1u) {
+            const int j = __ffs(rest) - 1;
+            const uint32_t w = j & 8 ? (j & 4 ? dg.w : dg.z) : (j & 4 ? dg.y : dg.x);
+            const uint32_t k = (w >> (8 * (j & 3))) & 0xFFu;
+            d += k == 255u ? (unsigned long long)(row_ptr[i0 + j + 1] - row_ptr[i0 + j]) : k;
+        }
+        if (nv > 0) {
+            if (dst0) st4(dst0 + i0, sv);
+            if (dst1) st4(dst1 + i0, sv);
+        }
+        uint32_t lo = (threadIdx.x & 2u) ? 0u : ib << (16 * (threadIdx.x & 1u));
+        uint32_t hi = (threadIdx.x & 2u) ? ib << (16 * (threadIdx.x & 1u)) : 0u;
+        lo |= (uint32_t)__shfl_xor((int32_t)lo, 1);
+        hi |= (uint32_t)__shfl_xor((int32_t)hi, 1);
+        lo |= (uint32_t)__shfl_xor((int32_t)lo, 2);
+        hi |= (uint32_t)__shfl_xor((int32_t)hi, 2);
+        if ((threadIdx.x & 3u) == 0u && nv > 0) {
+            if (bits0) bits0[i0 >> 6] = (uint64_t)hi << 32 | lo;
+            if (bits1) bits1[i0 >> 6] = (uint64_t)hi << 32 | lo;
+        }
+        if (cnt0 && i0 < (n_local + 63) / 64 * 64) {
+            const uint4 z = make_uint4(0u, 0u, 0u, 0u);
+            st4(cnt0 + i0, z); st4(cnt0 + i0 + 8, z);
+            st4(cnt1 + i0, z); st4(cnt1 + i0 + 8, z);
+        }
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        d += __shfl_down(d, off);
+        c += __shfl_down(c, off);
+    }
+    __shared__ unsigned long long red[2 * 256 / 64];
+    const int wv = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) {
+        red[2 * wv] = d;
+        red[2 * wv + 1] = c;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        unsigned long long t = red[threadIdx.x];
+        for (int q = 1; q < 4; ++q) t += red[2 * q + threadIdx.x];
+        part[2 * blockIdx.x + threadIdx.x] = t;
+    }
+}
+
+// From the parts (every block sums them): the statistics of the current tick
+// into slot `slot` (block 0; the other slots cleared), the push decision for it
+// (push when 16 * sum_deg(I) <= push_num * #S), and, when it pushes, its
+// infectious-neighbour counts (cleared before), along the rows of its infectious
+// agents.  Rows [0, heavy) (the rows of degree >= 64 of a degree-sorted replica)
+// are walked by a wavefront each, the others by a thread.
+__global__ __launch_bounds__(256) void count_init_kernel(const unsigned long long *part, int parts,
+                                                         const int64_t *__restrict__ row_ptr,
+                                                         const int32_t *__restrict__ col,
+                                                         const uint64_t *__restrict__ bits, int64_t n_local,
+                                                         int64_t heavy, uint16_t *cnt, uint32_t *dec,
+                                                         unsigned long long *acc, int slot, uint32_t push_num) {
+    unsigned long long d = 0, c = 0;
+    for (int q = threadIdx.x; q < parts; q += 256) {
+        d += part[2 * q];
+        c += part[2 * q + 1];
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        d += __shfl_down(d, off);
+        c += __shfl_down(c, off);
+    }
+    __shared__ unsigned long long red[2 * 256 / 64];
+    if ((threadIdx.x & 63) == 0) {
+        red[2 * (threadIdx.x >> 6)] = d;
+        red[2 * (threadIdx.x >> 6) + 1] = c;
+    }
+    __syncthreads();
+    d = red[0] + red[2] + red[4] + red[6];
+    c = red[1] + red[3] + red[5] + red[7];
+    // the counts of this tick come from here, not from a previous tick's tile tags
+    const bool push = cnt && push_num != 0u && d * 16ull <= (unsigned long long)push_num * c;
+    if (blockIdx.x == 0) {
+        for (int q = threadIdx.x; q < SS_ACC_WORDS; q += 256) {
+            const int w = q - slot * (SS_ACC_SLOTS * 2);
+            acc[q] = w == 0 ? d : w == 1 ? c : 0ull;
+        }
+        if (cnt && threadIdx.x == 0) *dec = push ? 2u : 0u;
+    }
+    if (!push) return;
     const int lane = threadIdx.x & 63;
     const int64_t gt = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, nt = (int64_t)gridDim.x * blockDim.x;
     for (int64_t i = gt >> 6; i < heavy; i += nt >> 6) {
@@ -1372,56 +1474,8 @@ __global__ void count_init_kernel(const int64_t *__restrict__ row_ptr, const int
     }
 }
 
-// The push decision of the current tick t from the statistics of tick t (one
-// thread): push when 16 * sum_deg(I) <= push_num * #S.
-__global__ void dec_init_kernel(const unsigned long long *acc_t, uint32_t push_num, uint32_t *dec) {
-    unsigned long long d = 0, c = 0;
-    for (int q = 0; q < SS_ACC_SLOTS; ++q) {
-        d += acc_t[2 * q];
-        c += acc_t[2 * q + 1];
-    }
-    // the counts of this tick come from here, not from a previous tick's tile tags
-    *dec = push_num != 0u && d * 16ull <= (unsigned long long)push_num * c ? 2u : 0u;
-}
-
 __global__ void dec_demote_kernel(uint32_t *dec) {
     if (threadIdx.x < 2 && dec[threadIdx.x] == 1u) dec[threadIdx.x] = 2u;
-}
-
-// Direction statistics of one state buffer (local agents): acc[0] += sum of
-// degrees of agents in state inf, acc[1] += number of agents in state s_code.
-__global__ void acc_init_kernel(const int8_t *__restrict__ st, const int64_t *__restrict__ row_ptr, int64_t n_local,
-                                int8_t s_code, int8_t inf, unsigned long long *acc) {
-    unsigned long long d = 0, c = 0;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_local;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int8_t s = st[i];
-        if (s == inf) d += (unsigned long long)(row_ptr[i + 1] - row_ptr[i]);
-        c += s == s_code;
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        d += __shfl_down(d, off);
-        c += __shfl_down(c, off);
-    }
-    // one pair of atomics per block, spread over the slots (same-address
-    // atomics serialise)
-    __shared__ unsigned long long red[2 * 256 / 64];
-    const int wv = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) {
-        red[2 * wv] = d;
-        red[2 * wv + 1] = c;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int q = 1; q < (int)(blockDim.x >> 6); ++q) {
-            d += red[2 * q];
-            c += red[2 * q + 1];
-        }
-        const int slot = (int)(blockIdx.x % SS_ACC_SLOTS);
-        if (d) atomicAdd(&acc[2 * slot], d);
-        if (c) atomicAdd(&acc[2 * slot + 1], c);
-    }
 }
 
 inline unsigned grid_for(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
@@ -1464,27 +1518,27 @@ hipError_t ss_launch_tick(const ss_rep_dev *reps, const ss_tile *tiles, int n_ti
     return hipGetLastError();
 }
 
-hipError_t ss_launch_count_init(const int64_t *row_ptr, const int32_t *col_idx, const uint64_t *bits,
-                                int64_t n_local, int64_t heavy, uint16_t *cnt, uint32_t *dec,
-                                const unsigned long long *acc_t, uint32_t push_num, int grid, hipStream_t s) {
-    hipLaunchKernelGGL(dec_init_kernel, dim3(1), dim3(1), 0, s, acc_t, push_num, dec);
-    if (n_local <= 0) return hipGetLastError();
-    hipLaunchKernelGGL(count_init_kernel, dim3(grid), dim3(256), 0, s, row_ptr, col_idx, bits, n_local, heavy, cnt,
-                       (const uint32_t *)dec);
+hipError_t ss_launch_begin(const int8_t *src, int8_t *dst0, int8_t *dst1, uint64_t *bits0, uint64_t *bits1,
+                           const ss_begin &q, int num_cus, hipStream_t s) {
+    int parts = 0;
+    if (q.n_total > 0) {
+        parts = (int)std::min<int64_t>(SS_BEGIN_PARTS(num_cus), (int64_t)grid_for(q.n_total, 16 * 256));
+        hipLaunchKernelGGL(begin_kernel, dim3(parts), dim3(256), 0, s, (const SS_G int8_t *)src, (SS_G int8_t *)dst0,
+                           (SS_G int8_t *)dst1, bits0, bits1, (SS_G uint16_t *)q.cnt[0], (SS_G uint16_t *)q.cnt[1],
+                           (const SS_G uint8_t *)q.deg8, q.row_ptr, q.n_local, q.n_total, (uint32_t)(uint8_t)q.s_code,
+                           (uint32_t)(uint8_t)q.inf_code, q.part);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    // without counts to push, one block for the statistics
+    const int64_t grid = q.cnt[0] ? std::min<int64_t>((int64_t)num_cus * 8, std::max<int64_t>(1, grid_for(q.n_local, 256))) : 1;
+    hipLaunchKernelGGL(count_init_kernel, dim3((unsigned)grid), dim3(256), 0, s, q.part, parts, q.row_ptr, q.col_idx,
+                       q.bits, q.n_local, q.heavy, q.cnt_now, q.dec, q.acc, q.slot, q.push_num);
     return hipGetLastError();
 }
 
 hipError_t ss_launch_dec_demote(uint32_t *dec, hipStream_t s) {
     hipLaunchKernelGGL(dec_demote_kernel, dim3(1), dim3(64), 0, s, dec);
-    return hipGetLastError();
-}
-
-hipError_t ss_launch_acc_init(const int8_t *st, const int64_t *row_ptr, int64_t n_local, int8_t s_code, int8_t inf_code,
-                              unsigned long long *acc, int slot, int grid, hipStream_t s) {
-    if (n_local <= 0) return hipSuccess;
-    int g = (int)std::min<int64_t>(grid, (int64_t)grid_for(n_local, 256));
-    hipLaunchKernelGGL(acc_init_kernel, dim3(g), dim3(256), 0, s, st, row_ptr, n_local, s_code, inf_code,
-                       acc + slot * (SS_ACC_SLOTS * 2));
     return hipGetLastError();
 }
 
