@@ -352,6 +352,9 @@ int build_tiles(ss_ctx *ctx) {
                                    ctx->stream));
     SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
     ctx->n_tiles = (int)all.size();
+    ctx->only_rep = all.empty() ? -1 : all[0].rep;
+    for (const ss_tile &t : all)
+        if (t.rep != ctx->only_rep) { ctx->only_rep = -1; break; }
     for (int32_t ri = 0; ri < (int32_t)ctx->reps.size(); ++ri) {
         ss_replica &r = ctx->reps[ri];
         r.dev.tact[0] = ctx->d_tact[0];
@@ -432,7 +435,7 @@ void advance_ticks(ss_ctx *ctx, int64_t ticks) {
 
 // launch step k of a tick loop
 hipError_t tick_launch(ss_ctx *ctx, int64_t k) {
-    return ss_launch_tick(ctx->d_reps, ctx->d_tiles, ctx->n_tiles, (int)k, ctx->apl, ctx->grid,
+    return ss_launch_tick(ctx->d_reps, ctx->d_tiles, ctx->n_tiles, (int)k, ctx->apl, ctx->grid, ctx->only_rep,
                           ctx->counting ? ctx->d_work : nullptr, ctx->halo_fused, ctx->stream);
 }
 

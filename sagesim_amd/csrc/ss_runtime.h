@@ -28,8 +28,9 @@
 #define SS_WORK_N 7
 
 // kernel launchers (tick_kernels.hip)
+// only: the replica all tiles belong to, or -1
 hipError_t ss_launch_tick(const ss_rep_dev *reps, const ss_tile *tiles, int n_tiles, int k, int apl, int grid,
-                          unsigned long long *counters, bool halo, hipStream_t st);
+                          int only, unsigned long long *counters, bool halo, hipStream_t st);
 // agents of one HEAVY tile (4 wavefronts x 4 agents, tick_kernels.hip SS_HPW)
 #define SS_HEAVY_TILE 16
 #define SS_HEAVY_SHIFT 4
@@ -197,6 +198,7 @@ struct ss_ctx {
     int64_t tiles_cap = 0;
     int64_t slots_cap = 0;                      // tag slots allocated in d_tact
     int n_tiles = 0;
+    int only_rep = -1;                          // the replica all tiles belong to, or -1
     bool tiles_dirty = true;
     // tiling (autotuned by the host library)
     int hub_deg = 1024;
