@@ -39,22 +39,26 @@ struct Job {
 };
 
 struct Lane {
-    char *mem = nullptr;                   // two chunks, page-locked
+    char *mem[2] = {};                     // two chunks, page-locked
     hipEvent_t ev[2] = {};                 // the transfer of chunk s is done
     bool flying[2] = {};                   // ... and may not be yet
 };
 
-hipError_t open_lane(Lane &l) {
-    if (l.mem) return hipSuccess;
-    for (auto &ev : l.ev)
-        if (!ev) {
-            const hipError_t e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
-            if (e != hipSuccess) return e;
-        }
-    return hipHostMalloc((void **)&l.mem, 2 * kChunk, hipHostMallocDefault);
+// A chunk is allocated by the lane that first needs it, and each by itself: 1 MB
+// of page-locked memory takes 45 us, 2 MB and more 320 us (both chunks at once made
+// an engine with its first replica of 100k agents, beside others, 1.3 ms dearer).
+bool open_slot(Lane &l, int s) {
+    if (l.mem[s]) return true;
+    if ((l.ev[s] || hipEventCreateWithFlags(&l.ev[s], hipEventDisableTiming) == hipSuccess) &&
+        hipHostMalloc((void **)&l.mem[s], kChunk, hipHostMallocDefault) == hipSuccess)
+        return true;
+    l.mem[s] = nullptr;
+    (void)hipGetLastError();
+    return false;
 }
 
-// chunks of the job, claimed one by one, until none is left
+// chunks of the job, claimed one by one, until none is left (or this lane has no
+// memory for more)
 void run_lane(Lane &l, Job &j, hipStream_t stream) {
     const size_t n = (j.bytes + kChunk - 1) / kChunk;
     auto len = [&](size_t c) { return std::min(kChunk, j.bytes - c * kChunk); };
@@ -65,8 +69,8 @@ void run_lane(Lane &l, Job &j, hipStream_t stream) {
     };
     size_t pending = n;                    // down: the chunk on its way into the other slot
     for (int s = 0;; s ^= 1) {
-        const size_t c = j.next.fetch_add(1);
-        char *slot = l.mem + s * kChunk;
+        const size_t c = j.next.load() < n && open_slot(l, s) ? j.next.fetch_add(1) : n;
+        char *slot = l.mem[s];
         hipError_t e = hipSuccess;
         if (c < n) {
             if (j.in) {
@@ -80,7 +84,7 @@ void run_lane(Lane &l, Job &j, hipStream_t stream) {
         if (e == hipSuccess && !j.in && pending < n) {
             e = hipEventSynchronize(l.ev[s ^ 1]);
             l.flying[s ^ 1] = false;
-            if (e == hipSuccess) std::memcpy(j.host + pending * kChunk, l.mem + (s ^ 1) * kChunk, len(pending));
+            if (e == hipSuccess) std::memcpy(j.host + pending * kChunk, l.mem[s ^ 1], len(pending));
         }
         if (e != hipSuccess) return stop(e);
         if (c >= n) return;
@@ -128,10 +132,6 @@ struct ss_stager {
         int cpus = sched_getaffinity(0, sizeof set, &set) == 0 ? CPU_COUNT(&set) : 1;
         while (helpers + 1 < std::min(cpus, (int)SS_STAGE_LANES)) {
             const int i = helpers + 1;
-            if (open_lane(lane[i]) != hipSuccess) {
-                (void)hipGetLastError();
-                return;
-            }
             try {
                 thread[i] = std::thread([this, i] { help(i); });
             } catch (...) {
@@ -142,8 +142,7 @@ struct ss_stager {
     }
 
     hipError_t run(Job &j) {
-        hipError_t e = open_lane(lane[0]);
-        if (e != hipSuccess) return e;
+        hipError_t e = hipSuccess;
         const bool many = j.bytes >= kManyFrom && getpid() == pid;
         if (many) {
             hire();
@@ -160,7 +159,9 @@ struct ss_stager {
             job = nullptr;                 // a thread that is not awake yet finds nothing to do
             done.wait(g, [&] { return busy == 0; });
         }
-        return (hipError_t)j.err.load();
+        e = (hipError_t)j.err.load();
+        const bool all = j.next.load() * kChunk >= j.bytes;
+        return e == hipSuccess && !all ? hipErrorOutOfMemory : e;
     }
 
     ~ss_stager() {
@@ -176,7 +177,8 @@ struct ss_stager {
                 else t.detach();
             }
         for (auto &l : lane) {
-            if (l.mem) (void)hipHostFree(l.mem);
+            for (auto &m : l.mem)
+                if (m) (void)hipHostFree(m);
             for (auto &ev : l.ev)
                 if (ev) (void)hipEventDestroy(ev);
         }
