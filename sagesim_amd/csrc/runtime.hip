@@ -883,8 +883,8 @@ int ss_state_download_ordered(ss_ctx *ctx, int32_t rep, int8_t *out, int64_t n) 
     }
     const int8_t *st = r.state[r.tick & 1];
     if (!ss_known_to_hip(out)) {
-        SS_HIP(ctx, ss_stage_out(ctx, out, (size_t)n, [&](size_t at, size_t len, void *slot) {
-            return ss_launch_order(st, r.order, (int8_t *)slot, (int64_t)at, (int64_t)(at + len), r.n_local, ctx->stream);
+        SS_HIP(ctx, ss_stage_out(ctx, out, (size_t)n, [&](size_t at, size_t len, void *slot, hipStream_t on) {
+            return ss_launch_order(st, r.order, (int8_t *)slot, (int64_t)at, (int64_t)(at + len), r.n_local, on);
         }));
         return SS_OK;
     }

@@ -73,8 +73,8 @@ struct ss_stager;
 hipError_t ss_copy_in(ss_ctx *ctx, void *dev, const void *host, size_t bytes);
 hipError_t ss_copy_out(ss_ctx *ctx, void *host, const void *dev, size_t bytes);
 // down, of what issue(at, len, slot) writes into page-locked memory: bytes
-// [at, at + len) of the result to slot, enqueued on the context's stream, by any of its threads
-typedef std::function<hipError_t(size_t at, size_t len, void *slot)> ss_stage_issue;
+// [at, at + len) of the result to slot, enqueued on st, by any of its threads
+typedef std::function<hipError_t(size_t at, size_t len, void *slot, hipStream_t st)> ss_stage_issue;
 hipError_t ss_stage_out(ss_ctx *ctx, void *host, size_t bytes, const ss_stage_issue &issue);
 bool ss_known_to_hip(const void *p);            // page-locked or device memory
 void ss_stager_close(ss_ctx *ctx);

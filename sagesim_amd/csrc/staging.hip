@@ -28,12 +28,21 @@ namespace {
 
 const size_t kChunk = 1u << 20;
 const size_t kManyFrom = 4u << 20;         // below this, waking threads costs what they save
+// From here on a copy up goes over two streams: a chunk's kernel reads at 38 GB/s
+// (27 us) and the next one starts 6 us after it, where two kernels at a time fill
+// the gap.  Uploads of 112 and 32 MB for a ghost discovery 6.79 and 6.37 ms, a
+// replica of 10M agents and 50M entries 12.2 and 11.1, 26 MB of history down 0.61
+// and 0.57; handing over to the second stream and back costs some 20 us, which
+// 4 to 16 MB do not win back.  (No gain: six or eight lanes, stores past the
+// host's caches.)
+const size_t kForkFrom = 16u << 20;
 
 struct Job {
     char *host;
     size_t bytes;
     bool in;                               // host to device
     const ss_stage_issue *issue;
+    hipStream_t on[2];                     // the streams of the lanes' slots
     std::atomic<size_t> next{0};
     std::atomic<int> err{hipSuccess};
 };
@@ -59,7 +68,7 @@ bool open_slot(Lane &l, int s) {
 
 // chunks of the job, claimed one by one, until none is left (or this lane has no
 // memory for more)
-void run_lane(Lane &l, Job &j, hipStream_t stream) {
+void run_lane(Lane &l, Job &j) {
     const size_t n = (j.bytes + kChunk - 1) / kChunk;
     auto len = [&](size_t c) { return std::min(kChunk, j.bytes - c * kChunk); };
     auto stop = [&](hipError_t e) {
@@ -77,8 +86,8 @@ void run_lane(Lane &l, Job &j, hipStream_t stream) {
                 if (l.flying[s]) e = hipEventSynchronize(l.ev[s]);
                 if (e == hipSuccess) std::memcpy(slot, j.host + c * kChunk, len(c));
             }
-            if (e == hipSuccess) e = (*j.issue)(c * kChunk, len(c), slot);
-            if (e == hipSuccess) e = hipEventRecord(l.ev[s], stream);
+            if (e == hipSuccess) e = (*j.issue)(c * kChunk, len(c), slot, j.on[s]);
+            if (e == hipSuccess) e = hipEventRecord(l.ev[s], j.on[s]);
             if (e == hipSuccess) l.flying[s] = true;
         }
         if (e == hipSuccess && !j.in && pending < n) {
@@ -96,7 +105,8 @@ void run_lane(Lane &l, Job &j, hipStream_t stream) {
 
 struct ss_stager {
     int device;
-    hipStream_t stream;
+    hipStream_t stream, second;
+    hipEvent_t fork = nullptr, join = nullptr;
     pid_t pid;                             // threads do not survive a fork
     Lane lane[SS_STAGE_LANES];
     std::thread thread[SS_STAGE_LANES];
@@ -119,7 +129,7 @@ struct ss_stager {
             Job &j = *job;
             ++busy;
             g.unlock();
-            run_lane(lane[i], j, stream);
+            run_lane(lane[i], j);
             g.lock();
             if (--busy == 0) done.notify_all();
         }
@@ -141,25 +151,49 @@ struct ss_stager {
         }
     }
 
+    hipError_t fork_second() {
+        hipError_t e = hipSuccess;
+        for (hipEvent_t *ev : {&fork, &join})
+            if (!*ev && (e = hipEventCreateWithFlags(ev, hipEventDisableTiming)) != hipSuccess) return e;
+        if ((e = hipEventRecord(fork, stream)) != hipSuccess) return e;
+        return hipStreamWaitEvent(second, fork, 0);
+    }
+    hipError_t join_second() {
+        hipError_t e = hipSuccess;
+        if (!join && (e = hipEventCreateWithFlags(&join, hipEventDisableTiming)) != hipSuccess) return e;
+        if ((e = hipEventRecord(join, second)) != hipSuccess) return e;
+        return hipStreamWaitEvent(stream, join, 0);
+    }
+
     hipError_t run(Job &j) {
         hipError_t e = hipSuccess;
         const bool many = j.bytes >= kManyFrom && getpid() == pid;
+        j.on[0] = j.on[1] = stream;
         if (many) {
             hire();
             // what is queued before the copies would hold every lane
             if (!j.in && (e = hipStreamSynchronize(stream)) != hipSuccess) return e;
+            // every other chunk goes over the second stream, up after what is
+            // queued on the first and before what will be
+            if (j.in && j.bytes >= kForkFrom && (e = fork_second()) != hipSuccess) return e;
+            if (!j.in || j.bytes >= kForkFrom) j.on[1] = second;
             std::lock_guard<std::mutex> g(m);
             job = &j;
             ++turn;
             go.notify_all();
         }
-        run_lane(lane[0], j, stream);
+        run_lane(lane[0], j);
         if (many) {
             std::unique_lock<std::mutex> g(m);
             job = nullptr;                 // a thread that is not awake yet finds nothing to do
             done.wait(g, [&] { return busy == 0; });
         }
         e = (hipError_t)j.err.load();
+        // (a copy down has been waited for on both streams, unless it failed)
+        if (j.on[1] == second && (j.in || e != hipSuccess)) {
+            const hipError_t e2 = join_second();
+            if (e == hipSuccess) e = e2;
+        }
         const bool all = j.next.load() * kChunk >= j.bytes;
         return e == hipSuccess && !all ? hipErrorOutOfMemory : e;
     }
@@ -182,6 +216,8 @@ struct ss_stager {
             for (auto &ev : l.ev)
                 if (ev) (void)hipEventDestroy(ev);
         }
+        if (fork) (void)hipEventDestroy(fork);
+        if (join) (void)hipEventDestroy(join);
     }
 };
 
@@ -196,6 +232,7 @@ static hipError_t stager(ss_ctx *ctx) {
     if (!s) return hipErrorOutOfMemory;
     s->device = ctx->device;
     s->stream = ctx->stream;
+    s->second = ctx->copy_stream;
     s->pid = getpid();
     ctx->stager = s;
     return hipSuccess;
@@ -226,8 +263,8 @@ hipError_t ss_copy_out(ss_ctx *ctx, void *host, const void *dev, size_t bytes) {
         const hipError_t e = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, ctx->stream);
         return e == hipSuccess ? hipStreamSynchronize(ctx->stream) : e;
     }
-    return ss_stage_out(ctx, host, bytes, [&](size_t at, size_t len, void *slot) {
-        return ss_launch_stage((const char *)dev + at, slot, (int64_t)len, nullptr, nullptr, 0, ctx->stream);
+    return ss_stage_out(ctx, host, bytes, [&](size_t at, size_t len, void *slot, hipStream_t st) {
+        return ss_launch_stage((const char *)dev + at, slot, (int64_t)len, nullptr, nullptr, 0, st);
     });
 }
 
@@ -239,8 +276,8 @@ hipError_t ss_copy_in(ss_ctx *ctx, void *dev, const void *host, size_t bytes) {
     }
     const hipError_t e = stager(ctx);
     if (e != hipSuccess) return e;
-    const ss_stage_issue issue = [&](size_t at, size_t len, void *slot) {
-        return ss_launch_stage(slot, (char *)dev + at, (int64_t)len, nullptr, nullptr, 0, ctx->stream);
+    const ss_stage_issue issue = [&](size_t at, size_t len, void *slot, hipStream_t st) {
+        return ss_launch_stage(slot, (char *)dev + at, (int64_t)len, nullptr, nullptr, 0, st);
     };
     Job j;
     j.host = (char *)const_cast<void *>(host);

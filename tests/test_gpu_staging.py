@@ -59,3 +59,22 @@ def test_two_contexts_at_once():
     for t in ts:
         t.join()
     assert not bad
+
+
+@pytest.mark.parametrize("n", [16 * MB - 1, 16 * MB, 21 * MB + 3])
+def test_uploads_over_two_streams(n):
+    """Around the 16 MiB from where every other chunk goes over the second
+    stream: after work that still reads the states, before work that does."""
+    print("two streams", n, flush=True)
+    rng = np.random.default_rng(n)
+    with Engine() as eng:
+        rep = eng.add_replica(np.zeros(n + 1, np.int64), np.zeros(0, np.int32), np.arange(n),
+                              rng.integers(0, 3, n, dtype=np.int8), sir_model(0.5, 1.0), 1)
+        for _ in range(3):
+            st = rng.integers(0, 3, n, dtype=np.int8)
+            eng.simulate(2)
+            eng.set_state(rep, st)
+            assert eng.census(rep)[:3].tolist() == np.bincount(st, minlength=3).tolist()
+            eng.simulate(1)                                     # every infectious agent recovers
+            st[st == 1] = 2
+            assert np.array_equal(eng.state(rep, n), st)
