@@ -304,28 +304,41 @@ __global__ void halo_unpack_ids_kernel(const unsigned long long *__restrict__ ke
 }
 
 // Pack (gpu_kernels.py:852-909 gathers rows of the send list): out[h] = st[slots[h]].
+// A slot outside [0, n_total) reads as 0 and sets *bad: the range check costs
+// nothing here, where a pass over 72k slots on the host took 16 of a pack's 47 us.
+__device__ __forceinline__ uint32_t state_at(const int8_t *__restrict__ st, int32_t slot, uint32_t n_total,
+                                             uint32_t &wrong) {
+    const bool in = (uint32_t)slot < n_total;
+    wrong |= in ? 0u : 1u;
+    return in ? (uint32_t)(uint8_t)st[slot] : 0u;
+}
+
 __global__ void gather_kernel(const int8_t *__restrict__ st, const int32_t *__restrict__ slots,
-                              int8_t *__restrict__ out, int64_t n) {
+                              int8_t *__restrict__ out, int64_t n, uint32_t n_total, uint32_t *bad) {
     const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g < n) out[g] = st[slots[g]];
+    if (g >= n) return;
+    uint32_t wrong = 0u;
+    out[g] = (int8_t)state_at(st, slots[g], n_total, wrong);
+    if (wrong && bad) *bad = 1u;
 }
 
 // The same as 2-bit codes, four records a byte (record h in bits 2 (h % 4)
 // and 2 (h % 4) + 1 of byte h / 4); states are taken modulo 4.
 __global__ void gather2_kernel(const int8_t *__restrict__ st, const int32_t *__restrict__ slots,
-                               uint8_t *__restrict__ out, int64_t n) {
+                               uint8_t *__restrict__ out, int64_t n, uint32_t n_total, uint32_t *bad) {
     const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (4 * j >= n) return;
-    uint32_t b = 0u;
+    uint32_t b = 0u, wrong = 0u;
     if (4 * j + 4 <= n) {                               // one load of the four slots
         struct __attribute__((packed, aligned(4))) Four { int32_t s[4]; };
         const Four f = *(const Four *)(slots + 4 * j);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) b |= ((uint32_t)(uint8_t)st[f.s[q]] & 3u) << (2 * q);
+        for (int q = 0; q < 4; ++q) b |= (state_at(st, f.s[q], n_total, wrong) & 3u) << (2 * q);
     } else {
-        for (int q = 0; 4 * j + q < n; ++q) b |= ((uint32_t)(uint8_t)st[slots[4 * j + q]] & 3u) << (2 * q);
+        for (int q = 0; 4 * j + q < n; ++q) b |= (state_at(st, slots[4 * j + q], n_total, wrong) & 3u) << (2 * q);
     }
     out[j] = (uint8_t)b;
+    if (wrong && bad) *bad = 1u;
 }
 
 // 0x80 in every byte of x that equals the byte whose copies fill y.
@@ -549,15 +562,19 @@ hipError_t ss_launch_halo_unpack_ids(const unsigned long long *keys, const int32
     return hipGetLastError();
 }
 
-hipError_t ss_launch_gather(const int8_t *st, const int32_t *slots, int8_t *out, int64_t n, hipStream_t s) {
+hipError_t ss_launch_gather(const int8_t *st, const int32_t *slots, int8_t *out, int64_t n, int64_t n_total,
+                            uint32_t *bad, hipStream_t s) {
     if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(gather_kernel, dim3(grid_for(n, 256)), dim3(256), 0, s, st, slots, out, n);
+    hipLaunchKernelGGL(gather_kernel, dim3(grid_for(n, 256)), dim3(256), 0, s, st, slots, out, n, (uint32_t)n_total,
+                       bad);
     return hipGetLastError();
 }
 
-hipError_t ss_launch_gather2(const int8_t *st, const int32_t *slots, uint8_t *out, int64_t n, hipStream_t s) {
+hipError_t ss_launch_gather2(const int8_t *st, const int32_t *slots, uint8_t *out, int64_t n, int64_t n_total,
+                             uint32_t *bad, hipStream_t s) {
     if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(gather2_kernel, dim3(grid_for((n + 3) / 4, 256)), dim3(256), 0, s, st, slots, out, n);
+    hipLaunchKernelGGL(gather2_kernel, dim3(grid_for((n + 3) / 4, 256)), dim3(256), 0, s, st, slots, out, n,
+                       (uint32_t)n_total, bad);
     return hipGetLastError();
 }
 

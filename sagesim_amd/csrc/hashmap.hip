@@ -34,6 +34,16 @@ __global__ void map_fill_kernel(unsigned long long *keys, int32_t *vals, int64_t
     }
 }
 
+// *bad = 1 (page-locked) when an id is reserved (-1, -2) or a slot outside [0, n_total)
+__global__ __launch_bounds__(256) void map_check_kernel(const int64_t *__restrict__ ids,
+                                                        const int32_t *__restrict__ slots, int64_t n, uint32_t n_total,
+                                                        uint32_t *bad) {
+    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (g >= n) return;
+    const int64_t id = ids[g];
+    if (id == -1 || id == -2 || (uint32_t)slots[g] >= n_total) *bad = 1u;
+}
+
 // ---- build ----
 // claim[s] = steps << 32 | index of the entry that holds slot s (all ones:
 // none).  A thread carries one entry at a time to its next slot until a slot
@@ -148,6 +158,13 @@ inline unsigned grid_of(int64_t n, int b) { return (unsigned)((n + b - 1) / b); 
 hipError_t ss_launch_map_clear(unsigned long long *keys, int32_t *vals, int64_t cap, hipStream_t s) {
     if (cap <= 0) return hipSuccess;
     hipLaunchKernelGGL(map_fill_kernel, dim3(grid_of(cap, 256)), dim3(256), 0, s, keys, vals, cap);
+    return hipGetLastError();
+}
+
+hipError_t ss_launch_map_check(const int64_t *ids, const int32_t *slots, int64_t n, int64_t n_total, uint32_t *bad,
+                               hipStream_t s) {
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(map_check_kernel, dim3(grid_of(n, 256)), dim3(256), 0, s, ids, slots, n, (uint32_t)n_total, bad);
     return hipGetLastError();
 }
 

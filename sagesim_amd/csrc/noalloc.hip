@@ -73,7 +73,7 @@ extern "C" int ss_halo_pack_noalloc(ss_ctx *ctx, int32_t rep, const int32_t *slo
     int8_t *d_out = static_cast<int8_t *>(base) + kSlotBytes;
     e = hipStreamSynchronize(ctx->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(d_slots, slots, sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice, ctx->stream);
-    if (e == hipSuccess) e = ss_launch_gather(r.state[r.tick & 1], d_slots, d_out, n, ctx->stream);
+    if (e == hipSuccess) e = ss_launch_gather(r.state[r.tick & 1], d_slots, d_out, n, r.n_total, nullptr, ctx->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(out, d_out, (size_t)n, hipMemcpyDeviceToHost, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess) return fail(ctx, SS_ERR_HIP, "halo pack: error %lld", (long long)e);

@@ -1109,8 +1109,6 @@ int ss_map_build(ss_ctx *ctx, int32_t rep, const int64_t *ids, const int32_t *sl
     if (!(lf > 0.0 && lf <= 0.9)) SS_FAIL(ctx, SS_ERR_INVALID, "load_factor must be in (0, 0.9]");
     if (n >= INT32_MAX) SS_FAIL(ctx, SS_ERR_INVALID, "at most 2^31 - 2 entries");
     ss_replica &r = ctx->reps[rep];
-    int rc = check_map_entries(ctx, r, ids, slots, n);
-    if (rc) return rc;
     const int64_t cap = std::max<int64_t>(64, (int64_t)std::ceil((double)n / lf));
     SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
     Scratch guard(ctx);
@@ -1119,13 +1117,22 @@ int ss_map_build(ss_ctx *ctx, int32_t rep, const int64_t *ids, const int32_t *sl
     SS_HIP(ctx, scratch(ctx, b_ids + b_vals + sizeof(unsigned long long) * (size_t)cap, &w));
     int64_t *d_ids = (int64_t *)w;
     int32_t *d_vals = (int32_t *)((char *)w + b_ids);
+    int rc = SS_OK;
+    // the entries are checked on the device (a pass over 1.6M of them on the host
+    // took 0.8 of 1.7 ms), before the table that is there is touched
+    if (n > 0) {
+        volatile uint32_t *bad = (volatile uint32_t *)ctx->h_stats;
+        *bad = 0u;
+        SS_HIP(ctx, ss_copy_in(ctx, d_ids, ids, sizeof(int64_t) * (size_t)n));
+        SS_HIP(ctx, ss_copy_in(ctx, d_vals, slots, sizeof(int32_t) * (size_t)n));
+        SS_HIP(ctx, ss_launch_map_check(d_ids, d_vals, n, r.n_total, (uint32_t *)ctx->h_stats, ctx->stream));
+        SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        if (*bad && (rc = check_map_entries(ctx, r, ids, slots, n))) return rc;
+    }
     if ((rc = alloc_map(ctx, r, cap, n == 0))) return rc;
     if (n > 0) {
-        hipError_t e = ss_copy_in(ctx, d_ids, ids, sizeof(int64_t) * (size_t)n);
-        if (e == hipSuccess) e = ss_copy_in(ctx, d_vals, slots, sizeof(int32_t) * (size_t)n);
-        if (e == hipSuccess)
-            e = ss_launch_map_build(r.map_keys, r.map_vals, cap, d_ids, d_vals, n,
-                                    (unsigned long long *)((char *)w + b_ids + b_vals), ctx->num_cus, ctx->stream);
+        hipError_t e = ss_launch_map_build(r.map_keys, r.map_vals, cap, d_ids, d_vals, n,
+                                           (unsigned long long *)((char *)w + b_ids + b_vals), ctx->num_cus, ctx->stream);
         if (e != hipSuccess) (void)ss_launch_map_clear(r.map_keys, r.map_vals, cap, ctx->stream);   // an empty table
         const hipError_t e2 = hipStreamSynchronize(ctx->stream);
         SS_HIP(ctx, e);
@@ -1359,15 +1366,16 @@ int ss_halo_unpack_ids(ss_ctx *ctx, int32_t rep, const int64_t *ids, const int8_
 static int halo_pack(ss_ctx *ctx, int32_t rep, const int32_t *slots, int64_t n, void *out, bool packed) {
     if (!valid_rep(ctx, rep) || (n && (!slots || !out))) SS_FAIL(ctx, SS_ERR_INVALID, "bad replica or NULL");
     ss_replica &r = ctx->reps[rep];
-    for (int64_t b = 0; b < n; b += 4096) {             // without branches, one by one only where one is wrong
-        const int64_t e = std::min<int64_t>(n, b + 4096);
-        uint32_t bad = 0;
-        for (int64_t i = b; i < e; ++i) bad |= (uint32_t)((uint64_t)(int64_t)slots[i] >= (uint64_t)r.n_total);
-        for (int64_t i = b; bad && i < e; ++i)
-            if (slots[i] < 0 || slots[i] >= r.n_total) SS_FAIL(ctx, SS_ERR_RANGE, "slot %d outside the replica", slots[i]);
-    }
     if (n == 0) return SS_OK;
     const size_t nb = (size_t)(packed ? (n + 3) / 4 : n), b_slots = up256(sizeof(int32_t) * (size_t)n);
+    // the kernel says here whether a slot was outside; nothing is returned then
+    uint32_t *bad = (uint32_t *)ctx->h_stats;
+    auto outside = [&]() -> int {
+        for (int64_t i = 0; i < n; ++i)
+            if (slots[i] < 0 || slots[i] >= r.n_total) SS_FAIL(ctx, SS_ERR_RANGE, "slot %d outside the replica", slots[i]);
+        return SS_OK;
+    };
+    *(volatile uint32_t *)bad = 0u;
     if (b_slots + nb <= (size_t)SS_STAGE_BYTES) {
         // the kernel reads the slots from page-locked memory and writes the
         // result there: no copy engine in the chain behind the tick
@@ -1375,9 +1383,13 @@ static int halo_pack(ss_ctx *ctx, int32_t rep, const int32_t *slots, int64_t n, 
         int8_t *h_out = (int8_t *)ctx->h_stage + b_slots;
         std::memcpy(ctx->h_stage, slots, sizeof(int32_t) * (size_t)n);
         const int32_t *h_slots = (const int32_t *)ctx->h_stage;
-        SS_HIP(ctx, packed ? ss_launch_gather2(r.state[r.tick & 1], h_slots, (uint8_t *)h_out, n, ctx->stream)
-                           : ss_launch_gather(r.state[r.tick & 1], h_slots, h_out, n, ctx->stream));
+        SS_HIP(ctx, packed ? ss_launch_gather2(r.state[r.tick & 1], h_slots, (uint8_t *)h_out, n, r.n_total, bad, ctx->stream)
+                           : ss_launch_gather(r.state[r.tick & 1], h_slots, h_out, n, r.n_total, bad, ctx->stream));
         SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        if (*(volatile uint32_t *)bad) {
+            const int rc = outside();
+            if (rc) return rc;
+        }
         std::memcpy(out, h_out, nb);
         return SS_OK;
     }
@@ -1386,8 +1398,13 @@ static int halo_pack(ss_ctx *ctx, int32_t rep, const int32_t *slots, int64_t n, 
     SS_HIP(ctx, scratch(ctx, b_slots + nb, &w));
     int8_t *d_out = (int8_t *)w + b_slots;
     SS_HIP(ctx, ss_copy_in(ctx, w, slots, sizeof(int32_t) * (size_t)n));
-    SS_HIP(ctx, packed ? ss_launch_gather2(r.state[r.tick & 1], (const int32_t *)w, (uint8_t *)d_out, n, ctx->stream)
-                       : ss_launch_gather(r.state[r.tick & 1], (const int32_t *)w, d_out, n, ctx->stream));
+    SS_HIP(ctx, packed ? ss_launch_gather2(r.state[r.tick & 1], (const int32_t *)w, (uint8_t *)d_out, n, r.n_total, bad, ctx->stream)
+                       : ss_launch_gather(r.state[r.tick & 1], (const int32_t *)w, d_out, n, r.n_total, bad, ctx->stream));
+    SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (*(volatile uint32_t *)bad) {
+        const int rc = outside();
+        if (rc) return rc;
+    }
     SS_HIP(ctx, ss_copy_out(ctx, out, d_out, nb));
     return SS_OK;
 }

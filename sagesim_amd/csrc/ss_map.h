@@ -19,6 +19,9 @@ __host__ __device__ __forceinline__ int64_t ss_map_home(int64_t id, int64_t cap)
 
 // keys = -1, values = -1 over the whole table
 hipError_t ss_launch_map_clear(unsigned long long *keys, int32_t *vals, int64_t cap, hipStream_t s);
+// *bad = 1 when an id is reserved or a slot outside [0, n_total)
+hipError_t ss_launch_map_check(const int64_t *ids, const int32_t *slots, int64_t n, int64_t n_total, uint32_t *bad,
+                               hipStream_t s);
 // build of n < cap entries into the whole table; claim: workspace of cap words
 hipError_t ss_launch_map_build(unsigned long long *keys, int32_t *vals, int64_t cap, const int64_t *ids,
                                const int32_t *slot_vals, int64_t n, unsigned long long *claim, int num_cus,

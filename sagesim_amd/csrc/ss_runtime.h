@@ -55,9 +55,13 @@ hipError_t ss_launch_halo_gather(int8_t *s0, int8_t *s1, const int8_t *cur, uint
 hipError_t ss_launch_halo_unpack_ids(const unsigned long long *keys, const int32_t *mvals, int64_t cap,
                                      const int64_t *ids, const int8_t *vals, int64_t n, int8_t *s0, int8_t *s1,
                                      int32_t *misses, hipStream_t s);
-hipError_t ss_launch_gather(const int8_t *st, const int32_t *slots, int8_t *out, int64_t n, hipStream_t s);
+// a slot outside [0, n_total) reads as 0 and stores 1 to *bad (page-locked; may
+// be null where the slots have been checked)
+hipError_t ss_launch_gather(const int8_t *st, const int32_t *slots, int8_t *out, int64_t n, int64_t n_total,
+                            uint32_t *bad, hipStream_t s);
 // out[h / 4] bits 2 (h % 4).. = st[slots[h]] & 3
-hipError_t ss_launch_gather2(const int8_t *st, const int32_t *slots, uint8_t *out, int64_t n, hipStream_t s);
+hipError_t ss_launch_gather2(const int8_t *st, const int32_t *slots, uint8_t *out, int64_t n, int64_t n_total,
+                             uint32_t *bad, hipStream_t s);
 hipError_t ss_launch_fill_i32(int32_t *p, int64_t n, int32_t v, hipStream_t s);
 // out[j - first] = st[slot[j]], j < n_local; st[j] for the ghosts; for
 // first <= j < end (slot and out padded to whole groups of 16, first a multiple)

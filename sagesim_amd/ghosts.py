@@ -63,7 +63,7 @@ def ghost_maps(engine: Engine, all_neighbors, agent2rank, my_rank: int, n_local:
         pos = index[offsets[r]:offsets[r + 1]]
         if pos.size:
             out.recv_ids[r] = ids[pos]
-            out.recv_slots[r] = (pos + int(n_local)).astype(np.int32)
+            out.recv_slots[r] = (pos + int(n_local)).astype(np.int32, copy=False)
     return out
 
 

@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 from sagesim_amd import Engine, pack_2bit, sir_model, workloads
+from sagesim_amd._lib import NativeError
 from sagesim_amd.engine import Replica
 
 pytestmark = pytest.mark.gpu
@@ -69,3 +70,26 @@ def test_pack_either_side_of_the_staging_size(n):
         slots = rep.inv[agents].astype(np.int32)
         assert np.array_equal(eng.halo_pack(rep.rep, slots), st[agents])
         assert np.array_equal(eng.halo_pack_2bit(rep.rep, slots), pack_2bit(st[agents]))
+
+
+@pytest.mark.parametrize("n", [1, 4, 5, 1027, 300_000])
+def test_pack_of_a_slot_outside(n):
+    """A slot outside the replica, anywhere in the list, is an error, and the
+    next pack is not."""
+    g = workloads.sbm_partition(n_blocks=4, block_size=1500, deg_in=8, deg_out=1, n_parts=2, part=0, ticks=1,
+                                seed=3).graph
+    state = np.random.default_rng(n).integers(0, 3, g.n_cols).astype(np.int8)
+    with Engine() as eng:
+        rep = Replica(eng, g, state, sir_model(0.3, 0.1), 9)
+        agents = np.random.default_rng(n + 1).integers(0, g.n, n)
+        slots = rep.inv[agents].astype(np.int32)
+        for at in sorted({0, n // 2, n - 1}):
+            for wrong in (-1, rep.n_total, 2**31 - 1, -(2**31)):
+                say("pack outside", n, at, wrong)
+                bad = slots.copy()
+                bad[at] = wrong
+                for pack in (eng.halo_pack, eng.halo_pack_2bit):
+                    with pytest.raises(NativeError, match="slot %d outside the replica" % wrong):
+                        pack(rep.rep, bad)
+        assert np.array_equal(eng.halo_pack(rep.rep, slots), state[agents])
+        assert np.array_equal(eng.halo_pack_2bit(rep.rep, slots), pack_2bit(state[agents]))

@@ -198,3 +198,28 @@ def test_halo_bound_twice_and_low_slots():
                     if i >= 1000:
                         want[i - 1000] = v
                 assert np.array_equal(e.state(r.rep, n + ghosts), want)
+
+
+@pytest.mark.parametrize("n", [1, 256, 4097])
+def test_build_of_wrong_entries_leaves_the_table(n):
+    """A reserved id or a slot outside the replica, anywhere in the batch, is an
+    error that names it, and the map of the build before stays as it was."""
+    g = graphs.from_edges(5000, np.arange(1), np.arange(1, 2))
+    ids, slots = np.arange(n, dtype=np.int64) * 7 - 3000, np.arange(n, dtype=np.int32)
+    ids[(ids == -1) | (ids == -2)] = 1 << 45
+    with Engine(0) as e:
+        r = Replica(e, g, np.zeros(5000, np.int8), sir_model(0.1, 0.1), 1)
+        e.map_build(r.rep, ids, slots, 0.5)
+        before = e.map_arrays(r.rep)
+        for at in sorted({0, n // 2, n - 1}):
+            for wrong_id, wrong_slot in ((-1, None), (-2, None), (None, -1), (None, 5000), (None, -(2**31))):
+                print("[case] wrong entry", n, at, wrong_id, wrong_slot, flush=True)
+                i, s = ids.copy(), slots.copy()
+                if wrong_id is not None:
+                    i[at] = wrong_id
+                else:
+                    s[at] = wrong_slot
+                with pytest.raises(NativeError, match="reserved" if wrong_id is not None else "slot %d outside" % wrong_slot):
+                    e.map_build(r.rep, i, s, 0.9)
+                assert all(np.array_equal(a, b) for a, b in zip(before, e.map_arrays(r.rep)))
+        assert e.map_lookup(r.rep, ids)[1] == 0
