@@ -56,3 +56,14 @@ def test_one_longer_row():
     g = graphs.from_edges(n, np.concatenate([u, [17, 17, 17]]), np.concatenate([(u + 1) % n, [900, 2000, 4000]]))
     for sort in (True, False):
         _check(g, 0.5, 12, False, 0.0, sort=sort)
+
+
+@pytest.mark.parametrize("beta", [0.02, 0.2])
+@pytest.mark.parametrize("d", [10, 12, 15, 24, 63, 64, 65, 71, 72, 73, 80])
+def test_scans_that_give_up(d, beta):
+    """Rows whose scan ends when what is left cannot infect: lengths around
+    whole rounds of eight and around the 64 thresholds held in LDS, few and many
+    hits needed, every tick pulled."""
+    print("[case] scans that give up", d, beta, flush=True)
+    for history in (False, True):
+        _check(_circulant(3002, d), beta, 8, history, 0.0)
