@@ -139,7 +139,8 @@ int ss_simulate(ss_ctx *ctx, int64_t ticks);
  * scan; the rest run agents_per_lane (1, 2, 4, 8 or 16) agents per lane.  Degrees
  * are one of 8,16,24,32,48,64,96,128,192,256,512,1024,2048,4096,16384,2^30.
  * grid_blocks = 0 sizes the persistent grid from occupancy; use_graph = 0
- * launches tick by tick instead of replaying a captured hipGraph. */
+ * launches tick by tick instead of replaying a captured hipGraph.  Without a
+ * call: 1024 (2048 when the replicas hold 64M entries or more), 256, 16, 0, 1. */
 int ss_set_tiling(ss_ctx *ctx, int32_t hub_degree, int32_t heavy_degree, int32_t agents_per_lane,
                   int32_t grid_blocks, int32_t use_graph);
 /* tiles and grid of the current launch shape (after ss_simulate built them) */

@@ -206,6 +206,7 @@ struct ss_ctx {
     bool tiles_dirty = true;
     // tiling (autotuned by the host library)
     int hub_deg = 1024;
+    bool tiling_given = false;                  // by ss_set_tiling (else build_tiles picks hub_deg)
     int heavy_deg = 256;
     int apl = 16;
     int grid_blocks = 0;                        // 0: persistent grid from occupancy
