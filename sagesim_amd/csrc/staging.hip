@@ -54,8 +54,7 @@ struct Lane {
 };
 
 // A chunk is allocated by the lane that first needs it, and each by itself: 1 MB
-// of page-locked memory takes 45 us, 2 MB and more 320 us (both chunks at once made
-// an engine with its first replica of 100k agents, beside others, 1.3 ms dearer).
+// of page-locked memory takes 45 us, 2 MB and more 320 us.
 bool open_slot(Lane &l, int s) {
     if (l.mem[s]) return true;
     if ((l.ev[s] || hipEventCreateWithFlags(&l.ev[s], hipEventDisableTiming) == hipSuccess) &&
