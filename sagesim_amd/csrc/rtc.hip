@@ -320,7 +320,9 @@ int ss_prog_create(ss_ctx *ctx, int64_t n_agents, ss_prog **out) {
     if (e == hipSuccess) e = hipMalloc((void **)&p->breeds, nn * sizeof(float));
     if (e == hipSuccess) e = hipMalloc((void **)&p->logical_ids64, nn * sizeof(int64_t));
     if (e == hipSuccess) e = hipMalloc((void **)&p->row_ptr, (nn + 1) * sizeof(int64_t));
-    if (e == hipSuccess) e = hipMemset(p->row_ptr, 0, (nn + 1) * sizeof(int64_t));
+    // on the context's stream, like the upload that follows (ss_prog_set_csr): a
+    // clear on the null stream could land after it and empty every row
+    if (e == hipSuccess) e = hipMemsetAsync(p->row_ptr, 0, (nn + 1) * sizeof(int64_t), ctx->stream);
     if (e != hipSuccess) {
         g_prog_err = std::string("ss_prog_create: ") + hipGetErrorString(e);
         pfree(p->d_args); pfree(p->agent_ids); pfree(p->logical_ids); pfree(p->breeds); pfree(p->row_ptr);
