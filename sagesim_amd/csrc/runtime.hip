@@ -512,7 +512,7 @@ int ss_create(int device, ss_ctx **out) {
         (e = hipEventCreate(&ctx->t_start)) != hipSuccess || (e = hipEventCreate(&ctx->t_stop)) != hipSuccess ||
         (e = hipMalloc((void **)&ctx->d_work, SS_WORK_N * sizeof(unsigned long long))) != hipSuccess ||
         (e = hipMalloc((void **)&ctx->d_stats, 8 * sizeof(unsigned long long))) != hipSuccess ||
-        (e = hipMemset(ctx->d_work, 0, SS_WORK_N * sizeof(unsigned long long))) != hipSuccess ||
+        (e = hipMemsetAsync(ctx->d_work, 0, SS_WORK_N * sizeof(unsigned long long), ctx->stream)) != hipSuccess ||
         (e = hipMalloc((void **)&ctx->d_part, 2 * sizeof(unsigned long long) * SS_BEGIN_PARTS(prop.multiProcessorCount))) != hipSuccess ||
         (e = hipMalloc((void **)&ctx->d_counters, 64 * sizeof(int32_t))) != hipSuccess ||
         (e = hipHostMalloc((void **)&ctx->h_stats,
@@ -1685,7 +1685,7 @@ int ss_read_counters(ss_ctx *ctx, int64_t *out) {
     SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
     unsigned long long h[SS_WORK_N];
     SS_HIP(ctx, hipMemcpy(h, ctx->d_work, sizeof h, hipMemcpyDeviceToHost));
-    SS_HIP(ctx, hipMemset(ctx->d_work, 0, sizeof h));
+    SS_HIP(ctx, hipMemsetAsync(ctx->d_work, 0, sizeof h, ctx->stream));   // before the next call's ticks
     for (int i = 0; i < SS_WORK_N; ++i) out[i] = (int64_t)h[i];
     return SS_OK;
 }

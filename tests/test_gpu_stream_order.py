@@ -49,3 +49,22 @@ def test_model_set_up_beside_queued_ticks(n, busy):
         m.simulate(10)
         assert np.array_equal(m.get_breed_data("SIR", "state"), want)
         m.reset()
+
+
+def test_counters_cleared_beside_queued_ticks(busy):
+    print("[case] counters beside queued ticks", flush=True)
+    g = graphs.barabasi_albert(3000, 5, 1)
+    st = (np.random.default_rng(1).random(g.n) < 0.02).astype(np.int8)
+    want = None
+    for _ in range(5):
+        busy()
+        with Engine(0) as eng:
+            eng.set_counting(True)
+            rep = Replica(eng, g, st, sir_model(0.05, 0.1), 1)
+            for _ in range(3):
+                rep.reset()
+                eng.simulate(20)
+                got = eng.read_counters()
+                busy()
+                want = got if want is None else want
+                assert np.array_equal(got, want)

@@ -16,7 +16,7 @@ def _code(name):
     return re.sub(r"//[^\n]*|/\*.*?\*/", "", text, flags=re.S)
 
 
-@pytest.mark.parametrize("name", ["rtc.hip"])
+@pytest.mark.parametrize("name", sorted(f for f in os.listdir(CSRC) if f.endswith((".hip", ".h"))))
 def test_no_clear_on_the_null_stream(name):
     calls = re.findall(r"\bhipMemset(?:D8|D16|D32|2D|3D)?\s*\([^;]*;", _code(name))
     assert not calls, calls
