@@ -834,7 +834,8 @@ class Model:
         s = np.asarray(start, np.int64)
         c = np.asarray(count, np.int64)
         prog.ck(L.ss_prog_set_schedule(h, len(k), ptr(k), ptr(s), ptr(c)))
-        if any(not np.array_equal(o[0], np.arange(o[0].size)) for o in orders):
+        # (staged rows are looked up in the order, whatever it is)
+        if any(o[1] or not np.array_equal(o[0], np.arange(o[0].size)) for o in orders):
             segs = [lo + o[0] for lo, o in zip(start, orders)]
             ordr = np.ascontiguousarray(np.concatenate(segs), np.int32)
             prog.ck(L.ss_prog_set_order(h, ptr(ordr), ordr.shape[0]))
