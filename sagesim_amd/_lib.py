@@ -12,8 +12,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 STEP_LIB_PATH = os.path.join(HERE, "libsagestep.so")
 GRAPH_LIB_PATH = os.path.join(HERE, "libsagegraph.so")
 
-SS_OK = 0
-SS_ERR = {-1: "SS_ERR_INVALID", -2: "SS_ERR_HIP", -3: "SS_ERR_OOM", -4: "SS_ERR_RANGE",
+SS_OK, SS_ERR_OOM = 0, -3
+SS_ERR = {-1: "SS_ERR_INVALID", -2: "SS_ERR_HIP", SS_ERR_OOM: "SS_ERR_OOM", -4: "SS_ERR_RANGE",
           -5: "SS_ERR_STATE", -6: "SS_ERR_RTC", -7: "SS_ERR_FULL"}
 HISTORY_WIDTH = 32
 

@@ -584,7 +584,7 @@ int ss_device_info(ss_ctx *ctx, int32_t *num_cus, int64_t *total_mem, int64_t *c
 int64_t ss_replica_footprint(int64_t n_local, int64_t n_ghost, int64_t nnz, int32_t with_history, int64_t max_deg) {
     int64_t n_total = n_local + n_ghost;
     int64_t words = (n_total + 63) / 64;
-    int64_t b = 8 * (n_total + 1) + 4 * (nnz + SS_COL_PAD) + 6 * pad_agents(n_local) + 3 * pad_agents(n_total) +
+    int64_t b = 8 * (n_total + 1) + 4 * (nnz + SS_COL_PAD) + 10 * pad_agents(n_local) + 3 * pad_agents(n_total) +
                 2 * 8 * words + 4 * (std::min<int64_t>(max_deg, 1 << 24) + 1) + 8 * SS_ACC_WORDS +
                 (n_ghost == 0 ? 4 * pad_agents(n_local) + 8 : 0);
     if (with_history) b += 2 * 4 * n_local * SS_HISTORY_WIDTH;

@@ -12,7 +12,7 @@ from dataclasses import dataclass
 
 import numpy as np
 
-from ._lib import (HISTORY_WIDTH, NativeError, SSModel, SSReplicaSpec, ptr, step_lib)
+from ._lib import (HISTORY_WIDTH, SS_ERR_OOM, NativeError, SSModel, SSReplicaSpec, ptr, step_lib)
 from .graphs import CSRGraph, degree_sort
 
 S, I, R = 0, 1, 2
@@ -457,9 +457,16 @@ class Replica:
 
     def states(self):
         """The states in the caller's agent order (put in order on the device,
-        which keeps the order from the first call on)."""
+        which keeps the order from the first call on; on the host when the device
+        has no memory left for it)."""
         if not self._order_set:
-            self.engine.set_order(self.rep, self.inv)
+            try:
+                self.engine.set_order(self.rep, self.inv)
+            except NativeError as e:
+                if e.code != SS_ERR_OOM:
+                    raise
+                st = self.engine.state(self.rep, self.n_total)
+                return np.concatenate([st[:self.n][self.inv], st[self.n:]])
             self._order_set = True
         return self.engine.state_ordered(self.rep, self.n_total)
 

@@ -1,0 +1,65 @@
+"""What a device without memory to spare still does: states() without the order
+table it keeps on the device, and a footprint that counts the table."""
+import numpy as np
+import pytest
+
+from sagesim_amd import Engine, Replica, graphs, sir_model
+from sagesim_amd._lib import SS_ERR_OOM, NativeError, step_lib
+from sagesim_amd.serving import footprint
+
+
+class _Full:
+    """An engine whose device has no memory for an order."""
+
+    def __init__(self, code):
+        self.code = code
+
+    def add_replica(self, rp, ci, ids, state, *a, **kw):
+        self.kept = np.array(state)
+        return 0
+
+    def set_order(self, rep, slots):
+        raise NativeError(self.code, "hipMalloc: out of memory")
+
+    def state(self, rep, n_total):
+        assert n_total == self.kept.size
+        return self.kept.copy()
+
+
+@pytest.mark.parametrize("ghosts", [0, 5])
+def test_states_without_memory_for_the_order(ghosts):
+    rng = np.random.default_rng(1)
+    n = 400
+    degs = rng.integers(0, 9, n)
+    rp = np.concatenate([[0], np.cumsum(degs)])
+    g = graphs.CSRGraph(rp, rng.integers(0, n + ghosts, rp[-1]).astype(np.int32), n_cols=n + ghosts)
+    st = rng.integers(0, 3, n + ghosts).astype(np.int8)
+    rep = Replica(_Full(SS_ERR_OOM), g, st, sir_model(0.3, 0.2), 1)
+    assert not np.array_equal(rep.engine.kept, st)
+    for _ in range(2):
+        assert np.array_equal(rep.states(), st)
+    with pytest.raises(NativeError):
+        Replica(_Full(-2), g, st, sir_model(0.3, 0.2), 1).states()
+
+
+def test_footprint_counts_the_order():
+    """An agent more costs its row bound (8), key and degree byte (5), three states
+    and its order (4) at least, groups of 64 agents at a time."""
+    L = step_lib()
+    a, b = (L.ss_replica_footprint(n, 0, 10_000, 0, 50) for n in (64_000, 128_000))
+    assert b - a >= 64_000 * (8 + 5 + 3 + 4 + 4)           # and the push counts (4)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,ghosts", [(1, 0), (1000, 0), (4097, 33), (50_000, 0)])
+def test_replica_bytes_within_footprint(n, ghosts):
+    print("[case] footprint", n, ghosts, flush=True)
+    rng = np.random.default_rng(n)
+    degs = rng.integers(0, min(9, n + ghosts), n)
+    rp = np.concatenate([[0], np.cumsum(degs)])
+    g = graphs.CSRGraph(rp, rng.integers(0, n + ghosts, rp[-1]).astype(np.int32), n_cols=n + ghosts)
+    with Engine(0) as eng:
+        rep = Replica(eng, g, np.zeros(n + ghosts, np.int8), sir_model(0.3, 0.2), 1)
+        eng.simulate(2)
+        rep.states()
+        assert eng.replica_bytes(rep.rep) <= footprint(g)
