@@ -165,7 +165,7 @@ extern "C" int ss_ghost_discover(ss_ctx *ctx, const int64_t *nbr_ids, int64_t nn
     if (e != hipSuccess) {
         char b[256];
         std::snprintf(b, sizeof b, "ss_ghost_discover: %s", hipGetErrorString(e));
-        return fail(ctx, e == hipErrorOutOfMemory ? SS_ERR_OOM : SS_ERR_HIP, b);
+        return fail(ctx, ss_hip_code(e), b);
     }
     *n_ghost = total;
     if (!ghost_ids) return SS_OK;
@@ -210,7 +210,7 @@ extern "C" int ss_ghost_discover(ss_ctx *ctx, const int64_t *nbr_ids, int64_t nn
     if (e != hipSuccess) {
         char b[256];
         std::snprintf(b, sizeof b, "ss_ghost_discover: %s", hipGetErrorString(e));
-        return fail(ctx, e == hipErrorOutOfMemory ? SS_ERR_OOM : SS_ERR_HIP, b);
+        return fail(ctx, ss_hip_code(e), b);
     }
     if (bad) return fail(ctx, SS_ERR_RANGE, "ss_ghost_discover: an owner rank is >= n_ranks");
     return SS_OK;

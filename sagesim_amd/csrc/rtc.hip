@@ -204,8 +204,7 @@ static thread_local std::string g_prog_err;
     do {                                                                                 \
         hipError_t _e = (expr);                                                          \
         if (_e != hipSuccess)                                                            \
-            P_FAIL(p, _e == hipErrorOutOfMemory ? SS_ERR_OOM : SS_ERR_HIP, "%s: %s", #expr, \
-                   hipGetErrorString(_e));                                               \
+            P_FAIL(p, ss_hip_code(_e), "%s: %s", #expr, hipGetErrorString(_e));          \
     } while (0)
 
 #define P_LIVE(p)                                                                                  \
@@ -328,7 +327,7 @@ int ss_prog_create(ss_ctx *ctx, int64_t n_agents, ss_prog **out) {
         pfree(p->d_args); pfree(p->agent_ids); pfree(p->logical_ids); pfree(p->breeds); pfree(p->row_ptr);
         pfree(p->logical_ids64);
         delete p;
-        return e == hipErrorOutOfMemory ? SS_ERR_OOM : SS_ERR_HIP;
+        return ss_hip_code(e);
     }
     ctx->progs.push_back(p);
     *out = p;

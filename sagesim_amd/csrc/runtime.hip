@@ -24,8 +24,7 @@ static thread_local std::string g_err;
     do {                                                                                \
         hipError_t _e = (expr);                                                         \
         if (_e != hipSuccess)                                                           \
-            SS_FAIL(ctx, _e == hipErrorOutOfMemory ? SS_ERR_OOM : SS_ERR_HIP, "%s: %s (%s:%d)", \
-                    #expr, hipGetErrorString(_e), __FILE__, __LINE__);                  \
+            SS_FAIL(ctx, ss_hip_code(_e), "%s: %s (%s:%d)", #expr, hipGetErrorString(_e), __FILE__, __LINE__); \
     } while (0)
 
 namespace {
@@ -520,6 +519,7 @@ int ss_create(int device, ss_ctx **out) {
                            hipHostMallocDefault)) != hipSuccess ||
         (e = create_halo_events(ctx)) != hipSuccess) {
         delete ctx;
+        (void)ss_hip_code(e);
         SS_FAIL(nullptr, SS_ERR_HIP, "context setup: %s", hipGetErrorString(e));
     }
     ctx->num_cus = prop.multiProcessorCount;
@@ -665,7 +665,7 @@ int ss_replica_create(ss_ctx *ctx, const ss_replica_spec *sp, int32_t *rep_out) 
         hipError_t _e = (expr);                                                      \
         if (_e != hipSuccess) {                                                      \
             ctx->err = std::string(#expr) + ": " + hipGetErrorString(_e);            \
-            return fail(_e == hipErrorOutOfMemory ? SS_ERR_OOM : SS_ERR_HIP);        \
+            return fail(ss_hip_code(_e));                                            \
         }                                                                            \
     } while (0)
     R_HIP(dalloc(ctx, &r, &r.row_ptr, (size_t)nt + 1));

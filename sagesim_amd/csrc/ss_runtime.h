@@ -27,6 +27,14 @@
 // tiles that ran
 #define SS_WORK_N 7
 
+// The code a call returns for e.  The runtime keeps an error until somebody asks
+// for it, and the check after the next launch would (an allocation that failed
+// would fail a later call that allocates nothing): asked for here.
+inline int ss_hip_code(hipError_t e) {
+    (void)hipGetLastError();
+    return e == hipErrorOutOfMemory ? SS_ERR_OOM : SS_ERR_HIP;
+}
+
 // kernel launchers (tick_kernels.hip)
 // only: the replica all tiles belong to, or -1
 hipError_t ss_launch_tick(const ss_rep_dev *reps, const ss_tile *tiles, int n_tiles, int k, int apl, int grid,

@@ -1,5 +1,6 @@
 """What a device without memory to spare still does: states() without the order
-table it keeps on the device, and a footprint that counts the table."""
+table it keeps on the device, a footprint that counts the table, and calls after
+one that ran out of memory."""
 import numpy as np
 import pytest
 
@@ -63,3 +64,22 @@ def test_replica_bytes_within_footprint(n, ghosts):
         eng.simulate(2)
         rep.states()
         assert eng.replica_bytes(rep.rep) <= footprint(g)
+
+
+@pytest.mark.gpu
+def test_calls_after_running_out_of_memory():
+    print("[case] out of memory", flush=True)
+    g = graphs.barabasi_albert(2000, 3, 1)
+    st = (np.arange(g.n) % 50 == 0).astype(np.int8)
+    with Engine(0) as eng:
+        rep = Replica(eng, g, st, sir_model(0.3, 0.2), 1)
+        eng.simulate(5)
+        want = rep.states()
+        rep.reset()
+        for _ in range(2):
+            with pytest.raises(NativeError) as ex:
+                eng.copy_probe(1 << 50)                     # a petabyte
+            assert ex.value.code == SS_ERR_OOM
+            assert np.array_equal(rep.states(), st)
+        eng.simulate(5)
+        assert np.array_equal(rep.states(), want)
