@@ -870,16 +870,18 @@ int ss_replica_set_order(ss_ctx *ctx, int32_t rep, const int32_t *slot, int64_t 
     SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
     if (!r.order) SS_HIP(ctx, dalloc(ctx, &r, &r.order, (size_t)pad_agents(n)));
     unsigned long long bad = ~0ull;
-    SS_HIP(ctx, hipMemsetAsync(ctx->d_stats, 0xFF, sizeof bad, ctx->stream));
-    SS_HIP(ctx, ss_copy_in(ctx, r.order, slot, sizeof(int32_t) * (size_t)n));
-    SS_HIP(ctx, ss_launch_check_cols(r.order, n, n, ctx->d_stats, ctx->num_cus * 8, ctx->stream));
-    SS_HIP(ctx, hipMemcpyAsync(&bad, ctx->d_stats, sizeof bad, hipMemcpyDeviceToHost, ctx->stream));
-    SS_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    if (bad != ~0ull) {
+    hipError_t e = hipMemsetAsync(ctx->d_stats, 0xFF, sizeof bad, ctx->stream);
+    if (e == hipSuccess) e = ss_copy_in(ctx, r.order, slot, sizeof(int32_t) * (size_t)n);
+    if (e == hipSuccess) e = ss_launch_check_cols(r.order, n, n, ctx->d_stats, ctx->num_cus * 8, ctx->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(&bad, ctx->d_stats, sizeof bad, hipMemcpyDeviceToHost, ctx->stream);
+    const hipError_t e2 = hipStreamSynchronize(ctx->stream);
+    if (e == hipSuccess) e = e2;
+    if (e != hipSuccess || bad != ~0ull) {              // slots that were not checked are not kept
         dfree(r.order);
         r.order = nullptr;
         r.bytes -= sizeof(int32_t) * (size_t)pad_agents(n);
         ctx->bytes -= sizeof(int32_t) * (size_t)pad_agents(n);
+        SS_HIP(ctx, e);
         SS_FAIL(ctx, SS_ERR_RANGE, "slot[%llu] = %d outside [0, %lld)", bad, slot[bad], (long long)n);
     }
     return SS_OK;

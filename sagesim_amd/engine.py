@@ -7,6 +7,7 @@ caller keeps its own agent order; the RNG stays keyed on the caller's ids, so
 results do not depend on the relabelling.
 """
 import ctypes
+import itertools
 import weakref
 from dataclasses import dataclass
 
@@ -51,6 +52,8 @@ class Engine:
         self.device = device
         self._pinned = {}                  # address -> byte count of live page-locked buffers
         self._halo_n = {}                  # replica -> records of its bound halo
+        self._orders = {}                  # replica -> number of the order it has (set_order)
+        self._order_numbers = itertools.count(1)
 
     # -- plumbing --
     def _ck(self, rc):
@@ -132,6 +135,7 @@ class Engine:
     def remove_replica(self, rep):
         self._ck(self._L.ss_replica_destroy(self._h, rep))
         self._halo_n.pop(rep, None)
+        self._orders.pop(rep, None)
 
     def reset(self, rep):
         self._ck(self._L.ss_replica_reset(self._h, rep))
@@ -161,9 +165,17 @@ class Engine:
         return out
 
     def set_order(self, rep, slots):
-        """The caller's agent order: slots[j] is the storage slot of agent j."""
+        """The caller's agent order: slots[j] is the storage slot of agent j.
+        Returns a number that order_of gives for as long as this order stands."""
         slots = np.ascontiguousarray(slots, np.int32)
+        self._orders.pop(rep, None)
         self._ck(self._L.ss_replica_set_order(self._h, rep, ptr(slots), slots.shape[0]))
+        self._orders[rep] = next(self._order_numbers)
+        return self._orders[rep]
+
+    def order_of(self, rep):
+        """The number of the order that state_ordered uses, None without one."""
+        return self._orders.get(rep)
 
     def state_ordered(self, rep, n_total):
         """The states with the local agents in the order of set_order."""
@@ -450,25 +462,26 @@ class Replica:
         self.n = data.n
         self.n_total = data.n_total
         self.n_ghost = self.n_total - self.n
-        self._order_set = False
+        self._order = None                  # the number of this replica's order on the engine
         self.rep = engine.add_replica(data.graph.row_ptr, data.graph.col_idx, data.rng_key_id, data.state, model,
                                       seed, n_ghost=self.n_ghost, history=data.history, tick0=tick0,
                                       tick_limit=tick_limit)
 
     def states(self):
-        """The states in the caller's agent order (put in order on the device,
-        which keeps the order from the first call on; on the host when the device
-        has no memory left for it)."""
-        if not self._order_set:
+        """The states in the caller's agent order: put in order on the device,
+        which keeps the order from the first call on, or on the host when the
+        device has no memory for it or Engine.set_order gave it another one."""
+        number = self.engine.order_of(self.rep)
+        if number is None:
             try:
-                self.engine.set_order(self.rep, self.inv)
+                number = self._order = self.engine.set_order(self.rep, self.inv)
             except NativeError as e:
                 if e.code != SS_ERR_OOM:
                     raise
-                st = self.engine.state(self.rep, self.n_total)
-                return np.concatenate([st[:self.n][self.inv], st[self.n:]])
-            self._order_set = True
-        return self.engine.state_ordered(self.rep, self.n_total)
+        if number is not None and number == self._order:
+            return self.engine.state_ordered(self.rep, self.n_total)
+        st = self.engine.state(self.rep, self.n_total)
+        return np.concatenate([st[:self.n][self.inv], st[self.n:]])
 
     def set_states(self, state):
         state = np.asarray(state, np.int8)

@@ -19,6 +19,9 @@ class _Full:
         self.kept = np.array(state)
         return 0
 
+    def order_of(self, rep):
+        return None
+
     def set_order(self, rep, slots):
         raise NativeError(self.code, "hipMalloc: out of memory")
 
