@@ -419,6 +419,7 @@ int ss_prog_add_array(ss_prog *p, int32_t elem_bytes, int64_t rows, int64_t widt
         P_HIP(p, e);
     }
     p->props.push_back(q);
+    p->loop_kernel = -1;                        // it writes back the arrays it was compiled for
     *id = (int32_t)p->props.size() - 1;
     return push_args(p);
 }
@@ -613,6 +614,7 @@ int ss_prog_set_schedule(ss_prog *p, int32_t n, const int32_t *kernel, const int
         s.push_back({kernel[i], start[i], count[i], -1});
     }
     p->schedule = s;
+    p->loop_kernel = -1;                        // it runs the schedule it was compiled for
     pfree(p->order);
     p->order = nullptr;
     p->order_n = 0;
