@@ -354,10 +354,12 @@ int ss_prog_set_order(ss_prog *prog, const int32_t *order, int64_t n);
 int ss_prog_set_long(ss_prog *prog, const int64_t *n_long, int32_t n_launches);
 /* Small programs: kernel `kernel` (const SSProgArgs*, long long tick, long long
  * ticks) runs whole ticks, schedule and write-back, on one block of `threads`
- * threads; ss_prog_simulate then launches it instead of the schedule.  -1: none,
- * as after every compile, schedule and added array, which such a kernel has
- * compiled in. */
+ * threads; ss_prog_simulate then launches it instead of the schedule, until its
+ * ticks turn out to be slower.  -1: none, as after every compile, schedule and
+ * added array, which such a kernel has compiled in. */
 int ss_prog_set_loop(ss_prog *prog, int32_t kernel, int32_t threads);
+/* the kernel the next ss_prog_simulate runs whole ticks with, -1: the schedule */
+int ss_prog_loop(ss_prog *prog, int32_t *kernel);
 /* Ticks tick0 .. tick0 + ticks - 1: the schedule, then write-back; waits. */
 int ss_prog_simulate(ss_prog *prog, int64_t tick0, int64_t ticks);
 /* Checkpoint of the program's state (replaces the pickle of Model.save /

@@ -129,6 +129,7 @@ def step_lib():
     _proto(L, "ss_prog_set_long", I, _P, _P, _c_i32)
     _proto(L, "ss_prog_set_unroll", I, _P, _c_i32)
     _proto(L, "ss_prog_set_loop", I, _P, _c_i32, _c_i32)
+    _proto(L, "ss_prog_loop", I, _P, _P)
     _proto(L, "ss_prog_save", I, _P, _c_i64, _P, _c_i64, _P)
     _proto(L, "ss_prog_restore", I, _P, _P, _c_i64, _P)
     _proto(L, "ss_prog_prop_upload", I, _P, _c_i32, _P)

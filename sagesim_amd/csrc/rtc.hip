@@ -9,6 +9,7 @@
 // runs the per-tick launch schedule followed by the write-back of
 // double-buffered arrays (model.py:2368-2408).
 #include <algorithm>
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -68,6 +69,42 @@ struct Launch {
     int64_t order_off;          // first entry of this launch in the order array, -1: agents in index order
     int64_t n_long = 0;         // agents at the front of the order that get a block each
     int64_t long_deg = 0;       // entries of the longest of their rows
+};
+
+// Whether the one-block kernel still pays, from the time its launches take.  What
+// a step does is the user's: one that walks all agents keeps a compute unit busy
+// for a millisecond a tick, where the schedule spreads it over several.  A
+// schedule's tick takes its launches at least (5 us each), so a tick below that
+// (and the 30 us of a launch that is waited for) is left alone; a longer one is set
+// against the schedule, two samples of either over ticks that are due anyway, and
+// the faster one goes on (asked again once a tick takes twice as long).  us a tick
+// of such a step, one block and schedule: 300 agents 70 and 62, 1000 agents 317 and
+// 190, 2000 agents 1260 and 376.  The first launch gets 16 ticks, the next ones four
+// times as many as the one before, at most 4096 and 20 ms of them.
+struct LoopTrial {
+    int64_t chunk = 16;         // ticks of the next launch
+    int samples = 0;            // taken since a launch took too long: that one, another, two of the schedule
+    double bar = 0.0;           // us a tick above which the schedule is tried; 0: what its launches take
+    double loop = 0.0, sched = 0.0;
+
+    void add(double us, int64_t n, size_t launches) {
+        const double tick = us / (double)n;
+        if (samples >= 2) {
+            sched = samples == 2 ? tick : std::min(sched, tick);
+            ++samples;
+            return;
+        }
+        loop = samples == 0 ? tick : std::min(loop, tick);
+        const double limit = bar > 0.0 ? bar : 5.0 * (double)launches;
+        if (samples || us > 30.0 + limit * (double)n) ++samples;
+        chunk = std::max<int64_t>(1, std::min<int64_t>({4 * chunk, (int64_t)(20000.0 / tick), 4096}));
+    }
+    bool schedule_wins() {
+        if (samples < 4) return false;
+        samples = 0;
+        bar = 2.0 * loop;
+        return sched < loop;
+    }
 };
 
 struct Extra {
@@ -180,6 +217,7 @@ struct ss_prog {
     std::vector<Launch> schedule;
     int32_t loop_kernel = -1;                   // kernel that runs whole ticks on one block, -1: none
     int32_t loop_threads = 0;
+    LoopTrial trial;
     std::vector<int64_t> h_row_ptr;             // row bounds, for the long rows' LDS
     int32_t *order = nullptr;                   // agent order of every launch (concatenated)
     std::vector<int32_t> h_order;
@@ -686,30 +724,23 @@ int ss_prog_set_loop(ss_prog *p, int32_t kernel, int32_t threads) {
         P_FAIL(p, SS_ERR_INVALID, "kernel %d of %zu with %d threads", kernel, p->kernels.size(), threads);
     p->loop_kernel = kernel;
     p->loop_threads = threads;
+    p->trial = LoopTrial();
+    return SS_OK;
+}
+
+int ss_prog_loop(ss_prog *p, int32_t *kernel) {
+    if (!p || !kernel) P_FAIL(p, SS_ERR_INVALID, "NULL argument");
+    P_LIVE(p);
+    *kernel = p->loop_kernel;
     return SS_OK;
 }
 
 // Every tick: the launches of the schedule in order (a kernel boundary
 // between priority groups is the grid barrier of model.py:2356-2366), then the
 // copy of every double-buffered array's write buffer into its read buffer
-// (model.py:2378-2406).
-int ss_prog_simulate(ss_prog *p, int64_t tick0, int64_t ticks) {
-    P_LIVE(p);
-    if (!p || ticks < 0) P_FAIL(p, SS_ERR_INVALID, "bad arguments");
-    if (!p->module) P_FAIL(p, SS_ERR_STATE, "no compiled step functions");
+// (model.py:2378-2406).  Waits.
+static int run_schedule(ss_prog *p, int64_t tick0, int64_t ticks) {
     hipStream_t st = p->ctx->stream;
-    if (p->loop_kernel >= 0) {
-        // at most 4096 ticks (tens of milliseconds) a launch
-        for (int64_t k = 0; k < ticks; k += 4096) {
-            const ProgArgsHost *a = p->d_args;
-            long long tick = (long long)(tick0 + k), n_ticks = (long long)std::min<int64_t>(ticks - k, 4096);
-            void *args[] = {(void *)&a, (void *)&tick, (void *)&n_ticks};
-            P_HIP(p, hipModuleLaunchKernel(p->kernels[p->loop_kernel], 1, 1, 1, (unsigned)p->loop_threads, 1, 1, 0, st,
-                                           args, nullptr));
-        }
-        P_HIP(p, hipStreamSynchronize(st));
-        return SS_OK;
-    }
     for (int64_t k = 0; k < ticks; ++k) {
         long long tick = (long long)(tick0 + k);
         for (const Launch &l : p->schedule) {
@@ -727,6 +758,39 @@ int ss_prog_simulate(ss_prog *p, int64_t tick0, int64_t ticks) {
         if (rc) return rc;
     }
     P_HIP(p, hipStreamSynchronize(st));
+    return SS_OK;
+}
+
+// The same ticks by the one-block kernel.  Waits.
+static int run_loop(ss_prog *p, int64_t tick0, int64_t ticks) {
+    const ProgArgsHost *a = p->d_args;
+    long long tick = (long long)tick0, n_ticks = (long long)ticks;
+    void *args[] = {(void *)&a, (void *)&tick, (void *)&n_ticks};
+    P_HIP(p, hipModuleLaunchKernel(p->kernels[p->loop_kernel], 1, 1, 1, (unsigned)p->loop_threads, 1, 1, 0,
+                                   p->ctx->stream, args, nullptr));
+    P_HIP(p, hipStreamSynchronize(p->ctx->stream));
+    return SS_OK;
+}
+
+int ss_prog_simulate(ss_prog *p, int64_t tick0, int64_t ticks) {
+    P_LIVE(p);
+    if (!p || ticks < 0) P_FAIL(p, SS_ERR_INVALID, "bad arguments");
+    if (!p->module) P_FAIL(p, SS_ERR_STATE, "no compiled step functions");
+    if (p->loop_kernel < 0 || ticks == 0) return run_schedule(p, tick0, ticks);
+    P_HIP(p, hipStreamSynchronize(p->ctx->stream));     // what is queued is not the step's time
+    LoopTrial &t = p->trial;
+    for (int64_t k = 0; k < ticks;) {
+        if (p->loop_kernel < 0) return run_schedule(p, tick0 + k, ticks - k);
+        const bool loop = t.samples < 2;
+        const int64_t n = std::min(ticks - k, t.samples ? std::min<int64_t>(t.chunk, 16) : t.chunk);
+        const auto from = std::chrono::steady_clock::now();
+        const int rc = loop ? run_loop(p, tick0 + k, n) : run_schedule(p, tick0 + k, n);
+        if (rc) return rc;
+        const double us = std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - from).count();
+        k += n;
+        t.add(us, n, p->schedule.size() + 1);
+        if (t.schedule_wins()) p->loop_kernel = -1;
+    }
     return SS_OK;
 }
 

@@ -78,7 +78,9 @@ _STAGED_ROW_MAX = 10_240          # 40 KB of LDS: four blocks per CU
 # where one compute unit's work catches up with the launches (us a tick,
 # launches / one block: rows of 20, 1000 agents 10.0 / 6.9 and 2000 agents
 # 10.4 / 12.4; rows of 6, 2000 agents 7.6 / 5.9; two breeds at three
-# priorities, 1000 agents 18.5 / 8.2 and 2000 agents 14.2 / 13.2).
+# priorities, 1000 agents 18.5 / 8.2 and 2000 agents 14.2 / 13.2).  The limits
+# are those of light steps; heavier ones go back to the launches, by the time
+# their ticks take (ss_prog_simulate).
 _LOOP_AGENTS = 2048
 _LOOP_ENTRIES = 24_000
 # Neighbour loops unrolled, by the longest row a thread walks alone (up to the

@@ -5,7 +5,8 @@ import ctypes
 import numpy as np
 import pytest
 
-from sagesim_amd import Engine
+from sagesim_amd import Breed, Engine, Model, NetworkSpace, StepFunction
+from sagesim_amd import model as model_mod
 from sagesim_amd._lib import ptr
 from sagesim_amd.model import _Program
 
@@ -81,3 +82,53 @@ def test_loop_then_array():
         p.add()
         assert np.array_equal(p.run(2, 2), np.array([[5.0], [2.0]]).repeat(100, 1))
         p.prog.close()
+
+
+_WALK = """
+__device__ void walk(auto tick, auto agent_index, auto n_agents, auto agent_ids, auto breeds, auto locations,
+                     auto state) {
+    float sum = 0.0f;
+    for (int j = 0; j < (int)n_agents; ++j)
+        sum += state[j] * (float)rand_uniform_philox(tick, agent_index, j);
+    state[agent_index] = 0.5f * state[agent_index] + sum / (float)n_agents;
+}
+"""
+
+
+def _walkers(n, limit, monkeypatch):
+    """n agents whose step walks all of them."""
+    monkeypatch.setattr(model_mod, "_LOOP_AGENTS", limit)
+    b = Breed("Walker")
+    b.register_property("state", 1.0)
+    b.register_step_func(StepFunction("walk", _WALK), priority=0)
+    m = Model(NetworkSpace())
+    m.register_breed(b)
+    m.register_global_property("n_agents", n)
+    m.set_seed(3)
+    for i in range(n):
+        m.create_agent_of_breed(b, state=float(i % 7))
+    m.get_space().connect_agents_bulk(np.arange(n - 1), np.arange(1, n))
+    m.setup()
+    return m
+
+
+def _loop_of(m):
+    k = ctypes.c_int32(-2)
+    m._prog.ck(m._prog._L.ss_prog_loop(m._prog._h, ctypes.byref(k)))
+    return k.value
+
+
+@pytest.mark.parametrize("calls", [[100], [1] * 8, [3, 30, 2]])
+@pytest.mark.parametrize("n", [1, 300, 2000])
+def test_heavy_step(n, calls, monkeypatch):
+    """A step that keeps one block busy for a millisecond a tick goes back to the
+    schedule after a few ticks, with the same results."""
+    print("[case] heavy step", n, calls, flush=True)
+    one, many = _walkers(n, 2048, monkeypatch), _walkers(n, 0, monkeypatch)
+    assert _loop_of(one) >= 0 and _loop_of(many) == -1
+    for c in calls:
+        one.simulate(c)
+        many.simulate(c)
+        assert np.array_equal(one.get_breed_data("Walker", "state"), many.get_breed_data("Walker", "state"))
+    if n == 2000:
+        assert _loop_of(one) == -1
