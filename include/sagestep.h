@@ -95,7 +95,9 @@ int ss_device_info(ss_ctx *ctx, int32_t *num_cus, int64_t *total_mem, int64_t *c
 int ss_replica_create(ss_ctx *ctx, const ss_replica_spec *spec, int32_t *rep);
 int ss_replica_destroy(ss_ctx *ctx, int32_t rep);
 /* device bytes a replica of this shape takes (serving admission), the order of
- * ss_replica_set_order among them */
+ * ss_replica_set_order among them.  Its creation uses some 10 bytes an agent of
+ * workspace beside them; of that a context keeps up to 256 MB for later calls,
+ * until an allocation of its own needs the room. */
 int64_t ss_replica_footprint(int64_t n_local, int64_t n_ghost, int64_t nnz, int32_t with_history, int64_t max_deg);
 /* back to the state, history and tick given at creation (Model.reset, model.py:944-958) */
 int ss_replica_reset(ss_ctx *ctx, int32_t rep);

@@ -91,7 +91,9 @@ int fail(ss_ctx *ctx, int code, const char *msg) {
 
 // device scratch of one discovery, freed by the destructor
 struct Scratch {
+    ss_ctx *ctx;
     std::vector<void *> p;
+    explicit Scratch(ss_ctx *c) : ctx(c) {}
     ~Scratch() {
         for (void *q : p)
             if (q) (void)hipFree(q);
@@ -100,7 +102,7 @@ struct Scratch {
     hipError_t get(T **out, size_t count) {
         *out = nullptr;
         void *q = nullptr;
-        hipError_t e = hipMalloc(&q, sizeof(T) * (count ? count : 1));
+        hipError_t e = ss_device_alloc(ctx, &q, sizeof(T) * (count ? count : 1));
         if (e == hipSuccess) {
             p.push_back(q);
             *out = static_cast<T *>(q);
@@ -125,7 +127,7 @@ extern "C" int ss_ghost_discover(ss_ctx *ctx, const int64_t *nbr_ids, int64_t nn
     (void)hipSetDevice(ctx->device);
     hipStream_t st = ctx->stream;
     const int64_t n_words = (n_owner + 31) / 32;
-    Scratch s;
+    Scratch s(ctx);
     int64_t *d_nbr = nullptr;
     int32_t *d_owner = nullptr, *d_cnt = nullptr, *d_pos = nullptr, *d_misc = nullptr;
     uint32_t *d_bits = nullptr;

@@ -351,12 +351,12 @@ int ss_prog_create(ss_ctx *ctx, int64_t n_agents, ss_prog **out) {
     p->n = n_agents;
     const size_t nn = (size_t)std::max<int64_t>(n_agents, 1);
     hipError_t e = hipSetDevice(ctx->device);
-    if (e == hipSuccess) e = hipMalloc((void **)&p->d_args, sizeof(ProgArgsHost));
-    if (e == hipSuccess) e = hipMalloc((void **)&p->agent_ids, nn * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc((void **)&p->logical_ids, nn * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc((void **)&p->breeds, nn * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc((void **)&p->logical_ids64, nn * sizeof(int64_t));
-    if (e == hipSuccess) e = hipMalloc((void **)&p->row_ptr, (nn + 1) * sizeof(int64_t));
+    if (e == hipSuccess) e = ss_device_alloc(ctx, (void **)&p->d_args, sizeof(ProgArgsHost));
+    if (e == hipSuccess) e = ss_device_alloc(ctx, (void **)&p->agent_ids, nn * sizeof(float));
+    if (e == hipSuccess) e = ss_device_alloc(ctx, (void **)&p->logical_ids, nn * sizeof(float));
+    if (e == hipSuccess) e = ss_device_alloc(ctx, (void **)&p->breeds, nn * sizeof(float));
+    if (e == hipSuccess) e = ss_device_alloc(ctx, (void **)&p->logical_ids64, nn * sizeof(int64_t));
+    if (e == hipSuccess) e = ss_device_alloc(ctx, (void **)&p->row_ptr, (nn + 1) * sizeof(int64_t));
     // on the context's stream, like the upload that follows (ss_prog_set_csr): a
     // clear on the null stream could land after it and empty every row
     if (e == hipSuccess) e = hipMemsetAsync(p->row_ptr, 0, (nn + 1) * sizeof(int64_t), ctx->stream);
@@ -395,7 +395,7 @@ int ss_prog_set_csr(ss_prog *p, const int64_t *row_ptr, const int32_t *col_idx, 
     P_HIP(p, hipStreamSynchronize(p->ctx->stream));
     pfree(p->col_idx);
     p->col_idx = nullptr;
-    P_HIP(p, hipMalloc((void **)&p->col_idx, sizeof(int32_t) * (size_t)std::max<int64_t>(nnz, 1)));
+    P_HIP(p, ss_device_alloc(p->ctx, (void **)&p->col_idx, sizeof(int32_t) * (size_t)std::max<int64_t>(nnz, 1)));
     P_HIP(p, ss_copy_in(p->ctx, p->col_idx, col_idx, sizeof(int32_t) * (size_t)nnz));
     P_HIP(p, ss_copy_in(p->ctx, p->row_ptr, row_ptr, sizeof(int64_t) * (size_t)(p->n + 1)));
     p->nnz = nnz;
@@ -436,9 +436,9 @@ int ss_prog_add_array(ss_prog *p, int32_t elem_bytes, int64_t rows, int64_t widt
     q.width = width;
     q.double_buffered = double_buffered != 0;
     const size_t b = std::max<size_t>(q.bytes(), 16);
-    P_HIP(p, hipMalloc(&q.r, b));
+    P_HIP(p, ss_device_alloc(p->ctx, &q.r, b));
     if (q.double_buffered) {
-        hipError_t e = hipMalloc(&q.w, b);
+        hipError_t e = ss_device_alloc(p->ctx, &q.w, b);
         if (e != hipSuccess) { pfree(q.r); P_HIP(p, e); }
     } else {
         q.w = q.r;
@@ -497,7 +497,7 @@ int ss_prog_set_globals(ss_prog *p, const double *values, int64_t count) {
     if (count != p->n_globals) {
         pfree(p->globals);
         p->globals = nullptr;
-        P_HIP(p, hipMalloc((void **)&p->globals, sizeof(double) * (size_t)std::max<int64_t>(count, 1)));
+        P_HIP(p, ss_device_alloc(p->ctx, (void **)&p->globals, sizeof(double) * (size_t)std::max<int64_t>(count, 1)));
         p->n_globals = count;
     }
     if (count) P_HIP(p, hipMemcpy(p->globals, values, sizeof(double) * count, hipMemcpyHostToDevice));
@@ -527,7 +527,7 @@ int ss_prog_set_extra(ss_prog *p, int32_t slot, int64_t bytes, const void *data)
         pfree(x.d);
         x.d = nullptr;
         x.bytes = 0;
-        P_HIP(p, hipMalloc(&x.d, (size_t)std::max<int64_t>(bytes, 16)));
+        P_HIP(p, ss_device_alloc(p->ctx, &x.d, (size_t)std::max<int64_t>(bytes, 16)));
         x.bytes = bytes;
     }
     P_HIP(p, ss_copy_in(p->ctx, x.d, data, (size_t)bytes));
@@ -684,7 +684,7 @@ int ss_prog_set_order(ss_prog *p, const int32_t *order, int64_t n) {
     P_HIP(p, hipStreamSynchronize(p->ctx->stream));
     pfree(p->order);
     p->order = nullptr;
-    P_HIP(p, hipMalloc((void **)&p->order, sizeof(int32_t) * (size_t)std::max<int64_t>(n, 1)));
+    P_HIP(p, ss_device_alloc(p->ctx, (void **)&p->order, sizeof(int32_t) * (size_t)std::max<int64_t>(n, 1)));
     if (n) P_HIP(p, hipMemcpy(p->order, order, sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice));
     p->order_n = n;
     p->h_order.assign(order, order + n);

@@ -37,7 +37,7 @@ hipError_t dalloc(ss_ctx *ctx, ss_replica *r, T **p, size_t count) {
     *p = nullptr;
     if (count == 0) count = 1;
     size_t b = sizeof(T) * count;
-    hipError_t e = hipMalloc((void **)p, b);
+    hipError_t e = ss_device_alloc(ctx, (void **)p, b);
     if (e == hipSuccess) {
         if (r) r->bytes += b;
         ctx->bytes += b;
@@ -49,25 +49,36 @@ void dfree(void *p) {
     if (p) (void)hipFree(p);
 }
 
+void drop_scratch(ss_ctx *ctx) {
+    (void)hipStreamSynchronize(ctx->stream);
+    dfree(ctx->scratch);
+    ctx->scratch = nullptr;
+    ctx->bytes -= ctx->scratch_bytes;
+    ctx->scratch_bytes = 0;
+}
+
 // The context's workspace, at least b bytes (256-byte aligned): kept for later
 // calls, replaced by a larger one when it is too small, freed with the context
-// (and by a Scratch guard's end when it is larger than what is worth keeping).  Every
-// user runs on the context's stream and is done with it when it returns.
+// (by a Scratch guard's end when it is larger than what is worth keeping, and by
+// an allocation that would fail otherwise).  Every user holds a guard, runs on the
+// context's stream and is done with it when it returns.
 hipError_t scratch(ss_ctx *ctx, size_t b, void **p) {
     if (ctx->scratch_bytes < b) {
         hipError_t e = hipStreamSynchronize(ctx->stream);
         if (e != hipSuccess) return e;
-        dfree(ctx->scratch);
-        ctx->scratch = nullptr;
-        ctx->bytes -= ctx->scratch_bytes;
-        ctx->scratch_bytes = 0;
-        const size_t want = std::max<size_t>(b + b / 4, 1 << 16);
-        if ((e = hipMalloc(&ctx->scratch, want)) != hipSuccess) {
+        drop_scratch(ctx);
+        // a quarter more, so that a little more next time fits; no more than is
+        // needed when the device has no room for it
+        for (const size_t want : {std::max<size_t>(b + b / 4, 1 << 16), b}) {
+            if ((e = hipMalloc(&ctx->scratch, want)) == hipSuccess) {
+                ctx->scratch_bytes = want;
+                ctx->bytes += want;
+                break;
+            }
             ctx->scratch = nullptr;
-            return e;
+            (void)hipGetLastError();
         }
-        ctx->scratch_bytes = want;
-        ctx->bytes += want;
+        if (e != hipSuccess) return e;
     }
     *p = ctx->scratch;
     return hipSuccess;
@@ -77,14 +88,9 @@ const size_t kScratchKept = 256u << 20;
 
 struct Scratch {
     ss_ctx *ctx;
-    explicit Scratch(ss_ctx *c) : ctx(c) {}
+    explicit Scratch(ss_ctx *c) : ctx(c) { ++ctx->scratch_users; }
     ~Scratch() {
-        if (ctx->scratch_bytes <= kScratchKept) return;
-        (void)hipStreamSynchronize(ctx->stream);
-        dfree(ctx->scratch);
-        ctx->scratch = nullptr;
-        ctx->bytes -= ctx->scratch_bytes;
-        ctx->scratch_bytes = 0;
+        if (--ctx->scratch_users == 0 && ctx->scratch_bytes > kScratchKept) drop_scratch(ctx);
     }
 };
 
@@ -476,6 +482,16 @@ int launch_loop(ss_ctx *ctx, int64_t ticks) {
 }
 
 }  // namespace
+
+hipError_t ss_device_alloc(ss_ctx *ctx, void **p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && ctx->scratch && ctx->scratch_users == 0) {
+        (void)hipGetLastError();
+        drop_scratch(ctx);
+        e = hipMalloc(p, bytes);
+    }
+    return e;
+}
 
 extern "C" {
 
@@ -902,6 +918,7 @@ int ss_state_download_ordered(ss_ctx *ctx, int32_t rep, int8_t *out, int64_t n) 
         }));
         return SS_OK;
     }
+    Scratch guard(ctx);
     void *d = nullptr;
     SS_HIP(ctx, scratch(ctx, (size_t)pad_agents(n), &d));
     SS_HIP(ctx, ss_launch_order(st, r.order, (int8_t *)d, 0, n, r.n_local, ctx->stream));
@@ -1075,9 +1092,9 @@ struct MapBatch {
     int64_t *ids = nullptr;
     int32_t *vals = nullptr;
     ~MapBatch() { dfree(ids); dfree(vals); }
-    hipError_t stage(const int64_t *h_ids, const int32_t *h_vals, int64_t n) {
-        hipError_t e = hipMalloc((void **)&ids, sizeof(int64_t) * (size_t)n);
-        if (e == hipSuccess && h_vals) e = hipMalloc((void **)&vals, sizeof(int32_t) * (size_t)n);
+    hipError_t stage(ss_ctx *ctx, const int64_t *h_ids, const int32_t *h_vals, int64_t n) {
+        hipError_t e = ss_device_alloc(ctx, (void **)&ids, sizeof(int64_t) * (size_t)n);
+        if (e == hipSuccess && h_vals) e = ss_device_alloc(ctx, (void **)&vals, sizeof(int32_t) * (size_t)n);
         if (e == hipSuccess) e = hipMemcpy(ids, h_ids, sizeof(int64_t) * (size_t)n, hipMemcpyHostToDevice);
         if (e == hipSuccess && h_vals) e = hipMemcpy(vals, h_vals, sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice);
         return e;
@@ -1109,7 +1126,7 @@ static int map_seq(ss_ctx *ctx, ss_replica &r, int op, const int64_t *ids, const
     out[0] = out[1] = 0;
     if (n == 0) return SS_OK;
     MapBatch b;
-    hipError_t e = b.stage(ids, vals, n);
+    hipError_t e = b.stage(ctx, ids, vals, n);
     if (e == hipSuccess) e = hipMemsetAsync(ctx->d_counters, 0, 2 * sizeof(int32_t), ctx->stream);
     if (e == hipSuccess)
         e = ss_launch_map_seq(r.map_keys, r.map_vals, r.map_cap, op, b.ids, b.vals, n, ctx->d_counters, ctx->stream);
@@ -1729,8 +1746,8 @@ int ss_census(ss_ctx *ctx, int32_t rep, int64_t *out) {
 int ss_copy_probe(ss_ctx *ctx, int64_t bytes, int32_t repeats, float *ms) {
     if (!ctx || !ms || bytes <= 0 || bytes % 16 || repeats < 1) SS_FAIL(ctx, SS_ERR_INVALID, "bad probe arguments");
     void *src = nullptr, *dst = nullptr;
-    SS_HIP(ctx, hipMalloc(&src, (size_t)bytes));
-    hipError_t e = hipMalloc(&dst, (size_t)bytes);
+    SS_HIP(ctx, ss_device_alloc(ctx, &src, (size_t)bytes));
+    hipError_t e = ss_device_alloc(ctx, &dst, (size_t)bytes);
     if (e != hipSuccess) { dfree(src); SS_HIP(ctx, e); }
     const int grid = ctx->num_cus * 8;
     e = ss_launch_fill_u32((uint32_t *)src, bytes / 4, 0x9E3779B9u, grid, ctx->stream);
@@ -1752,8 +1769,8 @@ int ss_gather_probe(ss_ctx *ctx, int64_t span_bytes, int64_t n_gathers, int32_t 
         SS_FAIL(ctx, SS_ERR_INVALID, "bad probe arguments");
     const int grid = ctx->num_cus * 8;
     uint32_t *src = nullptr, *out = nullptr;
-    SS_HIP(ctx, hipMalloc((void **)&src, (size_t)span_bytes));
-    hipError_t e = hipMalloc((void **)&out, sizeof(uint32_t) * (size_t)grid * 256);
+    SS_HIP(ctx, ss_device_alloc(ctx, (void **)&src, (size_t)span_bytes));
+    hipError_t e = ss_device_alloc(ctx, (void **)&out, sizeof(uint32_t) * (size_t)grid * 256);
     if (e != hipSuccess) { dfree(src); SS_HIP(ctx, e); }
     const int64_t words = span_bytes / 4;
     e = ss_launch_fill_u32(src, words, 0x9E3779B9u, grid, ctx->stream);

@@ -76,11 +76,13 @@ hipError_t ss_launch_fill_i32(int32_t *p, int64_t n, int32_t v, hipStream_t s);
 hipError_t ss_launch_order(const int8_t *st, const int32_t *slot, int8_t *out, int64_t first, int64_t end,
                            int64_t n_local, hipStream_t s);
 hipError_t ss_launch_copy(const void *src, void *dst, int64_t bytes, int grid, hipStream_t s);
+struct ss_ctx;
+// device memory; a kept workspace of the context goes before the device is out of it
+hipError_t ss_device_alloc(ss_ctx *ctx, void **p, size_t bytes);
 // ---- staging.hip: copies of ordinary host memory on the context's stream ----
 // Up: the caller's memory is read when it returns, the device has it for what
 // follows on the stream.  Down: the caller has it when it returns.
 #define SS_STAGE_LANES 4
-struct ss_ctx;
 struct ss_stager;
 hipError_t ss_copy_in(ss_ctx *ctx, void *dev, const void *host, size_t bytes);
 hipError_t ss_copy_out(ss_ctx *ctx, void *host, const void *dev, size_t bytes);
@@ -242,6 +244,7 @@ struct ss_ctx {
     void *h_stage = nullptr;                    // page-locked, SS_STAGE_BYTES: a small pack's slots and result
     void *scratch = nullptr;                    // workspace of one call at a time, on the context's stream
     size_t scratch_bytes = 0;
+    int scratch_users = 0;                      // calls under way that use it
     std::string err;
     size_t bytes = 0;
 };

@@ -86,3 +86,26 @@ def test_calls_after_running_out_of_memory():
             assert np.array_equal(rep.states(), st)
         eng.simulate(5)
         assert np.array_equal(rep.states(), want)
+
+
+@pytest.mark.gpu
+def test_kept_workspace_makes_room():
+    """The workspace that a map build leaves with the context goes before an
+    allocation fails, and comes back with the next build."""
+    print("[case] kept workspace", flush=True)
+    n = 200_000
+    g = graphs.CSRGraph(np.zeros(n + 1, np.int64), np.zeros(0, np.int32))
+    ids = np.arange(n, dtype=np.int64) * 7
+    with Engine(0) as eng:
+        rep = Replica(eng, g, np.zeros(n, np.int8), sir_model(0.3, 0.2), 1)
+        eng.simulate(1)
+        rep.states()
+        for _ in range(2):
+            eng.map_build(rep.rep, ids, np.arange(n))
+            full = eng.info()["ctx_bytes"]
+            with pytest.raises(NativeError):
+                eng.copy_probe(1 << 50)
+            assert eng.info()["ctx_bytes"] <= full - 20 * n            # ids, slots and claims
+            slots, missing = eng.map_lookup(rep.rep, ids)
+            assert missing == 0 and np.array_equal(slots, np.arange(n))
+            assert np.array_equal(rep.states(), np.zeros(n, np.int8))
