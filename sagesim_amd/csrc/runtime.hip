@@ -273,8 +273,10 @@ int build_tiles(ss_ctx *ctx) {
     // from 2048 when the replicas hold 64M entries and more, enough work for every
     // block beside the longest rows'.  Passes at 1024 and at 2048: BA(10M, 5), 100M
     // entries, 8.49 and 8.17 ms; ensembles of 129M and 180M 10.35 and 10.06, 13.85 and
-    // 13.58; BA(6M, 5) SEIR, 60M, 6.15 and 6.06; but BA(9M, 3), 54M, 8.15 and 8.24,
-    // BA(2M, 5) 3.12 and 3.17, BA(1M, 5) 2.51 and 2.56.
+    // 13.58; BA(6M, 5) SEIR, 60M, 6.15 and 6.06; BA(9M, 3), 54M, 8.15 and 8.24;
+    // BA(2M, 5) 3.12 and 3.17, BA(1M, 5) 2.51 and 2.56.  The line lies above all sizes
+    // at which 1024 was the faster one; entries alone do not separate the two (the
+    // 60M network, below it, would gain 1.5 %), and either costs 2 to 4 % at most.
     if (!ctx->tiling_given) {
         int64_t entries = 0;
         for (const ss_replica &r : ctx->reps)

@@ -225,7 +225,7 @@ struct ss_ctx {
     std::map<int64_t, hipGraphExec_t> graphs;   // by tick count
     int32_t *d_counters = nullptr;              // misc device counters (misses, overflow)
     unsigned long long *d_work = nullptr;       // [SS_WORK_N] tick-kernel work counters
-    unsigned long long *d_stats = nullptr;      // [8] results of the checks at replica creation
+    unsigned long long *d_stats = nullptr;      // [8] first slot of an order outside the replica (ss_replica_set_order)
     unsigned long long *d_part = nullptr;       // parts of a tick's start, 2 words a block
     unsigned long long *h_stats = nullptr;      // census rows, page-locked, 4 blocks per CU
     bool counting = false;
